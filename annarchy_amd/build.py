@@ -99,7 +99,8 @@ def build_core(jobs: int = 8) -> Path:
 # The library name hashes the generated source together with the headers it
 # is compiled against (the plug-in ABI and the device helpers), so a library
 # built against other headers is never picked up under the same name.
-_ABI_HEADERS = (INCLUDE / "annarchy_hip_model.h", INCLUDE / "annarchy_hip_synapse.h", CSRC / "ahip_device.hpp")
+_ABI_HEADERS = (INCLUDE / "annarchy_hip_model.h", INCLUDE / "annarchy_hip_synapse.h", CSRC / "ahip_device.hpp",
+                CSRC / "rate_rows.hpp")
 
 
 def _headers_digest() -> bytes:

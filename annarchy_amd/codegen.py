@@ -28,11 +28,11 @@ import re
 
 from .equations import DISTRIBUTIONS, NeuronDescription, analyse_neuron, equation_code
 
-ABI = 10  # AHIP_MODEL_ABI in include/annarchy_hip_model.h
+ABI = 11  # AHIP_MODEL_ABI in include/annarchy_hip_model.h
 
 _PRELUDE = r"""// Generated neuron-model library for the MI355X simulation backend.
 // Model: %(name)s
-#include "ahip_device.hpp"
+#include "rate_rows.hpp"
 #include <cmath>
 #include <cstdint>
 
@@ -83,15 +83,16 @@ __global__ __launch_bounds__(AHIP_UPDATE_BLOCK) void local_update(ahip_pop_args 
 %(global_loads)s
 %(div_consts)s
 %(local_ptrs)s
+    const bool _act = i < a.size;
     // the neuron's values the delivery below does not write, in registers
     // (their loads overlap the delivery's)
 %(reg_pre)s
     // this step's spike events of the ordered conductances (end of compute_psp)
-    if (a.n_deliver > 0 && i < a.size) ahip::deliver_buckets<T>(a, i);
+    if (a.n_deliver > 0 && _act) ahip::deliver_buckets<T>(a, i);
     asm volatile("" ::: "memory");  // the equations below read the delivered values
 %(reg_post)s
     bool _spike = false;
-    if (i < a.size) {
+    if (_act) {
 %(refrac_in)s
 %(local_rand)s
 %(local_eqs)s
@@ -118,6 +119,7 @@ int launch_f32(const ahip_pop_args* a, void* s) { return launch<float>(a, s); }
 %(preloop_fn)s
 
 %(persist_fn)s
+%(fused_fn)s
 
 const char* const kSlotNames[] = {%(slot_names)s};
 const int32_t kSlotLocal[] = {%(slot_local)s};
@@ -129,7 +131,7 @@ const double kRandArgs[] = {%(rand_args)s};
 const ahip_model_desc kDesc = {
     %(abi)d, "%(name)s", %(spiking)d, %(n_slots)d, kSlotNames, kSlotLocal, kSlotInit, kSlotKind,
     %(n_rand)d, kRandDist, kRandArgs, %(has_refractory)d, %(has_global)d,
-    launch_f64, launch_f32, %(preloop_ptr)s, "%(hash)s", %(persist_ptrs)s};
+    launch_f64, launch_f32, %(preloop_ptr)s, "%(hash)s", %(persist_ptrs)s, %(fused_ptrs)s};
 
 }  // namespace
 
@@ -471,6 +473,103 @@ const int32_t kPersistSlotsHost[] = {%(pslot_list)s};
 """
 
 
+# psp and update of a rate-coded population in one launch (ahip_fuse_args).  At
+# the sizes it serves, a step is latency: a dependent launch of a captured graph
+# costs 1.1 us before its first instruction, the random draw of a neuron about
+# as much, a row's chain of loads more.  So the step is one launch, and some
+# waves draw while the others sum.  With STAGE a workgroup of 1024 threads first
+# copies the pre-synaptic rates to LDS (a gather from global memory takes a
+# cycle of the CU's address unit per lane).  Separate launches -> this, us per
+# step: 800 neurons x 80 synapses 5.1 -> 3.4, 10007 x 300 in FP32 12.5 -> 8.1
+# (staged), dense 2503 x 2503 17.2 -> 10.9, two projections with delays into
+# 5001 neurons 29 -> 14 (the gather, copy and queue launches gone too).  The
+# first form, in which the lane that holds a row's sum went on with the
+# statements, took 5.6 at 800 x 80: the draw alone is 1800 cycles, twice that
+# with a cold instruction cache.
+_FUSED_KERNEL = r"""
+constexpr int kSums = %(n_sums)d;
+
+template <typename T, int KIND, bool STAGE>
+__global__ __launch_bounds__(STAGE ? AHIP_FUSE_STAGE_THREADS : AHIP_FUSE_THREADS) void fused_update(
+    const ahip_pop_args a, const ahip_fuse_args F) {
+    constexpr int kWaves = (STAGE ? AHIP_FUSE_STAGE_THREADS : AHIP_FUSE_THREADS) / ahip::kWave;
+    extern __shared__ unsigned char lds_raw[];
+    __shared__ T sums_s[kSums][AHIP_FUSE_ROWS];
+    __shared__ ahip::Partial<T> part_s[KIND == AHIP_FUSE_DENSE ? AHIP_FUSE_DENSE_ROWS * kWaves : 1];
+    const int32_t place = ahip::fused_place();
+    if (place >= F.blocks) return;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / ahip::kWave));
+    const int64_t t = ahip::sim_time(a);
+    const int sum_waves = kWaves - F.update_waves;
+    T* xs = reinterpret_cast<T*>(lds_raw);
+    if (wave >= F.update_waves) {
+        if constexpr (STAGE) {
+            const int32_t first = F.update_waves * ahip::kWave;
+            ahip::stage_rates<T>(F, t, xs, (int32_t)threadIdx.x - first, AHIP_FUSE_STAGE_THREADS - first);
+            __syncthreads();
+        }
+        ahip::fused_rows<T, kSums, KIND, STAGE>(F, place, t, a.size, wave - F.update_waves, sum_waves, xs, sums_s,
+                                                part_s);
+        __syncthreads();
+        return;
+    }
+    const int32_t i = ahip::fused_neuron(F, place, (int32_t)threadIdx.x);
+    const bool _act = i >= 0;
+    const T dt = (T)a.dt;
+    (void)dt;
+%(global_loads)s
+%(div_consts)s
+%(local_ptrs)s
+%(reg_pre)s
+%(fused_rand)s
+    if constexpr (STAGE) __syncthreads();
+    __syncthreads();
+    T _psp[kSums];
+#pragma unroll
+    for (int k = 0; k < kSums; k++) _psp[k] = sums_s[k][threadIdx.x %% AHIP_FUSE_ROWS];
+    if constexpr (KIND == AHIP_FUSE_DENSE)
+        if (_act) {
+            const T s = ahip::join_parts(part_s + threadIdx.x * sum_waves, sum_waves);
+#pragma unroll
+            for (int k = 0; k < kSums; k++) _psp[k] = F.p[0].sum == k ? s : T(0);
+        }
+%(reg_sum)s
+    if (_act) {
+%(local_eqs)s
+%(reg_out)s
+    }
+}
+
+template <typename T>
+int fused(const ahip_pop_args* a, const ahip_fuse_args* F, void* stream) {
+    hipStream_t s = (hipStream_t)stream;
+%(launch_global)s
+    if (F->blocks <= 0) return (int)hipErrorInvalidValue;
+#define AHIP_FUSED_CASE(KIND, STAGE)                                                                      \
+    case 2 * KIND + STAGE:                                                                                \
+        hipLaunchKernelGGL((fused_update<T, KIND, STAGE>), dim3((F->blocks + 7) / 8 * 8),                 \
+                           dim3(STAGE ? AHIP_FUSE_STAGE_THREADS : AHIP_FUSE_THREADS),                     \
+                           STAGE ? (size_t)F->lds_values * sizeof(T) : 0, s, *a, *F);                     \
+        break;
+    switch (2 * F->kind + (F->stage ? 1 : 0)) {
+        AHIP_FUSED_CASE(AHIP_FUSE_CSR, false)
+        AHIP_FUSED_CASE(AHIP_FUSE_CSR, true)
+        AHIP_FUSED_CASE(AHIP_FUSE_SELL, false)
+        AHIP_FUSED_CASE(AHIP_FUSE_SELL, true)
+        AHIP_FUSED_CASE(AHIP_FUSE_DENSE, false)
+        AHIP_FUSED_CASE(AHIP_FUSE_MIX, false)
+        AHIP_FUSED_CASE(AHIP_FUSE_MIX, true)
+        default:
+            return (int)hipErrorInvalidValue;
+    }
+#undef AHIP_FUSED_CASE
+    return (int)hipGetLastError();
+}
+int fused_f64(const ahip_pop_args* a, const ahip_fuse_args* F, void* s) { return fused<double>(a, F, s); }
+int fused_f32(const ahip_pop_args* a, const ahip_fuse_args* F, void* s) { return fused<float>(a, F, s); }
+"""
+
+
 def _indent(code: str, n: int) -> str:
     pad = " " * n
     return "\n".join(pad + line if line.strip() else line for line in code.split("\n"))
@@ -748,7 +847,13 @@ def generate(desc: NeuronDescription, stop_condition: str | None = None) -> Mode
     # read: any reference other than the target of a plain assignment
     lreads = lambda c: re.search(lref(c) + r"(?!\s*=(?!=))", ljoined) is not None
     reg_pre, reg_post, reg_out = [], [], []
+    # of the fused psp and update: loads before and after the row sums
+    # (stores only at the end: a load or branch after one waits for it)
+    reg_fpre, reg_sum, sum_out = [], [], []
     kind_of = {s_[0]: s_[3] for s_ in slots}
+    sums = [s_[0] for s_ in slots if s_[3] == 2]
+    # a rate that other launches read from the population's rings
+    ring_r = not desc.spiking and "r" in local_names
     cands = [(_u(n), "T", f"{_u(n)}[i]", n.startswith("g_")) for n in local_names]
     if has_ref:
         cands.append(("refrac_rem", "int32_t", "a.refractory_remaining[i]", False))
@@ -756,7 +861,8 @@ def generate(desc: NeuronDescription, stop_condition: str | None = None) -> Mode
         # a psp sum the psp may leave in panel partials: completed (and
         # stored) by the update, read or not
         if kind_of.get(n) == 2 and not lreads(_u(n)):
-            reg_pre.append(f"    if (a.n_psum > 0 && i < a.size) (void)ahip::psp_sum<T>(a, {slot_of[n]}, {_u(n)}, i);")
+            reg_pre.append(f"    if (a.n_psum > 0 && _act) (void)ahip::psp_sum<T>(a, {slot_of[n]}, {_u(n)}, i);")
+            sum_out.append(f"        if (ahip::has_sum(F, {sums.index(n)})) {_u(n)}[i] = _psp[{sums.index(n)}];")
     for c, ty, mem, after in cands:
         if not lreads(c):
             if lwrites(c):
@@ -768,11 +874,40 @@ def generate(desc: NeuronDescription, stop_condition: str | None = None) -> Mode
         name = {_u(n): n for n in local_names}.get(c)
         if name is not None and kind_of.get(name) == 2:
             load = f"ahip::psp_sum<T>(a, {slot_of[name]}, {c}, i)"
-        (reg_post if after else reg_pre).append(f"    {ty} {c}__r = i < a.size ? {load} : {ty}(0);")
+            k = sums.index(name)
+            reg_fpre.append(f"    T {c}__r = _act && !ahip::has_sum(F, {k}) ? {c}[i] : T(0);")
+            reg_sum.append(f"    if (ahip::has_sum(F, {k})) {c}__r = _psp[{k}];")
+            sum_out.append(f"        if (ahip::has_sum(F, {k})) {c}[i] = _psp[{k}];")
+        else:
+            reg_fpre.append(f"    {ty} {c}__r = _act ? {load} : {ty}(0);")
+        (reg_post if after else reg_pre).append(f"    {ty} {c}__r = _act ? {load} : {ty}(0);")
         if lwrites(c):
             reg_out.append(f"        {mem} = {c}__r;")
         for key in lparts:
             lparts[key] = re.sub(lref(c), c + "__r", lparts[key])
+
+    if ring_r:
+        r_now = _u("r") + ("__r" if lreads(_u("r")) else "[i]")
+        reg_out.append(f"        ahip::push_rate<T>(a, t, i, {r_now});")
+
+    fused_fn, fused_ptrs = "", "nullptr, nullptr"
+    if ring_r and sums:
+        fused_fn = _FUSED_KERNEL % {
+            "n_sums": len(sums),
+            "global_loads": global_loads,
+            "div_consts": div_consts,
+            "local_ptrs": local_ptrs,
+            "reg_pre": "\n".join(reg_fpre),
+            "reg_sum": "\n".join(reg_sum),
+            # drawn by the update waves before they wait for the sums
+            "fused_rand": "\n".join(
+                re.sub(r"^const T (\w+) = (.*);$", r"    const T \1 = _act ? \2 : T(0);\n"
+                       r'    asm volatile("" ::"v"(\1));', line) for line in lparts["local_rand"].split("\n")),
+            "local_eqs": _indent(lparts["local_eqs"], 8),
+            "reg_out": "\n".join(reg_out + sum_out),
+            "launch_global": launch_global,
+        }
+        fused_ptrs = "fused_f64, fused_f32"
 
     body = _PRELUDE % {"name": desc.name}
     if has_global:
@@ -812,6 +947,8 @@ def generate(desc: NeuronDescription, stop_condition: str | None = None) -> Mode
         "preloop_ptr": preloop_ptr,
         "persist_fn": persist_fn,
         "persist_ptrs": persist_ptrs,
+        "fused_fn": fused_fn,
+        "fused_ptrs": fused_ptrs,
         "hash": "%(hash)s",
     }
     cond, _ = parse_stop_condition(stop_condition)

@@ -72,19 +72,77 @@ __device__ inline double draw(uint64_t seed, uint32_t stream, int32_t i, int32_t
 }
 
 // ---------------------------------------------------------------------------
-// Wave reductions (64 lanes; butterfly over the lanes of a group of width W).
+// Wave reductions over aligned groups of W lanes, in the vector unit: the
+// partner at distance 1 and 2 by a quad permutation, at 4 and 8 by mirroring a
+// half row and a row (the groups below are uniform by then), at 16 and 32 by a
+// row swap.  (A shuffle through the LDS unit costs some 190 cycles a level:
+// 1170 for the FP64 sum of a wave, against about 200.)  Every lane of a group
+// ends with the same sum.
 // ---------------------------------------------------------------------------
+struct u32pair {
+    uint32_t a, b;
+};
+// the two values that lanes at distance O (a power of two) add: {own, other}
+// below 16 and {lower row's, upper row's} from there on
+template <int O>
+__device__ inline u32pair lane_pair(uint32_t v) {
+    if constexpr (O == 1) return {v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, true)};
+    else if constexpr (O == 2) return {v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, true)};
+    else if constexpr (O == 4) return {v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, true)};
+    else if constexpr (O == 8) return {v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, true)};
+    else if constexpr (O == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return {(uint32_t)r[0], (uint32_t)r[1]};
+    } else {
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return {(uint32_t)r[0], (uint32_t)r[1]};
+    }
+}
+template <int O>
+__device__ inline void lane_pair(float v, float& a, float& b) {
+    const u32pair p = lane_pair<O>(__float_as_uint(v));
+    a = __uint_as_float(p.a);
+    b = __uint_as_float(p.b);
+}
+template <int O>
+__device__ inline void lane_pair(double v, double& a, double& b) {
+    const uint64_t w = (uint64_t)__double_as_longlong(v);
+    const u32pair lo = lane_pair<O>((uint32_t)w), hi = lane_pair<O>((uint32_t)(w >> 32));
+    a = __longlong_as_double((long long)(((uint64_t)hi.a << 32) | lo.a));
+    b = __longlong_as_double((long long)(((uint64_t)hi.b << 32) | lo.b));
+}
+template <int O>
+__device__ inline void lane_pair(int32_t v, int32_t& a, int32_t& b) {
+    const u32pair p = lane_pair<O>((uint32_t)v);
+    a = (int32_t)p.a;
+    b = (int32_t)p.b;
+}
+template <int O, typename T>
+__device__ inline T level_sum(T v) {
+    T a, b;
+    lane_pair<O>(v, a, b);
+    return a + b;
+}
 template <int W, typename T>
 __device__ inline T group_sum(T v) {
-#pragma unroll
-    for (int o = W / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, W);
+    if constexpr (W > 1) v = level_sum<1>(v);
+    if constexpr (W > 2) v = level_sum<2>(v);
+    if constexpr (W > 4) v = level_sum<4>(v);
+    if constexpr (W > 8) v = level_sum<8>(v);
+    if constexpr (W > 16) v = level_sum<16>(v);
+    if constexpr (W > 32) v = level_sum<32>(v);
     return v;
 }
 
-// The same butterfly over aligned groups of w lanes, w a power of two known
-// only at run time (uniform across the wave).
-__device__ inline double group_sum_rt(double v, int w) {
-    for (int o = w / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+// The same over groups of 2^shift lanes, known only at run time (uniform).
+template <typename T>
+__device__ inline T group_sum_rt(T v, int shift) {
+    if (shift > 0) v = level_sum<1>(v);
+    if (shift > 1) v = level_sum<2>(v);
+    if (shift > 2) v = level_sum<4>(v);
+    if (shift > 3) v = level_sum<8>(v);
+    if (shift > 4) v = level_sum<16>(v);
+    if (shift > 5) v = level_sum<32>(v);
     return v;
 }
 
@@ -103,33 +161,48 @@ struct Kahan {
 };
 
 // Compensated reduction over a lane group: pairs (s, c) are combined with a
-// two-sum at every butterfly level.
+// two-sum at every level.
+template <int O>
+__device__ inline void level_kahan(float& s, float& c) {
+    float s0, s1, c0, c1;
+    lane_pair<O>(s, s0, s1);
+    lane_pair<O>(c, c0, c1);
+    const float t = s0 + s1;
+    const float bp = t - s0;
+    const float err = (s0 - (t - bp)) + (s1 - bp);
+    s = t;
+    c = (c0 + c1) + err;
+}
+// groups of 2^shift lanes; every lane of a group ends with the pair
+__device__ inline void group_join_kahan(float& s, float& c, int shift) {
+    if (shift > 0) level_kahan<1>(s, c);
+    if (shift > 1) level_kahan<2>(s, c);
+    if (shift > 2) level_kahan<4>(s, c);
+    if (shift > 3) level_kahan<8>(s, c);
+    if (shift > 4) level_kahan<16>(s, c);
+    if (shift > 5) level_kahan<32>(s, c);
+}
+constexpr int log2_of(int w) { return w <= 1 ? 0 : 1 + log2_of(w / 2); }
 template <int W>
 __device__ inline float group_sum_kahan(float s, float c) {
-#pragma unroll
-    for (int o = W / 2; o > 0; o >>= 1) {
-        float so = __shfl_xor(s, o, W);
-        float co = __shfl_xor(c, o, W);
-        float t = s + so;
-        float bp = t - s;
-        float err = (s - (t - bp)) + (so - bp);
-        s = t;
-        c = c + co + err;
-    }
+    group_join_kahan(s, c, log2_of(W));
     return s + c;
 }
 
-__device__ inline float group_sum_kahan_rt(float s, float c, int w) {
-    for (int o = w / 2; o > 0; o >>= 1) {
-        float so = __shfl_xor(s, o, kWave);
-        float co = __shfl_xor(c, o, kWave);
-        float t = s + so;
-        float bp = t - s;
-        float err = (s - (t - bp)) + (so - bp);
-        s = t;
-        c = c + co + err;
+// u mod n in [0, n), n > 0.  The compiler's 64-bit remainder is some 150
+// instructions that a latency-bound kernel has to fetch; steps fit in 32 bits
+// for a long time, and the rest is a short loop of shifts and subtractions.
+__device__ inline int64_t mod_pos(int64_t u, int64_t n) {
+    if ((((uint64_t)u | (uint64_t)n) >> 32) == 0) return (uint32_t)u % (uint32_t)n;
+    const uint64_t a = u < 0 ? ~(uint64_t)u : (uint64_t)u;
+    uint64_t r = 0;
+#pragma unroll 1
+    for (int b = 63; b >= 0; b--) {
+        r = (r << 1) | ((a >> b) & 1);
+        if (r >= (uint64_t)n) r -= (uint64_t)n;
     }
-    return s + c;
+    // u < 0: a = -u - 1, and u mod n = n - 1 - (a mod n)
+    return u < 0 ? n - 1 - (int64_t)r : (int64_t)r;
 }
 
 __device__ inline int64_t sim_time(const ahip_pop_args& a) { return *a.t_base + a.step; }
@@ -170,10 +243,7 @@ __device__ inline T random_value(const ahip_pop_args& a, int32_t i, int32_t k, i
                                  int32_t dist, double pa, double pb) {
     const void* inj = a.rand_inject[k];
     if (inj) {
-        int64_t row = t - a.rand_t0;
-        int64_t n = a.rand_inject_steps;
-        row %= n;
-        if (row < 0) row += n;
+        const int64_t row = mod_pos(t - a.rand_t0, a.rand_inject_steps);
         return ((const T*)inj)[row * (int64_t)a.size + i];
     }
     return (T)draw(a.seed, a.stream_id, i, k, t, dist, pa, pb);

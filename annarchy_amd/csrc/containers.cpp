@@ -12,7 +12,8 @@
 //             inside windows of sigma rows; slice width padded to a multiple
 //             of TPR; entry (r, k) at off + (k/TPR)*64 + r*TPR + k%TPR
 //   BSR       square tiles (2, 4 or 8), row-major inside a tile
-//   DENSE     row-major n_rows x n_cols
+//   DENSE     row-major n_rows x n_cols, rows padded to a multiple of 4 values
+//             (16-byte loads at every row)
 //   CSR_PANEL CSR whose rows are split in column panels: panel-major order,
 //             aux[q][r] = first entry of row r in panel q
 //   SELL_PANEL the tiles of CSR_PANEL, each stored as sorted 64-row slices
@@ -79,7 +80,7 @@ bool pow2(int v) { return v > 0 && (v & (v - 1)) == 0; }
 // too little work per tile.
 // Compute units of the current device (256 on MI355X; that figure when no
 // device answers, as on a build host).
-static int32_t device_cus() {
+int32_t device_cus() {
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) {
@@ -232,10 +233,12 @@ int build_layout(const Proj& p, int32_t precision, const ahip_format_opts& o, Ra
         case AHIP_FMT_DENSE: {
             const size_t total = (size_t)R * p.n_cols;
             if (total > ((size_t)1 << 33)) { err = "dense layout too large"; return AHIP_EINVAL; }
-            std::vector<double> val(total, 0.0);
+            const size_t ld = ((size_t)p.n_cols + 3) / 4 * 4;
+            std::vector<double> val((size_t)R * ld, 0.0);
             for (int32_t r = 0; r < R; r++)
-                for (int64_t j = rp[r]; j < rp[r + 1]; j++) val[(size_t)r * p.n_cols + ci[j]] = wval(p, j);
-            L.stored = (int64_t)total;
+                for (int64_t j = rp[r]; j < rp[r + 1]; j++) val[(size_t)r * ld + ci[j]] = wval(p, j);
+            L.width = (int32_t)ld;
+            L.stored = (int64_t)R * (int64_t)ld;
             if ((rc = upload_vals(L.val, val, precision, err))) return rc;
             return 0;
         }

@@ -39,7 +39,7 @@ struct RateLayout {
     int32_t sigma = 1;
     int32_t panel_cols = 0;
     int64_t stored = 0;       // stored entries including padding
-    int32_t width = 0;        // ELL max row length
+    int32_t width = 0;        // ELL max row length / DENSE values per stored row
     int32_t n_units = 0;      // SELL slices / BSR block rows / panels
     DevBuf ptr;               // CSR row_ptr (int64) / SELL slice offsets (int64) / BSR block row ptr (int32)
     DevBuf idx;               // column indices (int32), padded formats included
@@ -67,6 +67,12 @@ struct Pop {
     // depth x size int32 with counts int32[depth]
     int32_t depth = 1;
     DevBuf hist, hist_count;
+    // rate-coded: r at the end of the last two steps (slot t & 1), kept by the
+    // population's update while a fused update reads it; and the population's
+    // own fused update (psp of every projection into it, then the statements)
+    DevBuf rbuf;
+    bool fused = false;
+    ahip_fuse_args fuse;
     // mean firing rate over fr_window steps (0: off): a fr_window-bit history
     // per neuron (uint32 words, word-major) and the number of spikes in it
     // stop_condition: 0 none, 1 the model's condition for any neuron, 2 for
@@ -272,6 +278,7 @@ struct ahip_net {
     ahip::DevBuf deliver_targets;               // DeliverTarget of the merged delivery launch
     int32_t deliver_n_tg = 0, deliver_waves = 0;
     int32_t delivery = AHIP_DELIVERY_ORDERED;
+    bool rbuf_stale = true;        // a rate changed outside a step since the rbufs were filled
     bool persist_enabled = true;   // small single-population networks: one launch per batch
     size_t elem() const { return precision == AHIP_F64 ? sizeof(double) : sizeof(float); }
 };
@@ -368,5 +375,8 @@ int report_error(int code, const char* msg);
 int build_layout(const Proj& p, int32_t precision, const ahip_format_opts& o, RateLayout& out,
                  std::string& err);
 double psp_bytes(const Proj& p, int32_t precision);
+// Compute units of the current device.
+int32_t device_cus();
+constexpr int32_t kWaveSize = 64;
 
 }  // namespace ahip

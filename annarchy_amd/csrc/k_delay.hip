@@ -16,18 +16,13 @@
 // post neuron, the number of events (one weight per projection: the weight is
 // then added that many times, in sequence, as the reference adds it event by
 // event) or the sum of their weights (one weight per synapse).
-#include "ahip_device.hpp"
 #include "internal.hpp"
+#include "rate_rows.hpp"
 
 namespace ahip {
 namespace {
 
 constexpr int kBlock = 256;
-
-__device__ inline int64_t ring_slot(int64_t t, int32_t D) {
-    const int64_t m = t % D;
-    return m < 0 ? m + D : m;
-}
 
 // hist[(t mod D)][i] = src[i]
 template <typename T>

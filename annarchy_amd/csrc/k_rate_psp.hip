@@ -8,30 +8,13 @@
 // FP64: plain sums (row order differs from the sequential loop: results agree
 // to rounding).  FP32: Neumaier-compensated lane sums and a compensated lane
 // reduction.
-#include "ahip_device.hpp"
 #include "internal.hpp"
+#include "rate_rows.hpp"
 
 namespace ahip {
 namespace {
 
 constexpr int kBlock = 256;
-
-template <typename T>
-struct Acc;
-template <>
-struct Acc<double> {
-    double s = 0.0;
-    __device__ inline void add(double x) { s += x; }
-    template <int W>
-    __device__ inline double reduce() { return group_sum<W>(s); }
-};
-template <>
-struct Acc<float> {
-    Kahan k{0.0f, 0.0f};
-    __device__ inline void add(float x) { k.add(x); }
-    template <int W>
-    __device__ inline float reduce() { return group_sum_kahan<W>(k.s, k.c); }
-};
 
 template <typename T>
 __device__ inline T ldnt(const T* p) {
@@ -230,42 +213,27 @@ __global__ __launch_bounds__(kBlock) void bsr_rows(int32_t n_brows, int32_t n_ro
         if (c < n_cols) a.add(v * x[c]);
     }
     // sum over the BS columns of a tile row (adjacent lanes), then over slots
-    T s;
-    if constexpr (sizeof(T) == 8) {
-        s = group_sum<BS>(a.s);
+    T s = a.template reduce<BS>();
 #pragma unroll
-        for (int o = TT; o < kWave; o <<= 1) s += __shfl_xor(s, o, kWave);
-    } else {
-        float ss = a.k.s, cc = a.k.c;
-        float v = group_sum_kahan<BS>(ss, cc);
-#pragma unroll
-        for (int o = TT; o < kWave; o <<= 1) v += __shfl_xor(v, o, kWave);
-        s = v;
-    }
+    for (int o = TT; o < kWave; o <<= 1) s += __shfl_xor(s, o, kWave);
     const int64_t row = br * BS + tr;
     if (slot == 0 && tc == 0 && row < n_rows) store_target(y, row, s, acc != 0);
 }
 
-// Dense row-major W [n_rows x n_cols]: one wave per row.
+// Dense row-major W (ld values per stored row): a workgroup sums 4 rows.
 template <typename T>
-__global__ __launch_bounds__(kBlock) void dense_rows(int32_t n_rows, int32_t n_cols,
+__global__ __launch_bounds__(kBlock) void dense_rows(int32_t n_rows, int32_t n_cols, int64_t ld,
                                                      const T* __restrict__ W,
                                                      const T* __restrict__ x, T* __restrict__ y,
                                                      int32_t acc) {
-    const int64_t row = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / kWave;
-    const int lane = threadIdx.x & (kWave - 1);
-    if (row >= n_rows) return;
-    const T* wr = W + row * (int64_t)n_cols;
-    Acc<T> a0, a1;
-    int32_t k = lane;
-    for (; k + kWave < n_cols; k += 2 * kWave) {
-        a0.add(ldnt(wr + k) * x[k]);
-        a1.add(ldnt(wr + k + kWave) * x[k + kWave]);
-    }
-    if (k < n_cols) a0.add(ldnt(wr + k) * x[k]);
-    a0.add(a1.template reduce<1>());
-    const T s = a0.template reduce<kWave>();
-    if (lane == 0) store_target(y, row, s, acc != 0);
+    constexpr int kWaves = kBlock / kWave;
+    __shared__ Partial<T> part[kDenseRows * kWaves];
+    const int64_t row0 = (int64_t)blockIdx.x * kDenseRows;
+    dense_rows4<T>(W, ld, n_cols, row0, n_rows, x, threadIdx.x / kWave, kWaves, part);
+    __syncthreads();
+    const int64_t row = row0 + threadIdx.x;
+    if (threadIdx.x < kDenseRows && row < n_rows)
+        store_target(y, row, join_parts(part + threadIdx.x * kWaves, kWaves), acc != 0);
 }
 
 // Row-block x column-panel tiles.  The gather of the pre-synaptic rates is
@@ -570,9 +538,9 @@ int launch_rate_t(const ahip_net* net, const Proj& p, const T* x, T* y, hipStrea
             return (int)hipGetLastError();
         }
         case AHIP_FMT_DENSE: {
-            const int64_t nb = ((int64_t)p.n_rows * kWave + kBlock - 1) / kBlock;
+            const int64_t nb = ((int64_t)p.n_rows + kDenseRows - 1) / kDenseRows;
             if (nb == 0) return 0;
-            hipLaunchKernelGGL((dense_rows<T>), dim3(nb), dim3(kBlock), 0, s, p.n_rows, p.n_cols,
+            hipLaunchKernelGGL((dense_rows<T>), dim3(nb), dim3(kBlock), 0, s, p.n_rows, p.n_cols, (int64_t)L.width,
                                L.val.as<T>(), x, y, acc);
             return (int)hipGetLastError();
         }

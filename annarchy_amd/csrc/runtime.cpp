@@ -103,6 +103,7 @@ void drop_graph(ahip_net* net) {
 void invalidate(ahip_net* net) {
     drop_graph(net);
     net->scatter_dirty = true;
+    net->rbuf_stale = true;
 }
 
 bool layout_covers_all_rows(const Proj& p) {
@@ -154,7 +155,10 @@ int ensure_delay_buffers(ahip_net* net) {
     }
     for (auto& pp : net->pops) {
         Pop& p = *pp;
-        const int32_t D = std::max(need[p.id], p.depth);
+        // one slot more for rates: a fused update may push step t's value
+        // while another workgroup of its launch reads step t - max_delay's
+        const int32_t want = need[p.id] > 1 && !p.model->spiking ? need[p.id] + 1 : need[p.id];
+        const int32_t D = std::max(want, p.depth);
         if (D == p.depth && (D == 1 || p.hist.p)) continue;
         HIPCHK(hipStreamSynchronize(net->stream));
         const int32_t d_old = p.hist.p ? p.depth : 0;
@@ -520,6 +524,8 @@ int build_ordered_targets(ahip_net* net, const std::vector<const void*>& targets
     return 0;
 }
 
+static int plan_fused(ahip_net* net);
+
 int prepare(ahip_net* net) {
     if (!net->initialized) return fail(AHIP_ESTATE, "network not initialized");
     for (auto& pp : net->projs) {
@@ -658,6 +664,194 @@ int prepare(ahip_net* net) {
             }
         }
     }
+    return plan_fused(net);
+}
+
+// A projection that a fused update can sum, as its descriptor.  False: the
+// layout has no row form there (panels, ELL, BSR).
+static bool fuse_desc(ahip_net* net, const Proj& p, int32_t sum, ahip_fuse_proj& d) {
+    const Pop& pre = *net->pops[p.pre];
+    const RateLayout& L = p.rate;
+    if (pre.model->spiking || L.val.p == nullptr || L.stored >= (int64_t)1 << 28) return false;
+    std::memset(&d, 0, sizeof(d));
+    switch (L.format) {
+        case AHIP_FMT_CSR:
+        case AHIP_FMT_CSR_VEC:
+            d.kind = p.delay_per_syn ? AHIP_FUSE_CSR_DELAY : AHIP_FUSE_CSR;
+            break;
+        case AHIP_FMT_SELL:
+            d.kind = AHIP_FUSE_SELL;
+            break;
+        case AHIP_FMT_DENSE:
+            d.kind = AHIP_FUSE_DENSE;
+            d.ld = L.width;
+            break;
+        default:
+            return false;
+    }
+    d.sum = sum;
+    d.n_cols = p.n_cols;
+    d.ptr = L.ptr.as<int64_t>();
+    d.col = L.idx.as<int32_t>();
+    d.w = L.val.p;
+    if (p.delay_per_syn || p.delay_uniform >= 2) {
+        // (32-bit offsets into the ring)
+        if (!pre.hist.p || (int64_t)pre.depth * pre.size >= INT32_MAX) return false;
+        d.x = pre.hist.p;
+        d.depth = pre.depth;
+        d.delay = p.delay_per_syn ? 0 : p.delay_uniform;
+        d.delays = p.delay_per_syn ? p.delay_dev.as<int16_t>() : nullptr;
+    } else {
+        d.x = pre.rbuf.p;   // set by plan_fused once the buffer exists
+        d.depth = 2;
+        d.delay = 1;
+    }
+    return true;
+}
+
+// Largest synapse count per population whose psp the update sums itself: where
+// the rates are gathered from global memory, the separate psp with its
+// streaming loads takes over above it (us per step, one launch / separate: CSR
+// FP64 75 / 101 at 40000 x 400, 194 / 182 at 100000 x 300, 320 / 310 at
+// 40000 x 1500); staged or dense rows gain or are equal as far as measured
+// (45.7 / 81.6 at 12000 x 2000, dense 89.3 / 90.2 at 8000 x 8000).
+constexpr int64_t kFuseMaxGathered = 1 << 24, kFuseMaxStaged = 1 << 27;
+
+// Which populations run psp and update in one launch: an active rate-coded
+// population whose every incoming projection is rate-coded with a row layout
+// (at most AHIP_MAX_FUSE of them; a SELL layout's row order serves CSR rows
+// beside it but no second SELL), in a network without inactive populations
+// (their rings stand still).
+static int plan_fused(ahip_net* net) {
+    bool all_active = true;
+    for (auto& pp : net->pops) all_active = all_active && pp->active;
+    for (auto& pp : net->pops) {
+        Pop& p = *pp;
+        p.fused = false;
+        const ahip_fused_fn fn = net->precision == AHIP_F64 ? p.model->fused_f64 : p.model->fused_f32;
+        if (!fn || !all_active) continue;
+        std::vector<int32_t> sums;   // slots of the model's psp sums
+        for (int32_t k = 0; k < p.model->n_slots; k++)
+            if (p.model->slot_kind[k] == 2) sums.push_back(k);
+        ahip_fuse_args& F = p.fuse;
+        std::memset(&F, 0, sizeof(F));
+        bool ok = sums.size() <= 32, dense = false, stage = true;
+        int64_t nnz = 0, values = 0;
+        int64_t widest = 0;   // mean entries per row of the widest projection
+        const Proj* sell = nullptr;
+        for (auto& qq : net->projs) {
+            Proj& q = *qq;
+            if (q.post != p.id) continue;
+            if (q.spiking || q.n_rows != p.size) { ok = false; break; }
+            const int32_t k = (int32_t)(std::find(sums.begin(), sums.end(), q.target_slot) - sums.begin());
+            if (k == (int32_t)sums.size()) { ok = false; break; }
+            F.mask |= 1u << k;
+            if (!transmits(net, q) || q.nnz == 0) continue;
+            if (F.n == AHIP_MAX_FUSE || !fuse_desc(net, q, k, F.p[F.n])) { ok = false; break; }
+            const ahip_fuse_proj& d = F.p[F.n++];
+            F.kind = F.n == 1 || F.kind == d.kind ? d.kind : AHIP_FUSE_MIX;
+            if (d.kind == AHIP_FUSE_SELL) {
+                if (sell) { ok = false; break; }
+                sell = &q;
+            }
+            dense = dense || d.kind == AHIP_FUSE_DENSE;
+            if (d.kind == AHIP_FUSE_DENSE || d.kind == AHIP_FUSE_CSR_DELAY) stage = false;
+            else values += q.n_cols;
+            nnz += d.kind == AHIP_FUSE_DENSE ? (int64_t)q.n_rows * q.n_cols : q.nnz;
+            widest = std::max(widest, q.nnz / std::max(1, q.n_rows));
+        }
+        if (!ok || F.n == 0 || (sell && dense)) continue;
+        if (F.kind == AHIP_FUSE_CSR_DELAY || (F.kind == AHIP_FUSE_DENSE && F.n > 1)) F.kind = AHIP_FUSE_MIX;
+        F.perm = sell ? sell->rate.perm.as<int32_t>() : nullptr;
+        F.units = sell ? sell->rate.n_units : p.size;
+        const int64_t lds = values * (int64_t)net->elem();
+        const int64_t cus = device_cus();
+        // Lanes per row: about 3 entries per lane (all in flight at once; a row
+        // of 50 took 4.2 / 3.5 / 4.1 us with 8 / 16 / 64 lanes at 3000 rows,
+        // one of 200 5.8 / 5.3 us with 16 / 64 at 5001), 10 when staged (a row of
+        // 300: 15.8 / 10.4 / 12.2 us with 16 / 32 / 64 at 10007 rows).
+        auto lanes_for = [&](int64_t per_lane) {
+            int32_t l = 1;
+            while (l < kWaveSize && l * per_lane < widest) l *= 2;
+            return sell ? sell->rate.lanes : dense ? kWaveSize : l;
+        };
+        // Staging the rates pays when a CU's gathers (one lane per cycle from
+        // global memory) outweigh copying them (64 bytes per cycle and about
+        // 2000 cycles of latency), and when the rows occupy its 15 summing
+        // waves on at least half the CUs.
+        int32_t lanes = lanes_for(10);
+        int32_t per_wave = sell ? 1 : kWaveSize / lanes;   // units of a wave
+        const int32_t stage_waves = AHIP_FUSE_STAGE_THREADS / kWaveSize - 1;
+        stage = stage && lds <= 128 * 1024 && nnz / cus > lds / 64 + 2000 &&
+                (int64_t)F.units * 2 >= cus * stage_waves * per_wave;
+        if (nnz > (stage || F.kind == AHIP_FUSE_DENSE ? kFuseMaxStaged : kFuseMaxGathered)) continue;
+        if (!stage) {
+            lanes = lanes_for(4);
+            per_wave = sell ? 1 : kWaveSize / lanes;
+        }
+        while ((1 << F.lane_shift) < lanes) F.lane_shift++;
+        const int32_t unit_rows = sell ? kWaveSize / lanes : 1;
+        const int32_t max_share = AHIP_FUSE_ROWS / unit_rows;
+        if (stage) {
+            // one round on the CUs, as many workgroups on each as its LDS holds
+            const int64_t slots = cus * (2 * (lds + 16 * 1024) <= 160 * 1024 ? 2 : 1);
+            F.share = (int32_t)std::min<int64_t>(max_share, std::max<int64_t>(per_wave, (F.units + slots - 1) / slots));
+            F.lds_values = (int32_t)values;
+        } else if (F.kind == AHIP_FUSE_DENSE) {
+            F.share = 4;
+        } else {
+            // one pass of the summing waves, the statements in one wave
+            F.share = std::min(max_share, std::max(1, std::min((AHIP_FUSE_THREADS / kWaveSize - 1) * per_wave,
+                                                              kWaveSize / unit_rows)));
+        }
+        F.update_waves = (F.share * unit_rows + kWaveSize - 1) / kWaveSize;
+        F.blocks = (F.units + F.share - 1) / F.share;
+        F.stage = stage ? 1 : 0;
+        p.fused = true;
+    }
+    // the pre-synaptic rates of undelayed projections: the last two steps'
+    std::vector<char> need(net->pops.size(), 0);
+    for (auto& pp : net->pops)
+        if (pp->fused)
+            for (auto& qq : net->projs)
+                if (qq->post == pp->id && !qq->delay_per_syn && qq->delay_uniform < 2) need[qq->pre] = 1;
+    for (auto& pp : net->pops) {
+        Pop& p = *pp;
+        if (need[p.id] && !p.rbuf.p) {
+            drop_graph(net);
+            int rc = dev_alloc(p.rbuf, 2 * (size_t)p.size * net->elem());
+            if (rc) return rc;
+            net->rbuf_stale = true;
+        } else if (!need[p.id] && p.rbuf.p) {
+            drop_graph(net);
+            HIPCHK(hipStreamSynchronize(net->stream));
+            p.rbuf.release();
+        }
+    }
+    for (auto& pp : net->pops) {
+        Pop& p = *pp;
+        if (!p.fused) continue;
+        int32_t n = 0;
+        for (auto& qq : net->projs)
+            if (qq->post == p.id && transmits(net, *qq) && qq->nnz != 0) {
+                ahip_fuse_proj& d = p.fuse.p[n++];
+                if (!qq->delay_per_syn && qq->delay_uniform < 2) d.x = net->pops[qq->pre]->rbuf.p;
+            }
+    }
+    return 0;
+}
+
+// The two-step rate buffers hold the rates as they are now: written by the
+// updates, refreshed here when something else changed a rate (or the clock).
+static int refresh_rates(ahip_net* net) {
+    if (!net->rbuf_stale) return 0;
+    for (auto& pp : net->pops) {
+        Pop& p = *pp;
+        if (!p.rbuf.p) continue;
+        // the slot of the last step, t - 1
+        LCHK(launch_push_values(net, p.slots[p.slot_index("r")].p, p.rbuf.p, p.size, 2, -1, net->stream));
+    }
+    net->rbuf_stale = false;
     return 0;
 }
 
@@ -674,7 +868,7 @@ static void assign_deferred_reduce(ahip_net* net) {
         p.defer_reduce = false;
         if (p.spiking || p.delay_per_syn || !transmits(net, p)) continue;
         const Pop& post = *net->pops[p.post];
-        if (post.model->spiking || post.model->has_global_update) continue;
+        if (post.model->spiking || post.model->has_global_update || post.fused) continue;
         const RateLayout& L = p.rate;
         if (L.format != AHIP_FMT_SELL_PANEL && L.format != AHIP_FMT_CSR_PANEL) continue;
         if ((int64_t)L.n_units * L.width == 0 || p.n_rows != post.size || !L.perm.p) continue;
@@ -747,6 +941,14 @@ ahip_pop_args make_args(ahip_net* net, Pop& p, int32_t step) {
         a.psum_stride[k] = q.n_rows;
         a.psum_part[k] = q.rate.perm.p;
     }
+    if (!p.model->spiking && p.depth > 1) {
+        a.push_buf[0] = p.hist.p;
+        a.push_depth[0] = p.depth;
+    }
+    if (p.rbuf.p) {
+        a.push_buf[1] = p.rbuf.p;
+        a.push_depth[1] = 2;
+    }
     return a;
 }
 
@@ -786,6 +988,7 @@ int enqueue_step(ahip_net* net, int32_t step, const std::vector<int32_t>& zero_b
             }
             continue;
         }
+        if (post.fused) continue;   // summed by the post population's update
         if (!transmits(net, p)) {
             // the sums of an active population are still cleared at every
             // step (OpenMPTemplates.py:266-276): a first writer that does not
@@ -833,7 +1036,8 @@ int enqueue_step(ahip_net* net, int32_t step, const std::vector<int32_t>& zero_b
         ahip_launch_fn fn = net->precision == AHIP_F64 ? p.model->launch_f64 : p.model->launch_f32;
         const bool probe_u = net->probe_kind == AHIP_PROBE_UPDATE && net->probe_proj == p.id;
         if (probe_u) HIPCHK(hipEventRecord(net->probe_ev[0], s));
-        int rc = fn(&a, (void*)s);
+        int rc = p.fused ? (net->precision == AHIP_F64 ? p.model->fused_f64 : p.model->fused_f32)(&a, &p.fuse, (void*)s)
+                         : fn(&a, (void*)s);
         if (rc != 0) return fail(AHIP_EHIP, "update of population %d failed: %s", p.id,
                                  hipGetErrorString((hipError_t)rc));
         if (probe_u) HIPCHK(hipEventRecord(net->probe_ev[1], s));
@@ -853,14 +1057,8 @@ int enqueue_step(ahip_net* net, int32_t step, const std::vector<int32_t>& zero_b
         if (p.model->spiking && p.fr_window > 0) LCHK(launch_update_rate(net, p, step, s));
         // delay queues: push this step's values (after the update and the
         // compaction, as the reference's update_delay)
-        if (p.depth > 1) {
-            if (p.model->spiking) {
-                LCHK(launch_push_spikes(net, p, step, s));
-            } else {
-                const int32_t rs = p.slot_index("r");
-                if (rs >= 0) LCHK(launch_push_values(net, p.slots[rs].p, p.hist.p, p.size, p.depth, step, s));
-            }
-        }
+        // (rates: by the update itself)
+        if (p.depth > 1 && p.model->spiking) LCHK(launch_push_spikes(net, p, step, s));
     }
     // plastic projections, after every population update: update_synapse,
     // then the post events (OpenMPBaseTemplate.py:217-325)
@@ -1217,6 +1415,7 @@ int ahip_set_time(ahip_net* net, int64_t t) {
     HIPCHK(hipStreamSynchronize(net->stream));
     HIPCHK(hipMemcpy(net->t_dev.p, &t, sizeof(int64_t), hipMemcpyHostToDevice));
     net->t = t;
+    net->rbuf_stale = true;
     return 0;
 }
 
@@ -1228,6 +1427,7 @@ int ahip_run(ahip_net* net, int64_t nsteps) {
     if (rc) return rc;
     std::vector<int32_t> zb;
     assign_accumulate(net, zb);
+    if ((rc = refresh_rates(net))) return rc;
     int64_t left = nsteps;
     const int32_t G = auto_batch(net);
     if (net->graph_enabled && left >= G) {
@@ -1401,6 +1601,7 @@ int ahip_pop_set(ahip_net* net, int32_t pop, const char* attr, const double* val
         HIPCHK(hipMemcpy(p->slots[k].p, f.data(), n * sizeof(float), hipMemcpyHostToDevice));
     }
     if (!p->model->slot_local[k]) p->slot_host_global[k] = values[0];
+    net->rbuf_stale = true;
     return 0;
 }
 
@@ -2266,6 +2467,7 @@ int ahip_time_kernel(ahip_net* net, int32_t what, int32_t index, int32_t iters, 
     }
     std::vector<int32_t> zb;
     assign_accumulate(net, zb);
+    if ((rc = refresh_rates(net))) return rc;
     HIPCHK(hipEventCreate(&net->probe_ev[0]));
     HIPCHK(hipEventCreate(&net->probe_ev[1]));
     net->probe_proj = index;

@@ -22,7 +22,7 @@
 extern "C" {
 #endif
 
-#define AHIP_MODEL_ABI 10
+#define AHIP_MODEL_ABI 11
 #define AHIP_MAX_SLOTS 48
 #define AHIP_MAX_RAND 8
 #define AHIP_UPDATE_BLOCK 256 /* threads per block of every update kernel */
@@ -78,9 +78,60 @@ typedef struct ahip_pop_args {
     int32_t psum_acc[AHIP_MAX_PSUM];
     int32_t psum_stride[AHIP_MAX_PSUM];
     const void* psum_part[AHIP_MAX_PSUM];
+    /* rate-coded: rings the update copies the new r to (depth 0: none), value
+     * of neuron i at push_buf[k][(t mod push_depth[k]) * size + i]: the delay
+     * queue and the two-step buffer that fused updates read */
+    void* push_buf[2];
+    int32_t push_depth[2];
 } ahip_pop_args;
 
 typedef int (*ahip_launch_fn)(const ahip_pop_args* args, void* stream);
+
+/* ---- psp and update of a rate-coded population in one launch --------------
+ * The rows (post neurons) of every projection into the population are summed
+ * by the update kernel itself, 2^lane_shift lanes per row, while the first
+ * update_waves waves of the workgroup load the neurons' values and draw their
+ * random numbers; they run the statements after a barrier.  Pre-synaptic rates come from rings indexed
+ * by the step (push_buf of the pre population's update), so no launch reads a
+ * rate that another workgroup of the same launch writes. */
+#define AHIP_MAX_FUSE 4
+#define AHIP_FUSE_CSR 0       /* ptr: row pointer; col, w: entries */
+#define AHIP_FUSE_SELL 1      /* ptr: slice offsets (SELL-C-sigma, 2^lane_shift threads per row) */
+#define AHIP_FUSE_DENSE 2     /* w: row-major, ld values per row; 64 lanes per row */
+#define AHIP_FUSE_CSR_DELAY 3 /* CSR with a delay (steps) per entry */
+#define AHIP_FUSE_MIX 4       /* launch: projections of several forms */
+#define AHIP_FUSE_THREADS 512
+#define AHIP_FUSE_STAGE_THREADS 1024
+#define AHIP_FUSE_ROWS 256    /* rows of a workgroup at most */
+#define AHIP_FUSE_DENSE_ROWS 8 /* of a dense projection alone */
+typedef struct ahip_fuse_proj {
+    int32_t kind;
+    int32_t sum;                        /* which psp sum of the model (slots of kind 2, in slot order) */
+    int32_t n_cols;                     /* pre-synaptic neurons */
+    int32_t depth;                      /* ring depth of x */
+    int32_t delay;                      /* x of step t: ring slot (t - delay) mod depth */
+    int32_t ld;                         /* dense: values per row, a multiple of 4 */
+    const int64_t* ptr;
+    const int32_t* col;
+    const void* w;
+    const int16_t* delays;
+    const void* x;                      /* ring of n_cols values per slot */
+} ahip_fuse_proj;
+typedef struct ahip_fuse_args {
+    int32_t n;                          /* projections, in creation order */
+    int32_t lane_shift;                 /* log2 of the lanes per row (0 .. 6) */
+    int32_t units;                      /* rows, or SELL slices of 64 >> lane_shift rows */
+    int32_t kind;                       /* the form of every projection, AHIP_FUSE_MIX: not one form */
+    int32_t blocks;                     /* workgroups */
+    int32_t share;                      /* units per workgroup */
+    int32_t update_waves;               /* waves that run the statements, 64 rows each */
+    int32_t stage;                      /* 1: x staged in LDS (lds_values values), 1024 threads */
+    int32_t lds_values;
+    uint32_t mask;                      /* psp sums that have a projection (bit = sum index) */
+    const int32_t* perm;                /* SELL: row of every slice position (-1: none), else NULL */
+    ahip_fuse_proj p[AHIP_MAX_FUSE];
+} ahip_fuse_args;
+typedef int (*ahip_fused_fn)(const ahip_pop_args* args, const ahip_fuse_args* fa, void* stream);
 
 /* ---- persistent steps of a small network --------------------------------
  * A network of one spiking population whose projections all start and end
@@ -152,6 +203,8 @@ typedef struct ahip_model_desc {
     ahip_persist_fn persist_f32;
     int32_t persist_n_slots;            /* local slots the persistent steps hold in LDS, in LDS order: */
     const int32_t* persist_slots;       /* those the statements touch and the conductances */
+    ahip_fused_fn fused_f64;            /* NULL for spiking models and models without a psp sum */
+    ahip_fused_fn fused_f32;
 } ahip_model_desc;
 
 /* Every model library exports this symbol. */

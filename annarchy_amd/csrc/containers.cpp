@@ -311,7 +311,7 @@ int build_layout(const Proj& p, int32_t precision, const ahip_format_opts& o, Ra
             // at off[s] + (e/g)*256 + 4*(b + e%g) + k%4 with e = k/4, so a
             // wave reads 4 synapses per lane with one 8-byte and one
             // 16/32-byte load.  Rows up to `cap` entries (twice the tile's
-            // mean, at least 64) get one lane and W = longest row / 4; a
+            // mean, at least 64; less where the tiles are few) get one lane and W = longest row / 4; a
             // longer row gets g = ceil(len/cap) lanes (at most 64), W follows
             // from it and the rows after it in the slice get just enough
             // lanes to fit in W.  Columns are uint16, relative to the panel;
@@ -319,30 +319,41 @@ int build_layout(const Proj& p, int32_t precision, const ahip_format_opts& o, Ra
             // weight 0.  rowof[s][lane] = (g << 16) | row for the first lane
             // of a row, -1 for the others.
             const size_t es = precision == AHIP_F64 ? 8 : 4;
-            // automatic: panels of up to 20479 columns (160 KiB of LDS in
-            // FP64, one workgroup per CU), and tiles of at most 2048 rows,
-            // as tall as lets every tile run in one round on the device's
-            // workgroup slots (CUs x the panels one CU's LDS holds): every
-            // slot busy, none waiting for a second round
+            // panels of up to 20479 columns when not given (160 KiB of LDS in
+            // FP64, one workgroup per CU)
             int32_t pc = o.panel_cols > 0 ? o.panel_cols : 20479;
             if (pc > 65535 || (size_t)(pc + 1) * es > 160 * 1024) { err = "panel exceeds 160 KiB of LDS or 65535 columns"; return AHIP_EINVAL; }
             pc = equal_panels(p.n_cols, pc);
-            int32_t rb_rows = o.chunk;
-            if (rb_rows <= 0) {
-                const int64_t panels = std::max<int32_t>(1, (p.n_cols + pc - 1) / pc);
-                const int64_t slots = (int64_t)device_cus() * std::max<int64_t>(1, (160 * 1024) / ((int64_t)(pc + 1) * es));
-                const int64_t nrb = std::max<int64_t>(1, slots / panels);
-                rb_rows = (int32_t)std::min<int64_t>(2048, std::max<int64_t>(256, ((R + nrb - 1) / nrb + 63) / 64 * 64));
-            }
-            if (rb_rows < 64 || rb_rows > 8192 || rb_rows % 64) { err = "tile rows must be a multiple of 64 in 64..8192"; return AHIP_EINVAL; }
             const int32_t steps = o.lanes_per_row > 0 ? o.lanes_per_row : 4;
             const int32_t waves = o.sigma > 1 ? o.sigma : 4;
+            int32_t rb_rows = o.chunk > 0 ? o.chunk : 2048;
+            if (rb_rows < 64 || rb_rows > 8192 || rb_rows % 64) { err = "tile rows must be a multiple of 64 in 64..8192"; return AHIP_EINVAL; }
             if (waves != 4 && waves != 8) { err = "sliced tiles: waves per workgroup must be 4 or 8"; return AHIP_EINVAL; }
             if (!(steps == 2 || steps == 4 || steps == 8 || (steps == 1 && waves == 4))) {
                 err = "sliced tiles: steps in flight must be 2, 4 or 8 (1 with 4 waves)";
                 return AHIP_EINVAL;
             }
+            // With fewer tiles than CUs at the height asked for, lower tiles fill
+            // the device's workgroup slots (CUs x the panels one CU's LDS holds,
+            // at most 32 waves a CU) in one round; at the default height of very
+            // large networks the last round is made full.  With fewer than half
+            // as many, the panels are narrower too (two workgroups a CU in FP64)
+            // and a row is shared by several lanes, so that every wave has
+            // slices.  40000 x 400: 40 tiles of 2048 x 20000 took 128 us a step
+            // (83 in FP32), 512 of 320 x 10000 43 us (30).  More tiles than CUs
+            // stay as they are, each stages its panel: 20000 x 200, 395 tiles of
+            // 256 rows 17 us, 790 of 128 20.6 us.
+            const int32_t cus = device_cus();
+            const int64_t asked = (int64_t)std::max<int32_t>(1, (p.n_cols + pc - 1) / pc) * ((R + rb_rows - 1) / rb_rows);
+            const bool few = asked < cus / 2;
+            if (few) pc = equal_panels(p.n_cols, std::min(pc, 10239));
             const int32_t np = std::max<int32_t>(1, (p.n_cols + pc - 1) / pc);
+            if (o.chunk <= 0 || asked < cus) {
+                const int64_t fit = std::min<int64_t>((160 * 1024) / ((int64_t)(pc + 1) * es), 32 / waves);
+                const int64_t slots = (int64_t)cus * std::max<int64_t>(1, fit);
+                const int64_t nrb = std::max<int64_t>(1, slots / np);
+                rb_rows = (int32_t)std::min<int64_t>(rb_rows, std::max<int64_t>(few ? 64 : 256, ((R + nrb - 1) / nrb + 63) / 64 * 64));
+            }
             // ceil(R / rb_rows) row blocks whose boundaries split the synapses
             // evenly (the psp ends with its heaviest tile; uneven in-degrees
             // would make equal-height blocks uneven), a block at most 65535
@@ -395,7 +406,11 @@ int build_layout(const Proj& p, int32_t precision, const ahip_format_opts& o, Ra
                 const int32_t* c = cnt.data() + (size_t)t * hmax;
                 int64_t tile_nnz = 0;
                 for (int32_t lr = 0; lr < nr; lr++) tile_nnz += c[lr];
-                const int64_t cap = std::max<int64_t>(64, (2 * tile_nnz / nr + 3) / 4 * 4);
+                // entries of one lane at most: twice the tile's mean row, and
+                // where the tiles are few and low no more than leaves every wave
+                // three slices
+                int64_t cap = std::max<int64_t>(64, (2 * tile_nnz / nr + 3) / 4 * 4);
+                if (few) cap = std::min(cap, 4 * std::max<int64_t>(4, tile_nnz / (256 * 3 * waves)));
                 std::iota(order.begin(), order.begin() + nr, 0);
                 std::stable_sort(order.begin(), order.begin() + nr, [&](int32_t a, int32_t b) { return c[a] > c[b]; });
                 int32_t ns = 0;

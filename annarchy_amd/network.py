@@ -611,7 +611,17 @@ class Projection:
         if self.csr.nnz >= 0.6 * float(self.csr.n_rows) * self.csr.n_cols:
             return dict(fmt="dense")
         from . import selector
-        return selector.select(self.csr, mode="mlp")
+        chosen = selector.select(self.csr, mode="mlp")
+        # Of the two sliced-tile configurations the one of few wide panels when
+        # the narrow ones would be many: the network was trained on timings in
+        # which a network below 1e5 neurons left most CUs without a wide tile
+        # (us per step, narrow / wide: 20000 x 200 17 / 19, 25000 x 500 38 / 38,
+        # 40001 x 500 lognormal 65 / 54, 60000 x 200 53 / 37; in FP32 37 / 39 at
+        # 31000 x 600 lognormal, 40 / 42 at 40001 x 500, 19 / 14 at 50000 x 50).
+        wide = 30000 if self.net.precision in ("double", "float64", "f64") else 45000
+        if chosen == selector.CLASSES[0] and self.csr.n_cols > wide:
+            return dict(selector.CLASSES[-1])
+        return chosen
 
     def fixed_probability(self, probability, weights, delays=0.0, allow_self_connections=False,
                           storage_format=None, generator="numpy", **fmt):

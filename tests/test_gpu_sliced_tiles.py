@@ -1,0 +1,41 @@
+"""Sliced tiles (sell_panel) as the builder sizes them: fewer tiles than half the
+CUs (narrower panels, rows shared by several lanes), fewer than the CUs (lower
+tiles), at least as many (as asked).  One psp of ragged rows with empty and
+very long ones against the dense product in float64; FP64 to the summation
+bound K u sum|w r| (K <= 2000 terms: 1e-12 of the largest sum), FP32 rows are
+compensated: 2e-6, the bar of every psp format."""
+
+import numpy as np
+import pytest
+
+import annarchy_amd as ah
+from annarchy_amd import connectivity as conn
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("precision,tol", [("double", 1e-12), ("float", 2e-6)])
+@pytest.mark.parametrize("n,opts", [
+    (1, dict(panel_cols=64, chunk=64)), (63, dict(panel_cols=20, chunk=64, sigma=8, lanes=2)),
+    (1500, dict(panel_cols=300, chunk=2048, sigma=8, lanes=2)),     # 5 tiles asked: few
+    (2000, dict(panel_cols=500, chunk=64, sigma=8, lanes=4)),       # 128 asked: lower, not narrower
+    (2900, dict(panel_cols=300, chunk=64, lanes=4)),                # 460 asked: kept
+])
+def test_tile_heights(gpu, n, opts, precision, tol):
+    rng = np.random.default_rng(n)
+    deg = np.minimum(n, rng.integers(0, 120, n))
+    deg[::5] = 0
+    deg[:: max(1, n // 7)] = min(n, 2000)
+    csr = conn.random_in_degree(n, n, rng, deg, conn.Normal(0.0, 0.1, rng=rng))
+    r0 = rng.random(n)
+    net = ah.Network(dt=1.0, seed=3, precision=precision)
+    pop = net.create(n, ah.RateNoisy)
+    proj = net.connect(pop, pop, "exc").from_csr(csr, storage_format="sell_panel", **opts)
+    net.compile()
+    pop.r = r0
+    pop.inject_random(0, np.zeros((1, n)))
+    net.step()
+    ref = csr.dense() @ (r0 if precision == "double" else r0.astype(np.float32).astype(np.float64))
+    np.testing.assert_allclose(np.asarray(pop.sum("exc")).reshape(-1), ref, rtol=0,
+                               atol=tol * max(1.0, np.max(np.abs(ref))))
+    assert proj.get_format()["panel_cols"] <= opts["panel_cols"]

@@ -28,7 +28,7 @@ import re
 
 from .equations import DISTRIBUTIONS, NeuronDescription, analyse_neuron, equation_code
 
-ABI = 11  # AHIP_MODEL_ABI in include/annarchy_hip_model.h
+ABI = 12  # AHIP_MODEL_ABI in include/annarchy_hip_model.h
 
 _PRELUDE = r"""// Generated neuron-model library for the MI355X simulation backend.
 // Model: %(name)s
@@ -93,12 +93,14 @@ __global__ __launch_bounds__(AHIP_UPDATE_BLOCK) void local_update(ahip_pop_args 
 %(reg_post)s
     bool _spike = false;
     if (_act) {
+%(rec_before)s
 %(refrac_in)s
 %(local_rand)s
 %(local_eqs)s
 %(refrac_dec)s
 %(gather)s
 %(reg_out)s
+%(rec_after)s
     }
     (void)_spike;
 %(publish)s
@@ -279,6 +281,8 @@ __global__ __launch_bounds__(AHIP_PERSIST_THREADS) void persistent_steps(ahip_po
         for (int32_t j = tid; j <= P.n_cols; j += AHIP_PERSIST_THREADS) cols[P.lds_cols + j] = (int32_t)P.col_ptr[j];
     }
     const int64_t t0 = *a.t_base + a.step;
+    const int64_t rec_t0 = pa.rec_counts ? pa.rec_state->t_start : 0;
+    const int64_t rec_rows = pa.rec_counts ? pa.rec_state->capacity : 0;
     const T dt = (T)a.dt;
     (void)dt;
 %(global_loads)s
@@ -398,8 +402,8 @@ __global__ __launch_bounds__(AHIP_PERSIST_THREADS) void persistent_steps(ahip_po
         //    counts; four rounds per pass, one 16-bit count each), recording
         int64_t slot = -1, f = 0;
         if (pa.rec_counts) {
-            slot = t - pa.rec_t_start;
-            if (slot >= 0 && slot < pa.rec_capacity) f = fill_s[slot & 1];
+            slot = t - rec_t0;
+            if (slot >= 0 && slot < rec_rows) f = fill_s[slot & 1];
             else slot = -1;
         }
         int32_t base = 0;
@@ -537,6 +541,7 @@ __global__ __launch_bounds__(STAGE ? AHIP_FUSE_STAGE_THREADS : AHIP_FUSE_THREADS
     if (_act) {
 %(local_eqs)s
 %(reg_out)s
+%(rec_after)s
     }
 }
 
@@ -890,6 +895,18 @@ def generate(desc: NeuronDescription, stop_condition: str | None = None) -> Mode
         r_now = _u("r") + ("__r" if lreads(_u("r")) else "[i]")
         reg_out.append(f"        ahip::push_rate<T>(a, t, i, {r_now});")
 
+    # value monitors: the value in its register, where it has one
+    def record_code(before: int) -> str:
+        cases = "".join(f" case {slot_of[n]}: _v = {_u(n)}__r; break;" for n in local_names if lreads(_u(n)))
+        return (f"        for (int _k = 0; _k < a.n_rec; _k++) {{\n"
+                f"            if (a.rec_before[_k] != {before}) continue;\n"
+                f"            T _v;\n"
+                f"            switch (a.rec_slot[_k]) {{{cases} default: _v = ((const T*)a.slot[a.rec_slot[_k]])[i]; }}\n"
+                f"            ahip::record_value<T>(a, _k, t, i, _v);\n"
+                f"        }}")
+    rec_after = record_code(0)
+    rec_before = record_code(1) if desc.spiking else ""
+
     fused_fn, fused_ptrs = "", "nullptr, nullptr"
     if ring_r and sums:
         fused_fn = _FUSED_KERNEL % {
@@ -905,6 +922,7 @@ def generate(desc: NeuronDescription, stop_condition: str | None = None) -> Mode
                        r'    asm volatile("" ::"v"(\1));', line) for line in lparts["local_rand"].split("\n")),
             "local_eqs": _indent(lparts["local_eqs"], 8),
             "reg_out": "\n".join(reg_out + sum_out),
+            "rec_after": rec_after,
             "launch_global": launch_global,
         }
         fused_ptrs = "fused_f64, fused_f32"
@@ -928,6 +946,8 @@ def generate(desc: NeuronDescription, stop_condition: str | None = None) -> Mode
         "reg_pre": "\n".join(reg_pre),
         "reg_post": "\n".join(reg_post),
         "reg_out": "\n".join(reg_out),
+        "rec_before": rec_before,
+        "rec_after": rec_after,
         "publish": publish,
         "launch_global": launch_global,
         "preloop_fn": preloop_fn,

@@ -207,6 +207,24 @@ __device__ inline int64_t mod_pos(int64_t u, int64_t n) {
 
 __device__ inline int64_t sim_time(const ahip_pop_args& a) { return *a.t_base + a.step; }
 
+// Row of a monitor at step t, -1: not recorded.
+__device__ inline int64_t record_row(const ahip_record_state& st, int64_t t) {
+    const int64_t d = t - st.t_start;
+    if (d < 0) return -1;
+    int64_t k = d;
+    if (st.period != 1) {
+        if (mod_pos(d, st.period) != 0) return -1;
+        k = (d >> 32) == 0 && (st.period >> 32) == 0 ? (int64_t)((uint32_t)d / (uint32_t)st.period) : d / st.period;
+    }
+    return st.base + k < st.capacity ? st.base + k : -1;
+}
+// Value v of neuron i into monitor k of the update.
+template <typename T>
+__device__ inline void record_value(const ahip_pop_args& a, int k, int64_t t, int32_t i, T v) {
+    const int64_t row = record_row(*a.rec_state[k], t);
+    if (row >= 0) static_cast<T*>(a.rec_data[k])[row * a.size + i] = v;
+}
+
 // The panel partial sums of row r of a sliced-tile psp, added in ascending
 // panel order (FP32: compensated), the one sequence both the psp's own
 // reduction and an update that completes the sum use.

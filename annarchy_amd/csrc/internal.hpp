@@ -162,6 +162,8 @@ struct Monitor {
     int64_t phase = 0;
     int64_t seg_base = 0;
     bool paused = false;
+    bool in_update = false;       // values: recorded by the population's update
+    DevBuf state;                 // ahip_record_state: what the kernels read of the above
     DevBuf data;                  // values [capacity][size] (T), or spike indices
     DevBuf counts;                // spikes: int32[capacity]
     DevBuf fill;                  // spikes: int64[2], indices written before recorded step s in fill[s & 1]
@@ -266,6 +268,10 @@ struct ahip_net {
     int32_t graph_batch = 0;
     hipGraphExec_t graph_exec = nullptr;
     int32_t graph_steps = 0;
+    // a run's remainder below a batch: its own graph, once the same length comes
+    // a second time
+    hipGraphExec_t rest_exec = nullptr;
+    int32_t rest_steps = 0, rest_seen = 0;
     bool dirty = true;             // structure changed since the last capture
     bool scatter_dirty = true;     // the fused scatter tables need rebuilding
     uint64_t scatter_gen = 0;       // bumped whenever the scatter tables are rebuilt

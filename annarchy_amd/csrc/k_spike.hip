@@ -57,8 +57,7 @@ struct SpikeRec {
     int32_t* idx;             // int32[idx_capacity]
     int64_t* fill;            // int64[2]
     int64_t idx_capacity;
-    int64_t t_start;
-    int64_t capacity;
+    const ahip_record_state* state;
 };
 
 // One population's compaction: its buffers and its first spike monitor.
@@ -90,9 +89,9 @@ __device__ inline void compact_chunk(const CompactArgs& c, int32_t b, const int6
     for (int32_t k = threadIdx.x; k < ub0; k += kCompactThreads) part += c.bcnt[k];
     int64_t slot = -1, f = 0;
     if (rec.counts) {
-        slot = *t_base + step - rec.t_start;
-        if (slot >= 0 && slot < rec.capacity) f = rec.fill[slot & 1];
-        else slot = -1;
+        const int64_t fill0 = rec.fill[0], fill1 = rec.fill[1];
+        slot = record_row(*rec.state, *t_base + step);
+        if (slot >= 0) f = (slot & 1) ? fill1 : fill0;
     }
     // base = sum(bcnt[0..ub0))
     part = group_sum<kWave>(part);
@@ -352,13 +351,14 @@ __global__ __launch_bounds__(256) void deliver_ordered(const DeliverTarget* __re
 __global__ __launch_bounds__(256) void record_spikes(const int32_t* __restrict__ spiked,
                                                      const int32_t* __restrict__ count,
                                                      const int64_t* __restrict__ t_base,
-                                                     int32_t step, int64_t t_start,
-                                                     int64_t capacity, int32_t* __restrict__ counts,
+                                                     int32_t step,
+                                                     const ahip_record_state* __restrict__ state,
+                                                     int32_t* __restrict__ counts,
                                                      int32_t* __restrict__ idx,
                                                      int64_t idx_capacity,
                                                      int64_t* __restrict__ fill) {
-    const int64_t slot = *t_base + step - t_start;
-    if (slot < 0 || slot >= capacity) return;
+    const int64_t slot = record_row(*state, *t_base + step);
+    if (slot < 0) return;
     const int32_t n = *count;
     const int64_t f = fill[slot & 1];   // same double-buffered fill as compact_spikes
     for (int32_t k = threadIdx.x; k < n; k += 256)
@@ -435,8 +435,7 @@ int launch_compact(const ahip_net* net, const std::vector<int32_t>& pops, const 
                 c.rec.idx = m->data.as<int32_t>();
                 c.rec.fill = m->fill.as<int64_t>();
                 c.rec.idx_capacity = m->idx_capacity;
-                c.rec.t_start = m->t_start;
-                c.rec.capacity = m->capacity;
+                c.rec.state = m->state.as<ahip_record_state>();
             }
             B.b0[B.n + 1] = B.b0[B.n] + c.nb;
             B.n++;
@@ -489,7 +488,7 @@ int launch_spike_psp(const ahip_net* net, const Proj& p, const Pop& pre, void* t
 int launch_record_spikes(const Monitor& m, const Pop& p, const int64_t* t_base, int32_t step,
                          hipStream_t s) {
     hipLaunchKernelGGL(record_spikes, dim3(1), dim3(256), 0, s, p.spiked.as<int32_t>(),
-                       p.spike_count.as<int32_t>(), t_base, step, m.t_start, m.capacity,
+                       p.spike_count.as<int32_t>(), t_base, step, m.state.as<ahip_record_state>(),
                        m.counts.as<int32_t>(), m.data.as<int32_t>(), m.idx_capacity,
                        m.fill.as<int64_t>());
     return (int)hipGetLastError();

@@ -92,6 +92,12 @@ Monitor* get_mon(ahip_net* net, int32_t id) {
 // reallocation of one of them must come with a recapture.
 void drop_graph(ahip_net* net) {
     net->dirty = true;
+    net->rest_seen = 0;
+    if (net->rest_exec) {
+        hipGraphExecDestroy(net->rest_exec);
+        net->rest_exec = nullptr;
+        net->rest_steps = 0;
+    }
     if (net->graph_exec) {
         hipGraphExecDestroy(net->graph_exec);
         net->graph_exec = nullptr;
@@ -464,7 +470,8 @@ int build_ordered_targets(ahip_net* net, const std::vector<const void*>& targets
         }
         for (auto& mp : net->mons) {
             const Monitor& m = *mp;
-            if (m.after_psp && m.pop == o.pop && net->pops[o.pop]->slots[m.slot].p == g) o.in_update = false;
+            if (m.after_psp && !m.in_update && m.pop == o.pop && net->pops[o.pop]->slots[m.slot].p == g)
+                o.in_update = false;
         }
         int32_t fused_here = 0;
         for (const OrderedTarget& q : net->ordered)
@@ -526,6 +533,22 @@ int build_ordered_targets(ahip_net* net, const std::vector<const void*>& targets
 
 static int plan_fused(ahip_net* net);
 
+// The value monitors that an update records: up to AHIP_MAX_REC of an active
+// population; not the firing rate, which its own kernel writes later.
+static void assign_records(ahip_net* net) {
+    std::vector<int32_t> n(net->pops.size(), 0);
+    for (auto& mp : net->mons) {
+        Monitor& m = *mp;
+        m.in_update = false;
+        if (m.spikes || m.paused) continue;
+        const Pop& p = *net->pops[m.pop];
+        if (!p.active || n[m.pop] >= AHIP_MAX_REC) continue;
+        if (p.model->spiking && p.fr_window > 0 && m.slot == p.slot_index("r")) continue;
+        m.in_update = true;
+        n[m.pop]++;
+    }
+}
+
 int prepare(ahip_net* net) {
     if (!net->initialized) return fail(AHIP_ESTATE, "network not initialized");
     for (auto& pp : net->projs) {
@@ -534,6 +557,7 @@ int prepare(ahip_net* net) {
     }
     int rc0 = ensure_delay_buffers(net);
     if (rc0) return rc0;
+    assign_records(net);
     for (auto& pp : net->pops) {
         Pop& p = *pp;
         if (p.active || p.depth <= 1 || !p.hist.p) continue;
@@ -876,7 +900,7 @@ static void assign_deferred_reduce(ahip_net* net) {
         for (auto& qq : net->projs)
             if (qq.get() != &p && qq->post == p.post && qq->target_slot == p.target_slot) alone = false;
         for (auto& mp : net->mons)
-            if (mp->after_psp && mp->pop == p.post && mp->slot == p.target_slot) alone = false;
+            if (mp->after_psp && !mp->in_update && mp->pop == p.post && mp->slot == p.target_slot) alone = false;
         if (!alone || n_def[p.post] >= AHIP_MAX_PSUM) continue;
         n_def[p.post]++;
         p.defer_reduce = true;
@@ -949,6 +973,17 @@ ahip_pop_args make_args(ahip_net* net, Pop& p, int32_t step) {
         a.push_buf[1] = p.rbuf.p;
         a.push_depth[1] = 2;
     }
+    for (auto& mp : net->mons) {
+        const Monitor& m = *mp;
+        if (!m.in_update || m.pop != p.id) continue;
+        const int32_t k = a.n_rec++;
+        a.rec_slot[k] = m.slot;
+        // psp sums of a rate-coded population stay what they are: recorded
+        // with the rest
+        a.rec_before[k] = m.after_psp && p.model->spiking ? 1 : 0;
+        a.rec_state[k] = m.state.as<ahip_record_state>();
+        a.rec_data[k] = m.data.p;
+    }
     return a;
 }
 
@@ -1010,7 +1045,7 @@ int enqueue_step(ahip_net* net, int32_t step, const std::vector<int32_t>& zero_b
     // 2. record targets
     for (auto& mp : net->mons) {
         Monitor& m = *mp;
-        if (!m.after_psp || m.paused) continue;
+        if (!m.after_psp || m.paused || m.in_update) continue;
         Pop& p = *net->pops[m.pop];
         LCHK(launch_record_values(m, p.slots[m.slot].p, p.size, (int32_t)es,
                                   net->t_dev.as<int64_t>(), step, s));
@@ -1077,7 +1112,7 @@ int enqueue_step(ahip_net* net, int32_t step, const std::vector<int32_t>& zero_b
     // 5. record variables and spikes
     for (auto& mp : net->mons) {
         Monitor& m = *mp;
-        if (m.after_psp || m.paused) continue;
+        if (m.after_psp || m.paused || m.in_update) continue;
         Pop& p = *net->pops[m.pop];
         if (m.spikes) {
             // an inactive population keeps its last spike list, which its
@@ -1169,8 +1204,7 @@ bool persist_plan(const ahip_net* net, ahip_persist_args& pa, size_t& lds, int32
         pa.rec_idx = rec->data.as<int32_t>();
         pa.rec_fill = rec->fill.as<int64_t>();
         pa.rec_idx_capacity = rec->idx_capacity;
-        pa.rec_t_start = rec->t_start;
-        pa.rec_capacity = rec->capacity;
+        pa.rec_state = rec->state.as<ahip_record_state>();
     }
     pop_id = 0;
     return true;
@@ -1205,8 +1239,7 @@ int enqueue_batch(ahip_net* net, int32_t nsteps, const std::vector<int32_t>& zb)
 // Captures `steps` steps with the scatter tables and buffers that prepare()
 // left in place (it must run first); only the previous executable graph is
 // dropped, so the tables stay valid for as long as the new graph lives.
-int build_graph(ahip_net* net, int32_t steps, const std::vector<int32_t>& zb) {
-    drop_graph(net);
+int capture_steps(ahip_net* net, int32_t steps, const std::vector<int32_t>& zb, hipGraphExec_t* exec) {
     HIPCHK(hipStreamBeginCapture(net->stream, hipStreamCaptureModeThreadLocal));
     int rc = enqueue_batch(net, steps, zb);
     hipGraph_t g = nullptr;
@@ -1216,15 +1249,49 @@ int build_graph(ahip_net* net, int32_t steps, const std::vector<int32_t>& zb) {
         return rc;
     }
     if (e != hipSuccess) return fail(AHIP_EHIP, "graph capture failed: %s", hipGetErrorString(e));
-    e = hipGraphInstantiate(&net->graph_exec, g, nullptr, nullptr, 0);
+    e = hipGraphInstantiate(exec, g, nullptr, nullptr, 0);
     hipGraphDestroy(g);
     if (e != hipSuccess) {
-        net->graph_exec = nullptr;
+        *exec = nullptr;
         return fail(AHIP_EHIP, "graph instantiation failed: %s", hipGetErrorString(e));
     }
+    return 0;
+}
+
+int build_graph(ahip_net* net, int32_t steps, const std::vector<int32_t>& zb) {
+    drop_graph(net);
+    int rc = capture_steps(net, steps, zb, &net->graph_exec);
+    if (rc) return rc;
     net->graph_steps = steps;
     net->graph_scatter_gen = net->scatter_gen;
     net->dirty = false;
+    return 0;
+}
+
+// The remainder of a run, shorter than a batch: launched step by step the first
+// time a length comes up, from a graph of its own from the second time on (a
+// program that simulates the same interval again and again; an eager launch
+// costs the host about twice what a graph node costs the GPU).
+constexpr int32_t kRestMin = 8;
+int run_rest(ahip_net* net, int32_t n, const std::vector<int32_t>& zb) {
+    if (!net->graph_enabled || n < kRestMin) return enqueue_batch(net, n, zb);
+    if (net->rest_exec && net->rest_steps == n && net->graph_scatter_gen == net->scatter_gen && !net->scatter_dirty) {
+        HIPCHK(hipGraphLaunch(net->rest_exec, net->stream));
+        return 0;
+    }
+    if (net->rest_seen != n) {
+        net->rest_seen = n;
+        return enqueue_batch(net, n, zb);
+    }
+    if (net->rest_exec) {
+        hipGraphExecDestroy(net->rest_exec);
+        net->rest_exec = nullptr;
+    }
+    int rc = capture_steps(net, n, zb, &net->rest_exec);
+    if (rc) return rc;
+    net->rest_steps = n;
+    net->graph_scatter_gen = net->scatter_gen;
+    HIPCHK(hipGraphLaunch(net->rest_exec, net->stream));
     return 0;
 }
 
@@ -1443,7 +1510,7 @@ int ahip_run(ahip_net* net, int64_t nsteps) {
     }
     while (left > 0) {
         const int32_t n = (int32_t)std::min<int64_t>(left, G);
-        rc = enqueue_batch(net, n, zb);
+        rc = n < G ? run_rest(net, n, zb) : enqueue_batch(net, n, zb);
         if (rc) return rc;
         left -= n;
     }
@@ -2549,6 +2616,14 @@ int ahip_scatter_groups(ahip_net* net, int32_t* n_groups) {
 
 // ---- monitors ---------------------------------------------------------------
 
+// What the recording kernels read of a monitor; the stream is idle.
+static int write_record_state(const Monitor& m) {
+    // spikes: rows count from t_start (the rows of earlier segments included)
+    const ahip_record_state st = {m.t_start, m.spikes ? 0 : m.seg_base, m.spikes ? 1 : m.period, m.capacity};
+    HIPCHK(hipMemcpy(m.state.p, &st, sizeof(st), hipMemcpyHostToDevice));
+    return 0;
+}
+
 int ahip_monitor_create(ahip_net* net, int32_t pop, const char* attr, int64_t capacity,
                         int32_t* mon_id) {
     Pop* p = get_pop(net, pop);
@@ -2577,6 +2652,8 @@ int ahip_monitor_create(ahip_net* net, int32_t pop, const char* attr, int64_t ca
         m->after_psp = (kind == 2) || (p->model->spiking && !strncmp(attr, "g_", 2));
         if ((rc = dev_alloc(m->data, (size_t)capacity * p->size * net->elem()))) return rc;
     }
+    if ((rc = dev_alloc(m->state, sizeof(ahip_record_state)))) return rc;
+    if ((rc = write_record_state(*m))) return rc;
     *mon_id = m->id;
     net->mons.push_back(std::move(m));
     invalidate(net);
@@ -2622,7 +2699,7 @@ int ahip_monitor_set_period(ahip_net* net, int32_t mon, int32_t period, int64_t 
         m->t_start = first_record_step(net->t, phase, period);
     }
     invalidate(net);
-    return 0;
+    return write_record_state(*m);
 }
 
 int ahip_monitor_pause(ahip_net* net, int32_t mon) {
@@ -2653,7 +2730,7 @@ int ahip_monitor_resume(ahip_net* net, int32_t mon) {
     // recorded step); values: the next step on the period grid
     m->t_start = m->spikes ? net->t - m->seg_base : first_record_step(net->t, m->phase, m->period);
     invalidate(net);
-    return 0;
+    return write_record_state(*m);
 }
 
 int ahip_monitor_get(ahip_net* net, int32_t mon, double* out, int64_t n) {
@@ -2707,8 +2784,8 @@ int ahip_monitor_clear(ahip_net* net, int32_t mon) {
         m->seg_base = 0;
         m->t_start = first_record_step(net->t, m->phase, m->period);
     }
-    invalidate(net);
-    return 0;
+    // the captured steps read the state: they stay
+    return write_record_state(*m);
 }
 
 }  // extern "C"

@@ -22,7 +22,7 @@
 extern "C" {
 #endif
 
-#define AHIP_MODEL_ABI 11
+#define AHIP_MODEL_ABI 12
 #define AHIP_MAX_SLOTS 48
 #define AHIP_MAX_RAND 8
 #define AHIP_UPDATE_BLOCK 256 /* threads per block of every update kernel */
@@ -47,6 +47,14 @@ typedef struct ahip_deliver_desc {
 #define AHIP_HEAD_COUNT ((1ull << AHIP_HEAD_SHIFT) - 1ull)
 #define AHIP_MAX_DELIVER 4 /* ordered conductances one update delivers */
 #define AHIP_MAX_PSUM 2    /* psp sums one update completes from panel partials */
+
+/* Recording of a monitor, in device memory (the host rewrites it when the
+ * monitor is emptied; a captured step reads it): step t_start + k * period goes
+ * to row base + k, below capacity. */
+typedef struct ahip_record_state {
+    int64_t t_start, base, period, capacity;
+} ahip_record_state;
+#define AHIP_MAX_REC 4     /* value monitors one update records */
 
 /* Arguments of one population update launch.  Device pointers unless noted. */
 typedef struct ahip_pop_args {
@@ -83,6 +91,14 @@ typedef struct ahip_pop_args {
      * queue and the two-step buffer that fused updates read */
     void* push_buf[2];
     int32_t push_depth[2];
+    /* value monitors the update records: local slot rec_slot[k] of every
+     * neuron, before its statements (after compute_psp) or after them, into
+     * rows of `size` values */
+    int32_t n_rec;
+    int32_t rec_slot[AHIP_MAX_REC];
+    int32_t rec_before[AHIP_MAX_REC];
+    const ahip_record_state* rec_state[AHIP_MAX_REC];
+    void* rec_data[AHIP_MAX_REC];
 } ahip_pop_args;
 
 typedef int (*ahip_launch_fn)(const ahip_pop_args* args, void* stream);
@@ -168,8 +184,7 @@ typedef struct ahip_persist_args {
     int32_t* rec_idx;
     int64_t* rec_fill;
     int64_t rec_idx_capacity;
-    int64_t rec_t_start;
-    int64_t rec_capacity;
+    const ahip_record_state* rec_state;
 } ahip_persist_args;
 typedef int (*ahip_persist_fn)(const ahip_pop_args* args, const ahip_persist_args* pa, size_t lds_bytes,
                                void* stream);

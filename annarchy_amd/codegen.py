@@ -1013,7 +1013,8 @@ __device__ inline bool update_due(const ahip_syn_args& a, int64_t t) {
 template <typename T>
 __global__ __launch_bounds__(256) void pre_event(ahip_syn_args a) {
     const int lane = threadIdx.x & (ahip::kWave - 1);
-    const int wid = threadIdx.x / ahip::kWave;
+    // the wave's index, uniform: lists, counts and ranges by scalar loads
+    const int32_t wid = __builtin_amdgcn_readfirstlane((int32_t)blockIdx.x * 4 + (int32_t)(threadIdx.x / ahip::kWave));
     const int64_t t = *a.t_base + a.step;
     const T dt = (T)a.dt;
     const int32_t _plasticity = a.plasticity;
@@ -1026,23 +1027,21 @@ __global__ __launch_bounds__(256) void pre_event(ahip_syn_args a) {
     (void)dt; (void)_plasticity; (void)_last_event; (void)_pre_last_spike; (void)_post_last_spike;
 %(ev_attrs)s
 %(deps)s
-    int64_t slot = 0;
-    if (a.pre_depth > 1) {
-        slot = (t - a.pre_delay) %% a.pre_depth;
-        if (slot < 0) slot += a.pre_depth;
-    }
-    const int32_t n = a.pre_count[slot];
+    const int64_t slot = a.pre_depth > 1 ? ahip::mod_pos(t - a.pre_delay, a.pre_depth) : 0;
     const int32_t* __restrict__ list = a.pre_spiked + slot * a.pre_stride;
-    const int32_t ch = a.pre_chunks;
-    const int64_t items = (int64_t)n * ch;
-    const int64_t waves = (int64_t)gridDim.x * 4;
-    for (int64_t it = (int64_t)blockIdx.x * 4 + wid; it < items; it += waves) {
-        const int64_t s = it / ch;
-        const int32_t c = (int32_t)(it - s * ch);
-        const int32_t pre = list[s];
+    const ahip::EventWalk W(wid, (int32_t)gridDim.x * 4, a.pre_chunks);
+    // (a list never holds more than n_cols entries: the first one loads with the count)
+    int32_t s = W.s0, c = W.c0;
+    int32_t next = s < a.n_cols ? list[s] : -1;
+    const int32_t n = a.pre_count[slot];
+    while (s < n) {
+        const int32_t pre = next, cc = c;
+        W.step(s, c);
+        next = s < n ? list[s] : -1;
         if (pre < 0 || pre >= a.n_cols) continue;
+        const int32_t ch = a.pre_chunks;
         const int64_t e = a.col_ptr[pre + 1];
-        for (int64_t q = a.col_ptr[pre] + (int64_t)c * ahip::kWave + lane; q < e; q += (int64_t)ch * ahip::kWave) {
+        for (int64_t q = a.col_ptr[pre] + (int64_t)cc * ahip::kWave + lane; q < e; q += (int64_t)ch * ahip::kWave) {
             const int32_t post = a.row_idx[q];
 %(pre_body)s
         }
@@ -1055,7 +1054,8 @@ __global__ __launch_bounds__(256) void pre_event(ahip_syn_args a) {
 template <typename T>
 __global__ __launch_bounds__(256) void post_event(ahip_syn_args a) {
     const int lane = threadIdx.x & (ahip::kWave - 1);
-    const int wid = threadIdx.x / ahip::kWave;
+    // the wave's index, uniform: lists, counts and ranges by scalar loads
+    const int32_t wid = __builtin_amdgcn_readfirstlane((int32_t)blockIdx.x * 4 + (int32_t)(threadIdx.x / ahip::kWave));
     const int64_t t = *a.t_base + a.step;
     const T dt = (T)a.dt;
     const int32_t _plasticity = a.plasticity;
@@ -1067,17 +1067,18 @@ __global__ __launch_bounds__(256) void post_event(ahip_syn_args a) {
     (void)dt; (void)_plasticity; (void)_last_event; (void)_pre_last_spike; (void)_post_last_spike;
 %(ev_attrs)s
 %(deps)s
+    const ahip::EventWalk W(wid, (int32_t)gridDim.x * 4, a.post_chunks);
+    int32_t s = W.s0, c = W.c0;
+    int32_t next = s < a.n_rows ? a.post_spiked[s] : -1;
     const int32_t n = *a.post_count;
-    const int32_t ch = a.post_chunks;
-    const int64_t items = (int64_t)n * ch;
-    const int64_t waves = (int64_t)gridDim.x * 4;
-    for (int64_t it = (int64_t)blockIdx.x * 4 + wid; it < items; it += waves) {
-        const int64_t s = it / ch;
-        const int32_t c = (int32_t)(it - s * ch);
-        const int32_t i = a.post_spiked[s];
+    while (s < n) {
+        const int32_t i = next, cc = c;
+        W.step(s, c);
+        next = s < n ? a.post_spiked[s] : -1;
         if (i < 0 || i >= a.n_rows) continue;
+        const int32_t ch = a.post_chunks;
         const int64_t e = a.row_ptr[i + 1];
-        for (int64_t j = a.row_ptr[i] + (int64_t)c * ahip::kWave + lane; j < e; j += (int64_t)ch * ahip::kWave) {
+        for (int64_t j = a.row_ptr[i] + (int64_t)cc * ahip::kWave + lane; j < e; j += (int64_t)ch * ahip::kWave) {
             const int64_t q = a.fwd2col ? a.fwd2col[j] : j;
             const int32_t pre = a.col_idx[j];
             const int32_t post = i;

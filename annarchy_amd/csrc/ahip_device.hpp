@@ -288,6 +288,26 @@ __device__ inline void publish_spikes(const ahip_pop_args& a, bool spk) {
     }
 }
 
+// Work items (spike s, chunk c) of a spike list, s major, dealt to the waves in
+// turn: a wave's next item without a division.
+struct EventWalk {
+    int32_t s0, c0, ds, dc, chunks;
+    __device__ inline EventWalk(int32_t wave, int32_t waves, int32_t ch) : chunks(ch) {
+        s0 = wave / ch;
+        c0 = wave - s0 * ch;
+        ds = waves / ch;
+        dc = waves - ds * ch;
+    }
+    __device__ inline void step(int32_t& s, int32_t& c) const {
+        s += ds;
+        c += dc;
+        if (c >= chunks) {
+            c -= chunks;
+            s++;
+        }
+    }
+};
+
 // ---- global-memory views -------------------------------------------------
 // A pointer read from a table in memory is generic to the compiler, which
 // then emits flat instructions (counted against the LDS wait counter as

@@ -284,6 +284,7 @@ struct ahip_net {
     ahip::DevBuf deliver_targets;               // DeliverTarget of the merged delivery launch
     int32_t deliver_n_tg = 0, deliver_waves = 0;
     int32_t delivery = AHIP_DELIVERY_ORDERED;
+    ahip::DevBuf io;               // staging of synaptic values between host and device, at most 32 MiB
     bool rbuf_stale = true;        // a rate changed outside a step since the rbufs were filled
     bool persist_enabled = true;   // small single-population networks: one launch per batch
     size_t elem() const { return precision == AHIP_F64 ? sizeof(double) : sizeof(float); }
@@ -335,6 +336,10 @@ int launch_record_values(const Monitor& m, const void* src, int32_t size, int32_
                          const int64_t* t_base, int32_t step, hipStream_t s);
 int launch_record_spikes(const Monitor& m, const Pop& p, const int64_t* t_base, int32_t step,
                          hipStream_t s);
+// field of synapse records <-> values in forward order (fwd2col of the chunk's
+// first synapse), doubles or int64
+int launch_syn_field(void* field, int32_t rec_bytes, int32_t elem, bool is_int, const int64_t* fwd2col, void* host_order,
+                     int64_t n, bool write, hipStream_t s);
 int launch_convert(const void* src, int32_t src_f64, void* dst, int32_t dst_f64, int64_t n,
                    hipStream_t s);
 int launch_copy16(const void* src, void* dst, int64_t n16, hipStream_t s);

@@ -2187,53 +2187,41 @@ int ahip_proj_nb_synapses(ahip_net* net, int32_t proj, int64_t* nnz) {
 
 // Per-synapse field of a plastic projection (field -1 = w, k = attribute k,
 // -2 = _last_event) between the device and a host array in forward order.
-// Spiking: fields of the column-order records, copied in chunks of records;
-// rate-coded: forward-order arrays.
+// Values that need a change of order (the column-order records of a spiking
+// projection) or of type (FP32) pass through a staging buffer of the network in
+// chunks, converted by a kernel; the others are copied as they are.
 static int syn_field_io(ahip_net* net, Proj& p, int field, double* dbl, int64_t* i64, bool write) {
     const size_t es = net->elem();
+    const bool is_int = field == -2;
+    char* host = is_int ? reinterpret_cast<char*>(i64) : reinterpret_cast<char*>(dbl);
+    HIPCHK(hipSetDevice(net->device));
     HIPCHK(hipStreamSynchronize(net->stream));
-    if (!p.spiking) {
-        void* dev = field == -1 ? p.rate.val.p : field == -2 ? p.last_event.p : p.syn_attr[field].p;
-        const size_t vb = field == -2 ? 8 : es;
-        std::vector<char> buf((size_t)p.nnz * vb);
-        if (write) {
-            for (int64_t q = 0; q < p.nnz; q++) {
-                if (field == -2) std::memcpy(&buf[q * 8], &i64[q], 8);
-                else if (es == 8) std::memcpy(&buf[q * 8], &dbl[q], 8);
-                else { const float f = (float)dbl[q]; std::memcpy(&buf[q * 4], &f, 4); }
-            }
-            if (p.nnz) HIPCHK(hipMemcpy(dev, buf.data(), buf.size(), hipMemcpyHostToDevice));
-        } else {
-            if (p.nnz) HIPCHK(hipMemcpy(buf.data(), dev, buf.size(), hipMemcpyDeviceToHost));
-            for (int64_t q = 0; q < p.nnz; q++) {
-                if (field == -2) std::memcpy(&i64[q], &buf[q * 8], 8);
-                else if (es == 8) std::memcpy(&dbl[q], &buf[q * 8], 8);
-                else { float f; std::memcpy(&f, &buf[q * 4], 4); dbl[q] = f; }
-            }
-        }
+    if (p.nnz == 0) return 0;
+    char* dev = !p.spiking ? (char*)(field == -1 ? p.rate.val.p : is_int ? p.last_event.p : p.syn_attr[field].p)
+                           : (char*)p.syn_rec.p + (field == -1 ? p.rec_off_w : is_int ? p.rec_off_last : p.rec_off[field]);
+    if (!p.spiking && (is_int || es == 8)) {
+        HIPCHK(hipMemcpy(write ? dev : host, write ? host : dev, (size_t)p.nnz * 8,
+                         write ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost));
         return 0;
     }
-    const int32_t off = field == -1 ? p.rec_off_w : field == -2 ? p.rec_off_last : p.rec_off[field];
-    const int64_t chunk = 1 << 20;
-    std::vector<char> buf((size_t)std::min<int64_t>(chunk, std::max<int64_t>(p.nnz, 1)) * p.rec_bytes);
-    for (int64_t q0 = 0; q0 < p.nnz; q0 += chunk) {
-        const int64_t m = std::min(chunk, p.nnz - q0);
-        char* dev = (char*)p.syn_rec.p + (size_t)q0 * p.rec_bytes;
-        HIPCHK(hipMemcpy(buf.data(), dev, (size_t)m * p.rec_bytes, hipMemcpyDeviceToHost));
-        for (int64_t i = 0; i < m; i++) {
-            char* r = buf.data() + (size_t)i * p.rec_bytes + off;
-            const int64_t j = p.h_inv_idx[q0 + i];
-            if (field == -2) {
-                if (write) std::memcpy(r, &i64[j], 8); else std::memcpy(&i64[j], r, 8);
-            } else if (es == 8) {
-                if (write) std::memcpy(r, &dbl[j], 8); else std::memcpy(&dbl[j], r, 8);
-            } else {
-                float f;
-                if (write) { f = (float)dbl[j]; std::memcpy(r, &f, 4); }
-                else { std::memcpy(&f, r, 4); dbl[j] = f; }
-            }
-        }
-        if (write) HIPCHK(hipMemcpy(dev, buf.data(), (size_t)m * p.rec_bytes, hipMemcpyHostToDevice));
+    const int64_t chunk = 1 << 22;
+    const size_t want = (size_t)std::min(chunk, p.nnz) * 8;
+    if (net->io.bytes < want) {
+        int rc = dev_alloc(net->io, want);
+        if (rc) return rc;
+    }
+    for (int64_t j0 = 0; j0 < p.nnz; j0 += chunk) {
+        const int64_t n = std::min(chunk, p.nnz - j0);
+        if (write) HIPCHK(hipMemcpy(net->io.p, host + j0 * 8, (size_t)n * 8, hipMemcpyHostToDevice));
+        if (p.spiking)
+            LCHK(launch_syn_field(dev, p.rec_bytes, (int32_t)es, is_int, p.fwd2col.as<int64_t>() + j0, net->io.p, n,
+                                  write, net->stream));
+        else if (write)
+            LCHK(launch_convert(net->io.p, 1, dev + j0 * es, 0, n, net->stream));
+        else
+            LCHK(launch_convert(dev + j0 * es, 0, net->io.p, 1, n, net->stream));
+        HIPCHK(hipStreamSynchronize(net->stream));
+        if (!write) HIPCHK(hipMemcpy(host + j0 * 8, net->io.p, (size_t)n * 8, hipMemcpyDeviceToHost));
     }
     return 0;
 }

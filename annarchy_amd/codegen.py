@@ -28,7 +28,7 @@ import re
 
 from .equations import DISTRIBUTIONS, NeuronDescription, analyse_neuron, equation_code
 
-ABI = 12  # AHIP_MODEL_ABI in include/annarchy_hip_model.h
+ABI = 13  # AHIP_MODEL_ABI in include/annarchy_hip_model.h
 
 _PRELUDE = r"""// Generated neuron-model library for the MI355X simulation backend.
 // Model: %(name)s
@@ -73,8 +73,11 @@ __global__ void global_update(ahip_pop_args a) {
 }
 """
 
+# The update has a second instance (EXTRA) for the populations with counted
+# events or recorded values: that code in the way of the others costs them 3 to
+# 4 % of a step (instructions to fetch, nothing to execute).
 _LOCAL_KERNEL = r"""
-template <typename T>
+template <typename T, bool EXTRA>
 __global__ __launch_bounds__(AHIP_UPDATE_BLOCK) void local_update(ahip_pop_args a) {
     const int32_t i = blockIdx.x * AHIP_UPDATE_BLOCK + threadIdx.x;
     const int64_t t = ahip::sim_time(a);
@@ -88,6 +91,7 @@ __global__ __launch_bounds__(AHIP_UPDATE_BLOCK) void local_update(ahip_pop_args 
     // (their loads overlap the delivery's)
 %(reg_pre)s
     // this step's spike events of the ordered conductances (end of compute_psp)
+%(counted)s
     if (a.n_deliver > 0 && _act) ahip::deliver_buckets<T>(a, i);
     asm volatile("" ::: "memory");  // the equations below read the delivered values
 %(reg_post)s
@@ -111,7 +115,11 @@ int launch(const ahip_pop_args* a, void* stream) {
     hipStream_t s = (hipStream_t)stream;
 %(launch_global)s
     const int nb = (a->size + AHIP_UPDATE_BLOCK - 1) / AHIP_UPDATE_BLOCK;
-    if (nb > 0) hipLaunchKernelGGL(local_update<T>, dim3(nb), dim3(AHIP_UPDATE_BLOCK), 0, s, *a);
+    if (nb <= 0) return 0;
+    if (a->n_counted > 0 || a->n_rec > 0)
+        hipLaunchKernelGGL((local_update<T, true>), dim3(nb), dim3(AHIP_UPDATE_BLOCK), 0, s, *a);
+    else
+        hipLaunchKernelGGL((local_update<T, false>), dim3(nb), dim3(AHIP_UPDATE_BLOCK), 0, s, *a);
     return (int)hipGetLastError();
 }
 
@@ -857,6 +865,8 @@ def generate(desc: NeuronDescription, stop_condition: str | None = None) -> Mode
     reg_fpre, reg_sum, sum_out = [], [], []
     kind_of = {s_[0]: s_[3] for s_ in slots}
     sums = [s_[0] for s_ in slots if s_[3] == 2]
+    # conductances that spike events reach
+    counted = desc.spiking and any(n.startswith("g_") for n in local_names)
     # a rate that other launches read from the population's rings
     ring_r = not desc.spiking and "r" in local_names
     cands = [(_u(n), "T", f"{_u(n)}[i]", n.startswith("g_")) for n in local_names]
@@ -886,11 +896,22 @@ def generate(desc: NeuronDescription, stop_condition: str | None = None) -> Mode
         else:
             reg_fpre.append(f"    {ty} {c}__r = _act ? {load} : {ty}(0);")
         (reg_post if after else reg_pre).append(f"    {ty} {c}__r = _act ? {load} : {ty}(0);")
+        if after and counted:
+            # the counted events of this conductance
+            store = "" if lwrites(c) else f" if (_act) {mem} = {c}__r;"
+            reg_post.append(f"    if constexpr (EXTRA) {{ {c}__r = ahip::add_counted<T>(a, _cnt, {slot_of[name]}, t, i, "
+                            f"{c}__r);{store} }}")
         if lwrites(c):
             reg_out.append(f"        {mem} = {c}__r;")
         for key in lparts:
             lparts[key] = re.sub(lref(c), c + "__r", lparts[key])
 
+    if counted:
+        for n in local_names:
+            # a conductance the statements do not read
+            if n.startswith("g_") and not lreads(_u(n)):
+                reg_post.append(f"    if (EXTRA && _act) {_u(n)}[i] = ahip::add_counted<T>(a, _cnt, {slot_of[n]}, "
+                                f"t, i, {_u(n)}[i]);")
     if ring_r:
         r_now = _u("r") + ("__r" if lreads(_u("r")) else "[i]")
         reg_out.append(f"        ahip::push_rate<T>(a, t, i, {r_now});")
@@ -944,10 +965,12 @@ def generate(desc: NeuronDescription, stop_condition: str | None = None) -> Mode
         "refrac_dec": _indent(lparts["refrac_dec"], 8),
         "gather": _indent(lparts["gather"], 8),
         "reg_pre": "\n".join(reg_pre),
+        "counted": ("    ahip::Counted<T> _cnt;\n"
+                    "    if constexpr (EXTRA) _cnt = ahip::load_counted<T>(a, t, i);") if counted else "",
         "reg_post": "\n".join(reg_post),
         "reg_out": "\n".join(reg_out),
-        "rec_before": rec_before,
-        "rec_after": rec_after,
+        "rec_before": f"        if constexpr (EXTRA) {{\n{rec_before}\n        }}" if rec_before else "",
+        "rec_after": f"        if constexpr (EXTRA) {{\n{rec_after}\n        }}",
         "publish": publish,
         "launch_global": launch_global,
         "preloop_fn": preloop_fn,

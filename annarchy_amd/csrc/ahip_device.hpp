@@ -447,6 +447,49 @@ __device__ inline void deliver_buckets(const ahip_pop_args& a, int32_t i) {
     }
 }
 
+// The counted events of neuron i at this step, all loads in flight together.
+template <typename T>
+struct Counted {
+    int32_t n[AHIP_MAX_COUNTED];
+    T sum[AHIP_MAX_COUNTED];
+};
+template <typename T>
+__device__ inline Counted<T> load_counted(const ahip_pop_args& a, int64_t t, int32_t i) {
+    Counted<T> c;
+#pragma unroll
+    for (int k = 0; k < AHIP_MAX_COUNTED; k++) {
+        c.n[k] = 0;
+        c.sum[k] = T(0);
+        if (k >= a.n_counted || i >= a.size) continue;
+        const ahip_counted_desc& d = a.counted[k];
+        const int64_t at = (t & (d.depth - 1)) * a.size + i;
+        if (d.sums) c.sum[k] = static_cast<const T*>(d.ring)[at];
+        else c.n[k] = static_cast<const int32_t*>(d.ring)[at];
+    }
+    return c;
+}
+// g + the counted events of conductance `slot`, projection by projection in
+// creation order, and the counts cleared.
+template <typename T>
+__device__ inline T add_counted(const ahip_pop_args& a, const Counted<T>& c, int32_t slot, int64_t t, int32_t i, T g) {
+#pragma unroll
+    for (int k = 0; k < AHIP_MAX_COUNTED; k++) {
+        if (k >= a.n_counted || a.counted[k].slot != slot) continue;
+        const ahip_counted_desc& d = a.counted[k];
+        if (c.n[k] == 0 && c.sum[k] == T(0)) continue;
+        const int64_t at = (t & (d.depth - 1)) * a.size + i;
+        if (d.sums) {
+            g += c.sum[k];
+            static_cast<T*>(d.ring)[at] = T(0);
+        } else {
+            const T w = (T)d.w;
+            for (int32_t m = 0; m < c.n[k]; m++) g += w;
+            static_cast<int32_t*>(d.ring)[at] = 0;
+        }
+    }
+    return g;
+}
+
 // Keep a value in vector registers (an empty asm that reads and writes it
 // there): a loop that would otherwise reload spilled scalar registers every
 // iteration reads the copy instead.  No arithmetic changes.

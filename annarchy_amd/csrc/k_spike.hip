@@ -250,6 +250,33 @@ __global__ __launch_bounds__(256) void scatter_multi(const ScatterArgs A, const 
         const T* wc = static_cast<const T*>(d.w_col);
         const auto wg = as_global(wc);
         const T wk = (T)d.w_const;
+        if (d.ring) {
+            // counted delivery: equal addends (or, with a weight and a delay per
+            // synapse, sums) wait in the slot of the step they arrive at
+            const int32_t now = d.delay_col ? (int32_t)(*t_base + step) - 1 : 0;
+            const auto dl = as_global(d.delay_col);
+            for (int64_t base = b + (int64_t)c * 256; base < e; base += (int64_t)d.chunks * 256) {
+                int32_t at[4];
+                T v[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int64_t j = base + lane + u * kWave;
+                    at[u] = -1;
+                    v[u] = T(0);
+                    if (j >= e) continue;
+                    const int32_t slot = d.delay_col ? (now + dl[j]) & (d.ring_depth - 1) : 0;
+                    at[u] = slot * d.n_post + ri[j];
+                    if (wc) v[u] = wg[j];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    if (at[u] < 0) continue;
+                    if (wc) unsafeAtomicAdd((T*)as_global(static_cast<T*>(d.ring) + at[u]), v[u]);
+                    else atomicAdd((int32_t*)as_global(static_cast<int32_t*>(d.ring) + at[u]), 1);
+                }
+            }
+            continue;
+        }
         if (d.head) {
             // ordered delivery: append (key gid_off + j, weight) to the post
             // neuron's bucket; each synapse fires at most once per step, so a

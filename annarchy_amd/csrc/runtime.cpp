@@ -189,9 +189,10 @@ int ensure_delay_buffers(ahip_net* net) {
             // pending events of steps [t, t + old depth) keep their delivery step
             const size_t slot = (size_t)p.n_rows * (p.single_w ? sizeof(int32_t) : es);
             const int32_t d_old = p.ring.p ? (int32_t)(p.ring.bytes / std::max<size_t>(slot, 1)) : 0;
-            if (!p.ring.p || d_old < p.max_delay) {
+            const int32_t d_new = std::max(p.ring_depth(), d_old);
+            if (!p.ring.p || d_old < d_new) {
                 HIPCHK(hipStreamSynchronize(net->stream));
-                int rc = regrow_ring(p.ring, slot, d_old, std::max(p.max_delay, d_old), net->t, net->t + d_old);
+                int rc = regrow_ring(p.ring, slot, d_old, d_new, net->t, net->t + d_old);
                 if (rc) return rc;
                 invalidate(net);
             }
@@ -465,7 +466,7 @@ int build_ordered_targets(ahip_net* net, const std::vector<const void*>& targets
         for (auto& pp : net->projs) {
             const Proj& p = *pp;
             if (net->pops[p.post]->slots[p.target_slot].p == g &&
-                std::find(o.projs.begin(), o.projs.end(), p.id) == o.projs.end() && transmits(net, p))
+                std::find(o.projs.begin(), o.projs.end(), p.id) == o.projs.end() && transmits(net, p) && !p.counted)
                 o.in_update = false;
         }
         for (auto& mp : net->mons) {
@@ -549,6 +550,50 @@ static void assign_records(ahip_net* net) {
     }
 }
 
+// Which spiking projections are counted (ahip_counted_desc): into a conductance
+// that no plastic projection and no monitor between compute_psp and the update
+// touches, with one weight each and no ordered delivery, or with a delay per
+// synapse; at most AHIP_MAX_COUNTED into a population.  Every such projection
+// then goes in one scatter launch (projections of different weights into one
+// conductance had to follow one another), and those with a delay per synapse
+// need neither their own scatter nor a delivery launch.
+static int assign_counted(ahip_net* net) {
+    for (auto& pp : net->projs) {
+        Proj& p = *pp;
+        p.counted = false;
+    }
+    for (auto& pop : net->pops) {
+        if (!pop->model->spiking || !pop->active) continue;
+        std::vector<Proj*> in;
+        for (auto& pp : net->projs)
+            if (pp->spiking && pp->post == pop->id && pp->nnz > 0 && transmits(net, *pp)) in.push_back(pp.get());
+        std::vector<Proj*> pick;
+        for (Proj* p : in) {
+            bool ok = !p->syn && (p->single_w || p->delay_per_syn) &&
+                      (int64_t)p->ring_depth() * p->n_rows < INT32_MAX;
+            for (const Proj* q : in) {
+                if (q->target_slot != p->target_slot) continue;
+                // plastic events add to the conductance themselves; ordered
+                // delivery keys single-weight projections beside it
+                if (q->syn || (!p->delay_per_syn && !q->delay_per_syn && !q->single_w)) ok = false;
+            }
+            for (auto& mp : net->mons)
+                if (mp->after_psp && !mp->in_update && !mp->paused && mp->pop == pop->id && mp->slot == p->target_slot) ok = false;
+            if (ok) pick.push_back(p);
+        }
+        if (pick.size() > AHIP_MAX_COUNTED) continue;
+        for (Proj* p : pick) {
+            p->counted = true;
+            if (!p->delay_per_syn && p->cnt.bytes < (size_t)p->n_rows * sizeof(int32_t)) {
+                drop_graph(net);
+                int rc = dev_alloc(p->cnt, (size_t)p->n_rows * sizeof(int32_t));
+                if (rc) return rc;
+            }
+        }
+    }
+    return 0;
+}
+
 int prepare(ahip_net* net) {
     if (!net->initialized) return fail(AHIP_ESTATE, "network not initialized");
     for (auto& pp : net->projs) {
@@ -558,6 +603,7 @@ int prepare(ahip_net* net) {
     int rc0 = ensure_delay_buffers(net);
     if (rc0) return rc0;
     assign_records(net);
+    if ((rc0 = assign_counted(net))) return rc0;
     for (auto& pp : net->pops) {
         Pop& p = *pp;
         if (p.active || p.depth <= 1 || !p.hist.p) continue;
@@ -581,11 +627,11 @@ int prepare(ahip_net* net) {
         std::vector<int64_t> blocks;
         std::vector<std::vector<const void*>> targets;
         auto fused = [&](const Proj& p) {
-            return p.spiking && p.nnz != 0 && !p.delay_per_syn && !p.syn && transmits(net, p);
+            return p.spiking && p.nnz != 0 && (!p.delay_per_syn || p.counted) && !p.syn && transmits(net, p);
         };
         std::vector<const void*> unordered;
         for (auto& pp : net->projs)
-            if (fused(*pp) && !pp->single_w) unordered.push_back(net->pops[pp->post]->slots[pp->target_slot].p);
+            if (fused(*pp) && !pp->counted && !pp->single_w) unordered.push_back(net->pops[pp->post]->slots[pp->target_slot].p);
         // ordered delivery: every fused projection into such a target appends
         // its events to the target's buckets (single-weight ones included, so
         // the projections' sums keep their creation order)
@@ -597,7 +643,7 @@ int prepare(ahip_net* net) {
             if (!fused(p)) continue;
             Pop& pre = *net->pops[p.pre];
             void* g = net->pops[p.post]->slots[p.target_slot].p;
-            const bool ordered = std::find(unordered.begin(), unordered.end(), g) == unordered.end();
+            const bool ordered = !p.counted && std::find(unordered.begin(), unordered.end(), g) == unordered.end();
             size_t k = 0;
             for (size_t q = 0; q < groups.size() && ordered; q++)
                 for (const void* t : targets[q])
@@ -638,8 +684,12 @@ int prepare(ahip_net* net) {
             d.shards = 1;
             d.shard_cap = 0;
             d.gid_off = 0;
+            d.ring = !p.counted ? nullptr : p.delay_per_syn ? p.ring.p : p.cnt.p;
+            d.delay_col = p.delay_per_syn ? p.delay_dev.as<int16_t>() : nullptr;
+            d.ring_depth = p.delay_per_syn ? p.ring_depth() : 1;
+            d.n_post = p.n_rows;
             for (OrderedTarget& o : net->ordered) {
-                if (o.g != g) continue;
+                if (o.g != g || p.counted) continue;
                 uint32_t off = 0;
                 for (size_t q = 0; q < o.projs.size(); q++)
                     if (o.projs[q] == p.id) off = (uint32_t)o.key_off[q];
@@ -654,7 +704,7 @@ int prepare(ahip_net* net) {
                 d.gid_off = off;
             }
             groups[k].push_back(d);
-            targets[k].push_back(g);
+            targets[k].push_back(p.counted ? nullptr : g);
             blocks[k] += ((int64_t)pre.size * p.scatter_chunks + 3) / 4;
         }
         // each descriptor of a group gets an equal share of the launch's
@@ -973,6 +1023,18 @@ ahip_pop_args make_args(ahip_net* net, Pop& p, int32_t step) {
         a.push_buf[1] = p.rbuf.p;
         a.push_depth[1] = 2;
     }
+    // the projections without a delay per synapse first, as their scatter was
+    for (int pass = 0; pass < 2; pass++)
+        for (auto& pp : net->projs) {
+            const Proj& q = *pp;
+            if (!q.counted || q.post != p.id || q.delay_per_syn != (pass == 1)) continue;
+            ahip_counted_desc& d = a.counted[a.n_counted++];
+            d.ring = q.delay_per_syn ? q.ring.p : q.cnt.p;
+            d.w = q.w_const;
+            d.slot = q.target_slot;
+            d.depth = q.delay_per_syn ? q.ring_depth() : 1;
+            d.sums = q.delay_per_syn && !q.single_w ? 1 : 0;
+        }
     for (auto& mp : net->mons) {
         const Monitor& m = *mp;
         if (!m.in_update || m.pop != p.id) continue;
@@ -1018,7 +1080,7 @@ int enqueue_step(ahip_net* net, int32_t step, const std::vector<int32_t>& zero_b
                     int rc = launch_syn(net, p, 0, step);
                     if (rc) return rc;
                 }
-            } else if (p.delay_per_syn && p.nnz > 0) {
+            } else if (p.delay_per_syn && p.nnz > 0 && !p.counted) {
                 LCHK(launch_spike_ring(net, p, pre, target, step, s));
             }
             continue;

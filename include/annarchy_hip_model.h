@@ -22,7 +22,7 @@
 extern "C" {
 #endif
 
-#define AHIP_MODEL_ABI 12
+#define AHIP_MODEL_ABI 13
 #define AHIP_MAX_SLOTS 48
 #define AHIP_MAX_RAND 8
 #define AHIP_UPDATE_BLOCK 256 /* threads per block of every update kernel */
@@ -47,6 +47,20 @@ typedef struct ahip_deliver_desc {
 #define AHIP_HEAD_COUNT ((1ull << AHIP_HEAD_SHIFT) - 1ull)
 #define AHIP_MAX_DELIVER 4 /* ordered conductances one update delivers */
 #define AHIP_MAX_PSUM 2    /* psp sums one update completes from panel partials */
+
+/* Spike events counted per post neuron: the scatter adds 1 (or, `sums`, the
+ * synapse's weight) at ring slot (arrival step) mod depth, a power of two, the
+ * update adds
+ * them to the conductance in slot `slot` before its statements, projection by
+ * projection, one addition of the weight per event, and clears them.  All
+ * addends of a projection are equal, so the result does not depend on the
+ * order in which the events were counted. */
+typedef struct ahip_counted_desc {
+    void* ring;                         /* depth x size int32 counts, or sums in the network precision */
+    double w;
+    int32_t slot, depth, sums, reserved;
+} ahip_counted_desc;
+#define AHIP_MAX_COUNTED 4 /* counted projections one update delivers */
 
 /* Recording of a monitor, in device memory (the host rewrites it when the
  * monitor is emptied; a captured step reads it): step t_start + k * period goes
@@ -99,6 +113,8 @@ typedef struct ahip_pop_args {
     int32_t rec_before[AHIP_MAX_REC];
     const ahip_record_state* rec_state[AHIP_MAX_REC];
     void* rec_data[AHIP_MAX_REC];
+    int32_t n_counted;
+    ahip_counted_desc counted[AHIP_MAX_COUNTED];
 } ahip_pop_args;
 
 typedef int (*ahip_launch_fn)(const ahip_pop_args* args, void* stream);

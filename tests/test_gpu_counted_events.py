@@ -1,0 +1,94 @@
+"""Spike events that the scatter counts and the post update adds.
+
+Projections of one weight each (no delay, one delay, a delay per synapse) and one
+with a weight and a delay per synapse into the same and into different
+conductances of one population.  The events of a step are added projection by
+projection, those without a delay per synapse first, one addition per event: a
+host loop in that order gives the same bits for the single-weight projections.
+The sums of the last projection arrive by atomics, in no fixed order: its
+conductance agrees to the rounding of its additions (in-degree 9 at most, values
+below 10: 1e-13).  With a fifth projection into the population, more than one
+update delivers, everything goes the other way (scatters and delivery launches)
+and has to give the same bits.  Delays up to 5 make a ring of 8 slots, 1 and 2
+its smallest."""
+
+import numpy as np
+import pytest
+
+import annarchy_amd as ah
+from annarchy_amd import connectivity as conn
+
+pytestmark = pytest.mark.gpu
+
+Every3 = ah.Neuron(equations="v = v + 1.0\nmp = t", spike="v == 3.0", reset="v = 0.0", name="Every3")
+LIF = ah.Neuron(
+    parameters="""
+    tau_m = 10.0    : population
+    E_L = -65.0     : population
+    V_th = -52.0    : population
+    V_r = -67.0     : population
+    tau_ref = 2.5
+    tau_s = 3.0     : population
+    I_b = 14.0      : population
+""", equations="""
+    tau_m * dv/dt = E_L - v + g_exc - g_inh + I_b : exponential
+    tau_s * dg_exc/dt = -g_exc : exponential
+    tau_s * dg_inh/dt = -g_inh : exponential
+""", spike="v > V_th", reset="v = V_r", refractory="tau_ref", name="LIFExpRefVar")
+
+
+def _pattern(n_post, n_pre, k, seed):
+    rng = np.random.default_rng(seed)
+    return conn.random_in_degree(n_pre, n_post, rng, rng.integers(0, k + 1, n_post), 0.0)
+
+
+@pytest.mark.parametrize("max_delay", [2, 5])
+@pytest.mark.parametrize("n", [5, 257])
+@pytest.mark.parametrize("extra", [False, True])
+def test_counted_events(gpu, n, max_delay, extra):
+    m, steps = 40, 21
+    rng = np.random.default_rng(n)
+    pats = [_pattern(n, m, 9, 100 * n + k) for k in range(4)]
+    per_syn = rng.integers(1, max_delay + 1, pats[2].nnz)
+    per_syn3 = rng.integers(1, max_delay + 1, pats[3].nnz)
+    w3 = rng.random(pats[3].nnz)
+    ws = [0.1, 0.3, 0.7]
+    net = ah.Network(dt=1.0, seed=1)
+    pre, pop = net.create(m, Every3), net.create(n, LIF)
+    for k, (target, delays) in enumerate((("exc", 0.0), ("exc", 2.0), ("exc", per_syn.astype(float)))):
+        c = pats[k]
+        net.connect(pre, pop, target).from_csr(conn.from_arrays(n, m, c.row_ptr, c.col_idx, None, ws[k]), delays=delays)
+    c = pats[3]
+    net.connect(pre, pop, "inh").from_csr(conn.from_arrays(n, m, c.row_ptr, c.col_idx, w3), delays=per_syn3.astype(float))
+    if extra:   # a fifth one, of weight 0
+        net.connect(pre, pop, "inh").from_csr(conn.from_arrays(n, m, c.row_ptr, c.col_idx, None, 0.0),
+                                              delays=per_syn3.astype(float))
+    mon = net.monitor(pop, ["g_exc", "g_inh"], capacity=steps)
+    net.compile(graph_batch=6)
+    u = (np.arange(m) % 3).astype(np.float64)
+    pre.v = u
+    net.run(steps)
+    exc, inh = mon.get("g_exc"), mon.get("g_inh")
+    fired = []                      # fired[t]: pre spikes of step t
+    for _ in range(steps):
+        u = u + 1.0
+        f = u == 3.0
+        u[f] = 0.0
+        fired.append(f)
+    rows = [np.repeat(np.arange(n), np.diff(p.row_ptr)) for p in pats]
+    delays = [np.ones(pats[0].nnz, int), np.full(pats[1].nnz, 2), per_syn, per_syn3]
+    step = 1.0 - np.exp(-1.0 / 3.0)
+    g, h = np.zeros(n), np.zeros(n)
+    for t in range(steps):
+        for k in range(4):
+            src = t - delays[k]
+            on = np.array([s >= 0 and fired[s][c] for s, c in zip(src, pats[k].col_idx)], dtype=bool)
+            if k == 3:
+                h = h + np.bincount(rows[3][on], weights=w3[on], minlength=n)
+                continue
+            count = np.bincount(rows[k][on], minlength=n)
+            for q in range(count.max(initial=0)):
+                g = np.where(count > q, g + ws[k], g)
+        np.testing.assert_array_equal(exc[t], g)
+        np.testing.assert_allclose(inh[t], h, rtol=0, atol=1e-13)
+        g, h = g + step * -g, h + step * -h

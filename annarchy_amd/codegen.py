@@ -33,6 +33,7 @@ ABI = 13  # AHIP_MODEL_ABI in include/annarchy_hip_model.h
 _PRELUDE = r"""// Generated neuron-model library for the MI355X simulation backend.
 // Model: %(name)s
 #include "rate_rows.hpp"
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 
@@ -1129,38 +1130,60 @@ __global__ void update_global(ahip_syn_args a) {
 %(glob_store)s
 }
 
-// Then one wave per post row: the per-post-neuron equations (evaluated in
-// every lane on the same values, stored by lane 0), then the per-synapse
-// equations, one lane per synapse.
+// Then the rows: the per-post-neuron equations (evaluated in every lane on the
+// same values, stored by lane 0), then the per-synapse equations, one lane per
+// synapse, 4 synapses of a lane at a time: their columns, values and
+// pre-synaptic rates are loaded before the first is computed (one at a time the
+// kernel was two dependent loads per 64 synapses; Oja on 1501 rows of 600, whole
+// step: 20.3 -> 17.0 us).  A row without per-post-neuron equations is shared by up to
+// `chunks` waves when there are few rows.
 template <typename T>
-__global__ __launch_bounds__(256) void update_local(ahip_syn_args a) {
+__global__ __launch_bounds__(256) void update_local(ahip_syn_args a, int32_t chunks) {
     const int lane = threadIdx.x & (ahip::kWave - 1);
-    const int wid = threadIdx.x / ahip::kWave;
+    const int32_t wid = __builtin_amdgcn_readfirstlane((int32_t)blockIdx.x * 4 + (int32_t)(threadIdx.x / ahip::kWave));
     const int64_t t = *a.t_base + a.step;
     if (!update_due(a, t)) return;
     const T dt = (T)(a.dt * (double)(a.update_period > 1 ? a.update_period : 1));
     const int32_t _plasticity = a.plasticity;
-    const int64_t _rs = a.state_stride;
+    const int64_t _rs = %(rs)s;
     T* __restrict__ w = (T*)a.w;
     const int64_t* __restrict__ _pre_last_spike = a.pre_last_spike;
     const int64_t* __restrict__ _post_last_spike = a.post_last_spike;
-    (void)dt; (void)_plasticity; (void)w; (void)_pre_last_spike; (void)_post_last_spike;
+    (void)dt; (void)_plasticity; (void)w; (void)_pre_last_spike; (void)_post_last_spike; (void)_rs;
 %(up_attrs)s
 %(deps)s
 %(preloop)s
-    const int64_t waves = (int64_t)gridDim.x * 4;
-    for (int64_t row = (int64_t)blockIdx.x * 4 + wid; row < a.n_rows; row += waves) {
-        const int32_t post = (int32_t)row;
+    const int32_t* __restrict__ cols = a.col_idx;
+    const ahip::EventWalk W(wid, (int32_t)gridDim.x * 4, chunks);
+    constexpr int kB = 4;
+    for (int32_t row = W.s0, c = W.c0; row < a.n_rows; W.step(row, c)) {
+        const int32_t post = row;
         (void)post;
+%(post_vals)s
 %(sg_load)s
 %(semiglobal_eqs)s
 %(sg_store)s
         const int64_t e = a.row_ptr[row + 1];
-        for (int64_t j = a.row_ptr[row] + lane; j < e; j += ahip::kWave) {
-            const int64_t q = a.fwd2col ? a.fwd2col[j] : j;
-            const int32_t pre = a.col_idx[j];
-            (void)q; (void)pre;
+        for (int64_t j0 = a.row_ptr[row] + (int64_t)c * (kB * ahip::kWave) + lane; j0 < e;
+             j0 += (int64_t)chunks * (kB * ahip::kWave)) {
+            int64_t _q[kB];
+            int32_t _p[kB];
+#pragma unroll
+            for (int u = 0; u < kB; u++) {
+                const int64_t j = j0 + u * ahip::kWave < e ? j0 + u * ahip::kWave : j0;
+                _q[u] = %(state_of)s;
+                _p[u] = cols[j];
+            }
+%(syn_loads)s
+#pragma unroll
+            for (int u = 0; u < kB; u++) {
+                if (j0 + u * ahip::kWave >= e) break;
+                const int64_t q = _q[u];
+                const int32_t pre = _p[u];
+                (void)q; (void)pre;
 %(local_eqs)s
+%(syn_stores)s
+            }
         }
     }
     (void)lane;
@@ -1305,9 +1328,43 @@ def generate_synapse(desc) -> SynapseSource:
     has_rows = bool(sg_eqs.strip() or local_eqs.strip())
     launch_global = ("    hipLaunchKernelGGL(update_global<T>, dim3(1), dim3(64), 0, s, *a);"
                      if has_global else "")
-    launch_local = ("    {\n        int nb = (a->n_rows + 3) / 4;\n        if (nb > 1024) nb = 1024;\n"
-                    "        if (nb > 0) hipLaunchKernelGGL(update_local<T>, dim3(nb), dim3(256), 0, s, *a);\n    }"
+    # waves of a row: its runs of 256 synapses, as long as the rows do not fill
+    # 4096 waves; one where a wave also runs the row's own equations
+    launch_local = ("    {\n" +
+                    ("        const int32_t ch = 1;\n" if sg_eqs.strip() else
+                     "        const int32_t ch = a->n_rows <= 0 ? 1 : std::max(1, std::min((a->post_chunks + 3) / 4,\n"
+                     "                                                                     4096 / a->n_rows));\n") +
+                    "        const int64_t nb = std::min<int64_t>(1024, ((int64_t)a->n_rows * ch + 3) / 4);\n"
+                    "        if (nb > 0) hipLaunchKernelGGL(update_local<T>, dim3(nb), dim3(256), 0, s, *a, ch);\n    }"
                     if has_rows else "")
+    # the per-synapse equations on register copies: w and the attributes they
+    # use, the pre-synaptic values; the post-synaptic ones once per row
+    ref = lambda c, idx: r"(?<![\w.])" + re.escape(c) + r"\[" + re.escape(idx) + r"\]"
+    syn_loads, syn_stores, post_vals = [], [], []
+    for c in ["w"] + ["_s_" + _c_name(n) for n, loc, _ in attrs if loc == "local"]:
+        pat = ref(c, "q*_rs")
+        if not re.search(pat, local_eqs):
+            continue
+        syn_loads.append((f"T {c}__b[kB];", f"{c}__b[u] = {c}[_q[u]*_rs];"))
+        if re.search(pat + r"\s*(?:[-+*/]?=(?!=)|\+\+|--)", local_eqs):
+            syn_stores.append(f"                {c}[q*_rs] = {c}__b[u];")
+        local_eqs = re.sub(pat, c + "__b[u]", local_eqs)
+    for n in desc.pre_deps:
+        pat = ref(f"_dpre_{n}", f"pre*_st_pre_{n}")
+        if not re.search(pat, local_eqs):
+            continue
+        syn_loads.append((f"T _vpre_{n}__b[kB];", f"_vpre_{n}__b[u] = _dpre_{n}[_p[u]*_st_pre_{n}];"))
+        local_eqs = re.sub(pat, f"_vpre_{n}__b[u]", local_eqs)
+    for n in desc.post_deps:
+        pat = ref(f"_dpost_{n}", f"post*_st_post_{n}")
+        if not re.search(pat, local_eqs + sg_eqs):
+            continue
+        post_vals.append(f"        const T _vpost_{n} = _dpost_{n}[post*_st_post_{n}];")
+        local_eqs, sg_eqs = re.sub(pat, f"_vpost_{n}", local_eqs), re.sub(pat, f"_vpost_{n}", sg_eqs)
+    syn_load_code = "\n".join("            " + d for d, _ in syn_loads)
+    if syn_loads:
+        syn_load_code += ("\n#pragma unroll\n            for (int u = 0; u < kB; u++) {\n" +
+                          "\n".join("                " + ld for _, ld in syn_loads) + "\n            }")
     body = _PRELUDE % {"name": desc.name} + "}  // namespace\n" + _SYN_KERNELS % {
         "ev_attrs": "\n".join(ev),
         "up_attrs": "\n".join(up),
@@ -1319,7 +1376,12 @@ def generate_synapse(desc) -> SynapseSource:
         "glob_store": "\n".join(glob_store),
         "global_eqs": _indent(global_eqs, 4),
         "semiglobal_eqs": _indent(sg_eqs, 8),
-        "local_eqs": _indent(local_eqs, 12),
+        "local_eqs": _indent(local_eqs, 16),
+        "rs": "a.state_stride" if desc.spiking else "1",
+        "state_of": "a.fwd2col ? a.fwd2col[j] : j" if desc.spiking else "j",
+        "post_vals": "\n".join(post_vals),
+        "syn_loads": syn_load_code,
+        "syn_stores": "\n".join(syn_stores),
         "pre_body": _indent("\n".join(pre), 12),
         "post_body": _indent("\n".join(post), 12),
         "launch_global": launch_global,

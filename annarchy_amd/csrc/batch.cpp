@@ -227,24 +227,32 @@ int ahip_batch_set_recurrent(ahip_batch* b, const int64_t* row_ptr, const int32_
     if ((rc = balloc(B.chunks, ch.size() * 4, ch.data()))) return rc;
     if ((rc = balloc(B.inst_base, b->offsets.size() * 8, b->offsets.data()))) return rc;
     B.mode = (size_t)max_n * sizeof(float) <= 64 * 1024 ? 1 : 0;
-    // mode 2: chunks of <= 512 rows of one instance, rows sorted by length
-    // (descending, stable) into 64-row slices, width rounded up to 4
+    // mode 2: chunks of <= 512 / G rows of one instance, rows sorted by length
+    // (descending, stable) into slices of 64 / G rows, G lanes per row, width
+    // rounded up to 4 G
     if (max_n < 65535 && (size_t)(max_n + 1) * sizeof(float) <= 64 * 1024) {
+        // lanes per row: enough that the slices occupy 8 waves of every CU, and
+        // at least 4 groups of 4 synapses a lane
+        int32_t G = 1;
+        while (G < 8 && (int64_t)(R / 64) * G < 8 * (int64_t)device_cus() && nnz / std::max(1, R) >= 16 * G) G *= 2;
+        B.sl_lanes = G;
+        const int64_t rows = 512 / G, slice = 64 / G;
         std::vector<int32_t> sch, sch_sl(1, 0), sl_row;
         std::vector<int64_t> sl_off(1, 0);
         std::vector<int32_t> order;
         for (int32_t i = 0; i < B.n_inst; i++) {
-            for (int64_t r0 = b->offsets[i]; r0 < b->offsets[i + 1]; r0 += 512) {
-                const int64_t r1 = std::min<int64_t>(r0 + 512, b->offsets[i + 1]);
+            for (int64_t r0 = b->offsets[i]; r0 < b->offsets[i + 1]; r0 += rows) {
+                const int64_t r1 = std::min<int64_t>(r0 + rows, b->offsets[i + 1]);
                 order.resize(r1 - r0);
                 for (int64_t r = r0; r < r1; r++) order[r - r0] = (int32_t)r;
                 std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t c) {
                     return row_ptr[a + 1] - row_ptr[a] > row_ptr[c + 1] - row_ptr[c];
                 });
-                for (size_t q = 0; q < order.size(); q += 64) {
+                for (size_t q = 0; q < order.size(); q += slice) {
                     const int64_t len0 = row_ptr[order[q] + 1] - row_ptr[order[q]];
-                    for (size_t l = 0; l < 64; l++) sl_row.push_back(q + l < order.size() ? order[q + l] : -1);
-                    sl_off.push_back(sl_off.back() + (len0 + 3) / 4 * 4 * 64);
+                    for (size_t l = 0; l < 64; l++)
+                        sl_row.push_back(l % G == 0 && q + l / G < order.size() ? order[q + l / G] : -1);
+                    sl_off.push_back(sl_off.back() + (len0 + 4 * G - 1) / (4 * G) * 4 * 64);
                 }
                 sch.push_back(i);
                 sch.push_back((int32_t)r0);
@@ -267,7 +275,8 @@ int ahip_batch_set_recurrent(ahip_batch* b, const int64_t* row_ptr, const int32_
                 if (row < 0) continue;
                 const int64_t lo = b->offsets[ii];
                 for (int64_t j = row_ptr[row], k = 0; j < row_ptr[row + 1]; j++, k++) {
-                    const int64_t pos = sl_off[sl] + (k / 4) * 256 + 4 * l + k % 4;
+                    const int64_t e = k / 4;   // l: the row's first lane
+                    const int64_t pos = sl_off[sl] + (e / G) * 256 + 4 * (l + e % G) + k % 4;
                     scol[pos] = (uint16_t)(col[j] - lo);
                     sw[pos] = wf[j];
                 }

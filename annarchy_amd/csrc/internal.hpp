@@ -382,8 +382,10 @@ struct BatchDev {
     int32_t n_chunks = 0, max_n = 0;
     DevBuf chunks;                   // int32 [n_chunks][3] = (instance, first row, end row)
     DevBuf inst_base;                // int64 [n_inst + 1]
-    // mode 2: chunks of <= 512 rows, their 64-row slices and the sliced arrays
+    // mode 2: chunks of <= 512 / sl_lanes rows, their slices of 64 / sl_lanes rows
+    // and the sliced arrays
     int32_t n_schunks = 0;
+    int32_t sl_lanes = 1;            // lanes per row
     int64_t sl_stored = 0;
     DevBuf schunks, schunk_slices;   // int32 [n][3], int32 [n + 1]
     DevBuf sl_off, sl_row;           // int64 [slices + 1], int32 [slices][64] (-1: no row)

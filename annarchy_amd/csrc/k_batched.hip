@@ -252,15 +252,26 @@ __global__ __launch_bounds__(256) void batch_spmv_lds(
     }
 }
 
-// Sliced chunks (mode 2): a chunk holds up to 512 rows of one instance,
-// sorted by length and packed into slices of 64 rows, one lane per row.  Step
+// Sliced chunks (mode 2): a chunk holds up to 512 / G rows of one instance,
+// sorted by length and packed into slices of 64 / G rows, G lanes per row.  Step
 // m of lane l is the 4 synapses at off + 256*m + 4*l: columns as uint16
 // relative to the instance (padding points at the zero slot xs[n]), weights
-// as one 16-byte load.  With U steps in flight and no cross-lane reduction,
-// the lane that owns a row finishes its Kahan sum and applies the update.
+// as one 16-byte load; the groups of 4 of a row go round its lanes.  With U
+// steps in flight the first lane of a row joins the G Kahan sums and applies
+// the update.  G = 1 streams best where the rows fill the chip; a small sweep
+// leaves most of it idle then (24 instances of 500 to 3000 neurons: some 95
+// workgroups, 20 us a step), so its rows are shared (G = 4: some 340, 8.0 us,
+// 4.4 TB/s of algorithmic bytes out of the caches).  NT: streaming loads, for weights that no cache holds from step to
+// step.
 typedef unsigned short v4u16_b __attribute__((ext_vector_type(4)));
 
-template <int U>
+template <bool NT, typename V>
+__device__ inline V ld_stream(const V* p) {
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+
+template <int U, int G, bool NT>
 __global__ __launch_bounds__(512) void batch_sell(
     const int32_t* __restrict__ chunks, const int32_t* __restrict__ chunk_slices,
     const int64_t* __restrict__ inst_base, const int64_t* __restrict__ off, const int32_t* __restrict__ slice_row,
@@ -289,8 +300,8 @@ __global__ __launch_bounds__(512) void batch_sell(
             v4f_b v[U];
 #pragma unroll
             for (int u = 0; u < U; u++) {
-                c[u] = __builtin_nontemporal_load(reinterpret_cast<const v4u16_b*>(cp + (m + u) * 256));
-                v[u] = __builtin_nontemporal_load(reinterpret_cast<const v4f_b*>(wp + (m + u) * 256));
+                c[u] = ld_stream<NT>(reinterpret_cast<const v4u16_b*>(cp + (m + u) * 256));
+                v[u] = ld_stream<NT>(reinterpret_cast<const v4f_b*>(wp + (m + u) * 256));
             }
 #pragma unroll
             for (int u = 0; u < U; u++) {
@@ -301,17 +312,24 @@ __global__ __launch_bounds__(512) void batch_sell(
             }
         }
         for (; m < nsteps; m++) {
-            const v4u16_b c = __builtin_nontemporal_load(reinterpret_cast<const v4u16_b*>(cp + m * 256));
-            const v4f_b v = __builtin_nontemporal_load(reinterpret_cast<const v4f_b*>(wp + m * 256));
+            const v4u16_b c = ld_stream<NT>(reinterpret_cast<const v4u16_b*>(cp + m * 256));
+            const v4f_b v = ld_stream<NT>(reinterpret_cast<const v4f_b*>(wp + m * 256));
             k0.add(v.x * xs[c.x]);
             k1.add(v.y * xs[c.y]);
             k0.add(v.z * xs[c.z]);
             k1.add(v.w * xs[c.w]);
         }
-        k0.add(k1.value());
         const int32_t row = slice_row[(int64_t)sl * kWave + lane];
+        float sum;
+        if constexpr (G == 1) {
+            k0.add(k1.value());
+            sum = k0.value();
+        } else {
+            k0.add(k1.s);
+            k0.c += k1.c;
+            sum = group_sum_kahan<G>(k0.s, k0.c);
+        }
         if (row >= 0) {
-            const float sum = k0.value();
             const int32_t nl = (int32_t)(row - base);
             const float s_in = nl < n_in ? y[(int64_t)inst * ld_y + nl] : 0.0f;
             const float r = xs[nl];
@@ -340,17 +358,23 @@ int batch_launch_input(const BatchDev& B, int32_t step0, int32_t n, hipStream_t 
     return (int)hipGetLastError();
 }
 
-constexpr int kGemmGM = 2, kGemmGN = 4;
-
-int batch_launch_gemm(const BatchDev& B, int32_t n, hipStream_t s) {
-    if (n < 1 || n > B.cap_steps) return (int)hipErrorInvalidValue;
-    const int32_t c_tiles = n * B.n_tiles;
-    const int64_t waves = (int64_t)((c_tiles + kGemmGM - 1) / kGemmGM) * ((B.m_tiles + kGemmGN - 1) / kGemmGN);
-    const int64_t nb = (waves + 3) / 4;
-    hipLaunchKernelGGL((batch_gemm<kGemmGM, kGemmGN>), dim3(nb), dim3(256), 0, s, c_tiles, B.m_tiles, B.k_steps,
+template <int GM, int GN>
+static int launch_gemm(const BatchDev& B, int32_t c_tiles, hipStream_t s) {
+    const int64_t waves = (int64_t)((c_tiles + GM - 1) / GM) * ((B.m_tiles + GN - 1) / GN);
+    hipLaunchKernelGGL((batch_gemm<GM, GN>), dim3((waves + 3) / 4), dim3(256), 0, s, c_tiles, B.m_tiles, B.k_steps,
                        B.x_hi.as<v8bf>(), B.x_lo.as<v8bf>(), B.w_hi.as<v8bf>(), B.w_lo.as<v8bf>(),
                        B.y.as<float>(), B.m_tiles * 32);
     return (int)hipGetLastError();
+}
+
+// 2 x 4 tiles a wave reuse the operands best (295 TFLOP/s of useful work at 400 x
+// 63 tiles); with too few of them to give every SIMD a wave (4 a CU), one tile a
+// wave: 50 x 32 tiles of depth 63, 200 waves 66 us a launch, 1600 waves 35.
+int batch_launch_gemm(const BatchDev& B, int32_t n, hipStream_t s) {
+    if (n < 1 || n > B.cap_steps) return (int)hipErrorInvalidValue;
+    const int32_t c_tiles = n * B.n_tiles;
+    if ((int64_t)c_tiles * B.m_tiles >= (int64_t)8 * 4 * device_cus()) return launch_gemm<2, 4>(B, c_tiles, s);
+    return launch_gemm<1, 1>(B, c_tiles, s);
 }
 
 int batch_launch_spmv(const BatchDev& B, int32_t parity, int32_t j, hipStream_t s) {
@@ -364,11 +388,30 @@ int batch_launch_spmv(const BatchDev& B, int32_t parity, int32_t j, hipStream_t 
     float* rout = B.r[parity ^ 1].as<float>();
     if (B.mode == 2) {
         const size_t lds = (size_t)(B.max_n + 1) * sizeof(float);
-        hipLaunchKernelGGL(batch_sell<2>, dim3(B.n_schunks), dim3(512), lds, s, B.schunks.as<int32_t>(),
-                           B.schunk_slices.as<int32_t>(), B.inst_base.as<int64_t>(), B.sl_off.as<int64_t>(),
-                           B.sl_row.as<int32_t>(), B.sl_col.as<uint16_t>(), B.sl_w.as<float>(), B.gain.as<float>(),
-                           yj, ld_y, B.n_in, rin, rout, B.sum_exc.as<float>(), (float)B.dt,
-                           (float)B.tau);
+        // 6 bytes per stored synapse: what the caches (256 MB) can hold between
+        // steps is loaded as data to keep
+        const bool nt = B.sl_stored * 6 > (int64_t)128 << 20;
+#define AHIP_SELL_CASE(G, NT)                                                                                     \
+    case 2 * G + NT:                                                                                              \
+        hipLaunchKernelGGL((batch_sell<2, G, NT>), dim3(B.n_schunks), dim3(512), lds, s, B.schunks.as<int32_t>(), \
+                           B.schunk_slices.as<int32_t>(), B.inst_base.as<int64_t>(), B.sl_off.as<int64_t>(),      \
+                           B.sl_row.as<int32_t>(), B.sl_col.as<uint16_t>(), B.sl_w.as<float>(),                   \
+                           B.gain.as<float>(), yj, ld_y, B.n_in, rin, rout, B.sum_exc.as<float>(), (float)B.dt,   \
+                           (float)B.tau);                                                                         \
+        break;
+        switch (2 * B.sl_lanes + (nt ? 1 : 0)) {
+            AHIP_SELL_CASE(1, false)
+            AHIP_SELL_CASE(1, true)
+            AHIP_SELL_CASE(2, false)
+            AHIP_SELL_CASE(2, true)
+            AHIP_SELL_CASE(4, false)
+            AHIP_SELL_CASE(4, true)
+            AHIP_SELL_CASE(8, false)
+            AHIP_SELL_CASE(8, true)
+            default:
+                return (int)hipErrorInvalidValue;
+        }
+#undef AHIP_SELL_CASE
         return (int)hipGetLastError();
     }
     if (B.mode == 1) {

@@ -28,7 +28,7 @@ import re
 
 from .equations import DISTRIBUTIONS, NeuronDescription, analyse_neuron, equation_code
 
-ABI = 13  # AHIP_MODEL_ABI in include/annarchy_hip_model.h
+ABI = 14  # AHIP_MODEL_ABI in include/annarchy_hip_model.h
 
 _PRELUDE = r"""// Generated neuron-model library for the MI355X simulation backend.
 // Model: %(name)s
@@ -131,6 +131,7 @@ int launch_f32(const ahip_pop_args* a, void* s) { return launch<float>(a, s); }
 
 %(persist_fn)s
 %(fused_fn)s
+%(ahead_fn)s
 
 const char* const kSlotNames[] = {%(slot_names)s};
 const int32_t kSlotLocal[] = {%(slot_local)s};
@@ -142,7 +143,7 @@ const double kRandArgs[] = {%(rand_args)s};
 const ahip_model_desc kDesc = {
     %(abi)d, "%(name)s", %(spiking)d, %(n_slots)d, kSlotNames, kSlotLocal, kSlotInit, kSlotKind,
     %(n_rand)d, kRandDist, kRandArgs, %(has_refractory)d, %(has_global)d,
-    launch_f64, launch_f32, %(preloop_ptr)s, "%(hash)s", %(persist_ptrs)s, %(fused_ptrs)s};
+    launch_f64, launch_f32, %(preloop_ptr)s, "%(hash)s", %(persist_ptrs)s, %(fused_ptrs)s, %(ahead_ptrs)s};
 
 }  // namespace
 
@@ -483,6 +484,55 @@ int persist_f32(const ahip_pop_args* a, const ahip_persist_args* pa, size_t lds,
     return persist<float>(a, pa, lds, s);
 }
 const int32_t kPersistSlotsHost[] = {%(pslot_list)s};
+"""
+
+
+# Several steps of an input population in one launch (annarchy_hip_model.h).  A
+# launch of a step's graph costs 1.1 us beside the kernel's own chain, and the
+# update of a Poisson or a sine population of a few thousand neurons is little
+# else.  Their steps do not depend on one another, so they run side by side,
+# AHIP_AHEAD of them, blockIdx.y the step (us per step, a launch a step / 16 at
+# a time: sine rates into two delayed projections of 5001 neurons 16.7 / 14.4;
+# 2000 Poisson inputs into 20003 COBA neurons 14.6 / 12.7, 8000 into 80000
+# 17.1 / 15.1).
+_AHEAD_KERNEL = r"""
+template <typename T>
+__global__ __launch_bounds__(AHIP_UPDATE_BLOCK) void ahead_update(ahip_pop_args a) {
+    const int32_t i = blockIdx.x * AHIP_UPDATE_BLOCK + threadIdx.x;
+    const int32_t _at = (int32_t)blockIdx.y;
+    const bool _last = blockIdx.y + 1 == gridDim.y;
+    const int64_t t = ahip::sim_time(a) + _at;
+    const T dt = (T)a.dt;
+    (void)t; (void)dt; (void)_last;
+%(global_loads)s
+%(div_consts)s
+%(local_ptrs)s
+    const bool _act = i < a.size;
+%(regs)s
+    bool _spike = false;
+    if (_act) {
+%(local_rand)s
+%(local_eqs)s
+%(gather)s
+        if (_last) {
+%(stores)s
+        }
+%(push)s
+%(rec_after)s
+    }
+    (void)_spike;
+%(publish)s
+}
+
+template <typename T>
+int ahead(const ahip_pop_args* a, int32_t steps, void* stream) {
+    const int nb = (a->size + AHIP_UPDATE_BLOCK - 1) / AHIP_UPDATE_BLOCK;
+    if (nb <= 0 || steps < 1 || steps > AHIP_AHEAD) return (int)hipErrorInvalidValue;
+    hipLaunchKernelGGL(ahead_update<T>, dim3(nb, steps), dim3(AHIP_UPDATE_BLOCK), 0, (hipStream_t)stream, *a);
+    return (int)hipGetLastError();
+}
+int ahead_f64(const ahip_pop_args* a, int32_t steps, void* s) { return ahead<double>(a, steps, s); }
+int ahead_f32(const ahip_pop_args* a, int32_t steps, void* s) { return ahead<float>(a, steps, s); }
 """
 
 
@@ -856,6 +906,7 @@ def generate(desc: NeuronDescription, stop_condition: str | None = None) -> Mode
     for key in lparts:
         lparts[key] = lparts[key].replace("a.refractory_remaining[i]", "refrac_rem[i]")
     ljoined = "\n".join(lparts.values())
+    aparts = dict(lparts)   # of the launch of several steps
     lref = lambda c: r"(?<![\w.])" + re.escape(c) + r"\[i\]"
     lwrites = lambda c: re.search(lref(c) + r"\s*(?:[-+*/]?=(?!=)|\+\+|--)", ljoined) is not None
     # read: any reference other than the target of a plain assignment
@@ -918,8 +969,8 @@ def generate(desc: NeuronDescription, stop_condition: str | None = None) -> Mode
         reg_out.append(f"        ahip::push_rate<T>(a, t, i, {r_now});")
 
     # value monitors: the value in its register, where it has one
-    def record_code(before: int) -> str:
-        cases = "".join(f" case {slot_of[n]}: _v = {_u(n)}__r; break;" for n in local_names if lreads(_u(n)))
+    def record_code(before: int, in_reg=lreads) -> str:
+        cases = "".join(f" case {slot_of[n]}: _v = {_u(n)}__r; break;" for n in local_names if in_reg(_u(n)))
         return (f"        for (int _k = 0; _k < a.n_rec; _k++) {{\n"
                 f"            if (a.rec_before[_k] != {before}) continue;\n"
                 f"            T _v;\n"
@@ -948,6 +999,49 @@ def generate(desc: NeuronDescription, stop_condition: str | None = None) -> Mode
             "launch_global": launch_global,
         }
         fused_ptrs = "fused_f64, fused_f32"
+
+    # steps that do not depend on one another: every local value the statements
+    # write is assigned, unconditionally and from nothing older, before they read it
+    def used(c: str) -> bool:
+        return lreads(c) or lwrites(c)
+
+    def assigned_first(c: str) -> bool:
+        if not lwrites(c):
+            return True
+        m = re.search(lref(c), ljoined)
+        before, after = re.sub(r"//[^\n]*", "", ljoined[:m.start()]), ljoined[m.end():]
+        return (before.count("{") == before.count("}")
+                and before.rstrip()[-1:] in ("", ";", "}")   # a statement of its own
+                and re.match(r"\s*=(?!=)", after) is not None
+                and re.search(lref(c), after[:after.find(";")]) is None)
+
+    ahead_fn, ahead_ptrs = "", "nullptr, nullptr"
+    if (not has_global and not has_ref and not sums and (desc.spiking or ring_r) and
+            "a.last_spike" not in local_eqs and all(assigned_first(_u(n)) for n in local_names)):
+        regs, stores = [], []
+        for n in local_names:
+            c = _u(n)
+            if not used(c):
+                continue
+            # (a value assigned first needs no load, a parameter does)
+            regs.append(f"    T {c}__r = T(0);" if lwrites(c) else f"    T {c}__r = _act ? {c}[i] : T(0);")
+            if lwrites(c):
+                stores.append(f"            {c}[i] = {c}__r;")
+            for key in aparts:
+                aparts[key] = re.sub(lref(c), c + "__r", aparts[key])
+        ahead_fn = _AHEAD_KERNEL % {
+            "global_loads": global_loads, "div_consts": div_consts, "local_ptrs": local_ptrs,
+            "regs": "\n".join(regs),
+            "local_rand": _indent(aparts["local_rand"], 8),
+            "local_eqs": _indent(aparts["local_eqs"], 8),
+            "gather": _indent("\n".join(ln for ln in aparts["gather"].split("\n") if "a.last_spike" not in ln), 8),
+            "stores": "\n".join(stores),
+            "push": (f"        ahip::push_rate<T>(a, t, i, {_u('r')}" +
+                     ("__r);" if used(_u("r")) else "[i]);")) if ring_r else "",
+            "rec_after": _indent(record_code(0, used), 0),
+            "publish": "    ahip::publish_spikes(a, _spike, _at);" if desc.spiking else "",
+        }
+        ahead_ptrs = "ahead_f64, ahead_f32"
 
     body = _PRELUDE % {"name": desc.name}
     if has_global:
@@ -993,6 +1087,8 @@ def generate(desc: NeuronDescription, stop_condition: str | None = None) -> Mode
         "persist_ptrs": persist_ptrs,
         "fused_fn": fused_fn,
         "fused_ptrs": fused_ptrs,
+        "ahead_fn": ahead_fn,
+        "ahead_ptrs": ahead_ptrs,
         "hash": "%(hash)s",
     }
     cond, _ = parse_stop_condition(stop_condition)

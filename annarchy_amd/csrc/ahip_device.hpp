@@ -269,14 +269,16 @@ __device__ inline T random_value(const ahip_pop_args& a, int32_t i, int32_t k, i
 
 // Spike flags of one update block: wave ballot -> one 64-bit word per wave,
 // and the number of spikes of the block (256 threads = 4 waves).
-__device__ inline void publish_spikes(const ahip_pop_args& a, bool spk) {
+// `at`: the step of a launch of several (its words and counts follow those of the
+// steps before).
+__device__ inline void publish_spikes(const ahip_pop_args& a, bool spk, int32_t at = 0) {
     __shared__ int32_t wave_cnt[AHIP_UPDATE_BLOCK / kWave];
     const int lane = threadIdx.x & (kWave - 1);
     const int wid = threadIdx.x / kWave;
     uint64_t m = __ballot(spk);
     const int64_t word = (int64_t)blockIdx.x * (AHIP_UPDATE_BLOCK / kWave) + wid;
     if (lane == 0) {
-        if (word * kWave < a.size) a.spike_mask[word] = m;
+        if (word * kWave < a.size) a.spike_mask[(int64_t)at * ((a.size + kWave - 1) / kWave) + word] = m;
         wave_cnt[wid] = __popcll(m);
     }
     __syncthreads();
@@ -284,7 +286,7 @@ __device__ inline void publish_spikes(const ahip_pop_args& a, bool spk) {
         int32_t s = 0;
 #pragma unroll
         for (int w = 0; w < AHIP_UPDATE_BLOCK / kWave; w++) s += wave_cnt[w];
-        a.block_counts[blockIdx.x] = s;
+        a.block_counts[(int64_t)at * gridDim.x + blockIdx.x] = s;
     }
 }
 

@@ -67,10 +67,16 @@ struct Pop {
     // depth x size int32 with counts int32[depth]
     int32_t depth = 1;
     DevBuf hist, hist_count;
-    // rate-coded: r at the end of the last two steps (slot t & 1), kept by the
-    // population's update while a fused update reads it; and the population's
-    // own fused update (psp of every projection into it, then the statements)
+    // rate-coded: r at the end of the last steps (rbuf_depth slots: 2, of an
+    // ahead population 2 AHIP_AHEAD), kept by the population's update while a
+    // fused update reads it; and the population's own fused update (psp of every
+    // projection into it, then the statements)
     DevBuf rbuf;
+    int32_t rbuf_depth = 2;
+    // an input population whose steps run AHIP_AHEAD at a time in a batch, and the
+    // slice of its mask and counts this step's compaction reads (-1: of one step)
+    bool ahead = false;
+    int32_t ahead_at = -1;
     bool fused = false;
     ahip_fuse_args fuse;
     // mean firing rate over fr_window steps (0: off): a fr_window-bit history

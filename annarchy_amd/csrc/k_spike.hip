@@ -47,6 +47,7 @@ struct CompactArgs {
     const int32_t* bcnt;
     int32_t* spiked;
     int32_t* count;
+    int64_t* last_spike;          // NULL: written by the update
     SpikeRec rec;
 };
 
@@ -74,9 +75,10 @@ __device__ inline void compact_chunk(const CompactArgs& c, int32_t b, const int6
     int32_t part = 0;
     for (int32_t k = threadIdx.x; k < ub0; k += kCompactThreads) part += c.bcnt[k];
     int64_t slot = -1, f = 0;
+    const int64_t t = *t_base + step;
     if (rec.counts) {
         const int64_t fill0 = rec.fill[0], fill1 = rec.fill[1];
-        slot = record_row(*rec.state, *t_base + step);
+        slot = record_row(*rec.state, t);
         if (slot >= 0) f = (slot & 1) ? fill1 : fill0;
     }
     part = group_sum<kWave>(part);
@@ -105,6 +107,7 @@ __device__ inline void compact_chunk(const CompactArgs& c, int32_t b, const int6
                                            (uint32_t)(word[k] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)word[k], 0u));
             const int32_t i = n0 + k * kWave + lane;
             c.spiked[pos] = i;
+            if (c.last_spike) c.last_spike[i] = t;
             if (slot >= 0 && f + pos < rec.idx_capacity) rec.idx[f + pos] = i;
         }
         pos0 += (int32_t)__popcll(word[k]);
@@ -448,6 +451,11 @@ int launch_compact(const ahip_net* net, const std::vector<int32_t>& pops, const 
             c.nb = (p.size + kCompactChunk - 1) / kCompactChunk;
             c.mask = p.spike_mask.as<uint64_t>();
             c.bcnt = p.block_counts.as<int32_t>();
+            if (p.ahead_at >= 0) {
+                c.mask += (int64_t)p.ahead_at * p.nwords();
+                c.bcnt += (int64_t)p.ahead_at * p.nblocks();
+                c.last_spike = p.last_spike.as<int64_t>();
+            }
             c.spiked = p.spiked.as<int32_t>();
             c.count = p.spike_count.as<int32_t>();
             if (m) {

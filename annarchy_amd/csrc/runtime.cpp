@@ -144,6 +144,18 @@ static int regrow_ring(DevBuf& buf, size_t slot_bytes, int32_t d_old, int32_t d_
     return 0;
 }
 
+// Populations whose statements allow several steps in one launch
+// (ahip_ahead_fn) and that no projection reaches.  Up to 2^18 neurons: a step
+// that fills the chip by itself gains nothing, and the rings grow by
+// AHIP_AHEAD slots (2 MB each there in FP64).
+constexpr int32_t kAheadMaxSize = 1 << 18;
+static bool may_run_ahead(const ahip_net* net, const Pop& p) {
+    if (!(net->precision == AHIP_F64 ? p.model->ahead_f64 : p.model->ahead_f32) || p.size > kAheadMaxSize) return false;
+    for (auto& q : net->projs)
+        if (q->post == p.id) return false;
+    return true;
+}
+
 // Delay queues: the depth of a population's queue is the largest delay that
 // reads it (rate-coded: every delayed projection; spiking: the uniform
 // delays, per-synapse delays keep their own event ring), and it never
@@ -163,7 +175,10 @@ int ensure_delay_buffers(ahip_net* net) {
         Pop& p = *pp;
         // one slot more for rates: a fused update may push step t's value
         // while another workgroup of its launch reads step t - max_delay's
-        const int32_t want = need[p.id] > 1 && !p.model->spiking ? need[p.id] + 1 : need[p.id];
+        // (AHIP_AHEAD slots more where the population's updates may run that
+        // many steps ahead of the readers)
+        const int32_t want = need[p.id] > 1 && !p.model->spiking
+                                 ? need[p.id] + (may_run_ahead(net, p) ? AHIP_AHEAD : 1) : need[p.id];
         const int32_t D = std::max(want, p.depth);
         if (D == p.depth && (D == 1 || p.hist.p)) continue;
         HIPCHK(hipStreamSynchronize(net->stream));
@@ -776,8 +791,7 @@ static bool fuse_desc(ahip_net* net, const Proj& p, int32_t sum, ahip_fuse_proj&
         d.delay = p.delay_per_syn ? 0 : p.delay_uniform;
         d.delays = p.delay_per_syn ? p.delay_dev.as<int16_t>() : nullptr;
     } else {
-        d.x = pre.rbuf.p;   // set by plan_fused once the buffer exists
-        d.depth = 2;
+        // (x and depth are set by plan_fused once the buffer exists)
         d.delay = 1;
     }
     return true;
@@ -790,6 +804,36 @@ static bool fuse_desc(ahip_net* net, const Proj& p, int32_t sum, ahip_fuse_proj&
 // 40000 x 1500); staged or dense rows gain or are equal as far as measured
 // (45.7 / 81.6 at 12000 x 2000, dense 89.3 / 90.2 at 8000 x 8000).
 constexpr int64_t kFuseMaxGathered = 1 << 24, kFuseMaxStaged = 1 << 27;
+
+// The input populations that run ahead: nothing inside a batch may read their
+// values other than through the rings and spike lists, which hold every step's
+// (plastic projections that read pre.<name>, monitors with a kernel of their own
+// and the firing-rate window do), and rates only fused updates, which read rings.
+static int assign_ahead(ahip_net* net) {
+    for (auto& pp : net->pops) {
+        Pop& p = *pp;
+        bool ok = p.active && p.n_deliver == 0 && p.fr_window == 0 && may_run_ahead(net, p);
+        int32_t oldest = 1;
+        for (auto& qq : net->projs) {
+            const Proj& q = *qq;
+            if (q.pre != p.id) continue;
+            if (q.syn ? !p.model->spiking || !q.dep_pre.empty() : !p.model->spiking && !net->pops[q.post]->fused) ok = false;
+            oldest = std::max(oldest, q.max_delay);
+        }
+        if (!p.model->spiking && p.depth > 1 && p.depth < oldest + AHIP_AHEAD) ok = false;
+        for (auto& mp : net->mons)
+            if (mp->pop == p.id && !mp->paused && !mp->spikes && (!mp->in_update || (mp->after_psp && p.model->spiking))) ok = false;
+        if (ok != p.ahead) drop_graph(net);
+        p.ahead = ok;
+        if (ok && p.model->spiking && p.spike_mask.bytes < (size_t)AHIP_AHEAD * p.nwords() * sizeof(uint64_t)) {
+            HIPCHK(hipStreamSynchronize(net->stream));
+            int rc = dev_alloc(p.spike_mask, (size_t)AHIP_AHEAD * p.nwords() * sizeof(uint64_t));
+            if (!rc) rc = dev_alloc(p.block_counts, (size_t)AHIP_AHEAD * p.nblocks() * sizeof(int32_t));
+            if (rc) return rc;
+        }
+    }
+    return 0;
+}
 
 // Which populations run psp and update in one launch: an active rate-coded
 // population whose every incoming projection is rate-coded with a row layout
@@ -883,6 +927,8 @@ static int plan_fused(ahip_net* net) {
         F.stage = stage ? 1 : 0;
         p.fused = true;
     }
+    int rc_a = assign_ahead(net);
+    if (rc_a) return rc_a;
     // the pre-synaptic rates of undelayed projections: the last two steps'
     std::vector<char> need(net->pops.size(), 0);
     for (auto& pp : net->pops)
@@ -891,10 +937,13 @@ static int plan_fused(ahip_net* net) {
                 if (qq->post == pp->id && !qq->delay_per_syn && qq->delay_uniform < 2) need[qq->pre] = 1;
     for (auto& pp : net->pops) {
         Pop& p = *pp;
-        if (need[p.id] && !p.rbuf.p) {
+        const int32_t depth = p.ahead ? 2 * AHIP_AHEAD : 2;
+        if (need[p.id] && (!p.rbuf.p || p.rbuf_depth != depth)) {
             drop_graph(net);
-            int rc = dev_alloc(p.rbuf, 2 * (size_t)p.size * net->elem());
+            HIPCHK(hipStreamSynchronize(net->stream));
+            int rc = dev_alloc(p.rbuf, depth * (size_t)p.size * net->elem());
             if (rc) return rc;
+            p.rbuf_depth = depth;
             net->rbuf_stale = true;
         } else if (!need[p.id] && p.rbuf.p) {
             drop_graph(net);
@@ -909,7 +958,10 @@ static int plan_fused(ahip_net* net) {
         for (auto& qq : net->projs)
             if (qq->post == p.id && transmits(net, *qq) && qq->nnz != 0) {
                 ahip_fuse_proj& d = p.fuse.p[n++];
-                if (!qq->delay_per_syn && qq->delay_uniform < 2) d.x = net->pops[qq->pre]->rbuf.p;
+                if (!qq->delay_per_syn && qq->delay_uniform < 2) {
+                    d.x = net->pops[qq->pre]->rbuf.p;
+                    d.depth = net->pops[qq->pre]->rbuf_depth;
+                }
             }
     }
     return 0;
@@ -923,7 +975,7 @@ static int refresh_rates(ahip_net* net) {
         Pop& p = *pp;
         if (!p.rbuf.p) continue;
         // the slot of the last step, t - 1
-        LCHK(launch_push_values(net, p.slots[p.slot_index("r")].p, p.rbuf.p, p.size, 2, -1, net->stream));
+        LCHK(launch_push_values(net, p.slots[p.slot_index("r")].p, p.rbuf.p, p.size, p.rbuf_depth, -1, net->stream));
     }
     net->rbuf_stale = false;
     return 0;
@@ -1021,7 +1073,7 @@ ahip_pop_args make_args(ahip_net* net, Pop& p, int32_t step) {
     }
     if (p.rbuf.p) {
         a.push_buf[1] = p.rbuf.p;
-        a.push_depth[1] = 2;
+        a.push_depth[1] = p.rbuf_depth;
     }
     // the projections without a delay per synapse first, as their scatter was
     for (int pass = 0; pass < 2; pass++)
@@ -1050,8 +1102,8 @@ ahip_pop_args make_args(ahip_net* net, Pop& p, int32_t step) {
 }
 
 
-// Enqueue one simulation step (index `step` inside the current batch).
-int enqueue_step(ahip_net* net, int32_t step, const std::vector<int32_t>& zero_before) {
+// Enqueue one simulation step (index `step` inside the current batch of `nsteps`).
+int enqueue_step(ahip_net* net, int32_t step, int32_t nsteps, const std::vector<int32_t>& zero_before) {
     hipStream_t s = net->stream;
     const size_t es = net->elem();
     // 1. compute_psp: the spiking projections in fused scatter groups, then
@@ -1130,6 +1182,16 @@ int enqueue_step(ahip_net* net, int32_t step, const std::vector<int32_t>& zero_b
             continue;
         }
         ahip_pop_args a = make_args(net, p, step);
+        p.ahead_at = -1;
+        if (p.ahead && nsteps > 1 && net->probe_kind < 0) {
+            if (step % AHIP_AHEAD == 0) {
+                const ahip_ahead_fn fn = net->precision == AHIP_F64 ? p.model->ahead_f64 : p.model->ahead_f32;
+                LCHK(fn(&a, std::min<int32_t>(AHIP_AHEAD, nsteps - step), (void*)s));
+            }
+            p.ahead_at = step % AHIP_AHEAD;
+            if (p.model->spiking) compact.push_back(p.id);
+            continue;
+        }
         ahip_launch_fn fn = net->precision == AHIP_F64 ? p.model->launch_f64 : p.model->launch_f32;
         const bool probe_u = net->probe_kind == AHIP_PROBE_UPDATE && net->probe_proj == p.id;
         if (probe_u) HIPCHK(hipEventRecord(net->probe_ev[0], s));
@@ -1291,7 +1353,7 @@ int enqueue_batch(ahip_net* net, int32_t nsteps, const std::vector<int32_t>& zb)
         return 0;
     }
     for (int32_t j = 0; j < nsteps; j++) {
-        int rc = enqueue_step(net, j, zb);
+        int rc = enqueue_step(net, j, nsteps, zb);
         if (rc) return rc;
     }
     LCHK(launch_advance_time(net->t_dev.as<int64_t>(), nsteps, net->stream));
@@ -1835,7 +1897,7 @@ int ahip_pop_size_in_bytes(ahip_net* net, int32_t pop, int64_t* bytes) {
     for (const DevBuf& d : p->slots) b += d.bytes;
     for (const DevBuf* d : std::initializer_list<const DevBuf*>{&p->refractory, &p->refractory_remaining, &p->last_spike, &p->spike_mask,
                             &p->block_counts, &p->spiked, &p->spike_count, &p->hist, &p->hist_count,
-                            &p->ring_tmp, &p->fr_bits, &p->fr_count})
+                            &p->ring_tmp, &p->fr_bits, &p->fr_count, &p->rbuf})
         b += d->bytes;
     for (const DevBuf& d : p->rand_inject) b += d.bytes;
     *bytes = (int64_t)b;

@@ -22,7 +22,7 @@
 extern "C" {
 #endif
 
-#define AHIP_MODEL_ABI 13
+#define AHIP_MODEL_ABI 14
 #define AHIP_MAX_SLOTS 48
 #define AHIP_MAX_RAND 8
 #define AHIP_UPDATE_BLOCK 256 /* threads per block of every update kernel */
@@ -118,6 +118,18 @@ typedef struct ahip_pop_args {
 } ahip_pop_args;
 
 typedef int (*ahip_launch_fn)(const ahip_pop_args* args, void* stream);
+
+/* ---- several steps of an input population in one launch --------------------
+ * A population that no projection reaches and whose values are functions of the
+ * step alone (draws, constants, the clock; no value of the step before) does not
+ * have to wait for the network: one launch computes `steps` steps from the
+ * args' step on, a workgroup per 256 neurons and step.  Rates go to the rings
+ * (push_buf), recorded values to their rows, spikes to the mask and the counts of
+ * each step (ceil(size / 64) words and ceil(size / 256) counts a step), the
+ * population's values are those of the last step.  last_spike is left to the
+ * compaction of each step. */
+#define AHIP_AHEAD 16      /* steps of a launch at most */
+typedef int (*ahip_ahead_fn)(const ahip_pop_args* args, int32_t steps, void* stream);
 
 /* ---- psp and update of a rate-coded population in one launch --------------
  * The rows (post neurons) of every projection into the population are summed
@@ -236,6 +248,8 @@ typedef struct ahip_model_desc {
     const int32_t* persist_slots;       /* those the statements touch and the conductances */
     ahip_fused_fn fused_f64;            /* NULL for spiking models and models without a psp sum */
     ahip_fused_fn fused_f32;
+    ahip_ahead_fn ahead_f64;            /* NULL: the statements read a value of the step before */
+    ahip_ahead_fn ahead_f32;
 } ahip_model_desc;
 
 /* Every model library exports this symbol. */

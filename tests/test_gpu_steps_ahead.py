@@ -1,0 +1,104 @@
+"""Input populations whose steps run several at a time.
+
+Inside a batch the updates of a population that nothing reaches and that keeps no
+state run up to 16 steps per launch; a run of one step uses the ordinary update.
+Both have to give the same values, spikes and records, whatever the lengths (20:
+launches of 16 and 4; 9: one, launched step by step the first time and captured
+from the second on; 33: a batch, then 13).
+
+Which statements qualify is decided by the generator: a value read before the
+step assigns it keeps its population out.
+"""
+
+import numpy as np
+import pytest
+
+import annarchy_amd as ah
+from annarchy_amd import codegen
+from annarchy_amd import connectivity as conn
+
+SinRate = ah.Neuron(parameters="phase = 0.0", equations="r = 0.5 + 0.5*sin(0.1*t + phase)", name="SinRate")
+SumRate = ah.Neuron(equations="r = sum(exc)", name="SumRate")
+PoissonPre = ah.Neuron(parameters="rates = 40.0", equations="p = Uniform(0.0, 1.0) * 1000.0 / dt",
+                       spike="p < rates", name="PoissonPre")
+Every5 = ah.Neuron(equations="v = v + 1.0\nmp = t\nq = g_exc", spike="v == 5.0", reset="v = 0.0", name="Every5")
+
+RUNS = (20, 9, 9, 33, 1, 40, 33)
+
+
+@pytest.mark.parametrize("equations, yes", [
+    ("r = 0.5 + 0.5*sin(0.1*t)", True),
+    ("a = Uniform(0.0, 1.0)\nr = 2.0 * a", True),
+    ("r = 2.0 * a\na = Uniform(0.0, 1.0)", False),       # reads last step's a
+    ("r += 0.1", False),
+    ("tau*dr/dt + r = 1.0", False),
+    ("r = if t > 5: 1.0 else: r", False),
+    ("r = if t > 5: 1.0 else: 0.5", True),
+    ("r = sum(exc)", False),                             # a psp target
+])
+def test_which_statements_run_ahead(equations, yes):
+    src = codegen.generate_from_text("M", "tau = 10.0", equations, None, None, None).source
+    assert ("void ahead_update" in src) == yes
+
+
+def _rate(pre_size, post_size, precision):
+    rng = np.random.default_rng(pre_size)
+    k = min(3, pre_size)
+    net = ah.Network(dt=1.0, seed=3, precision=precision)
+    inp, pop = net.create(pre_size, SinRate), net.create(post_size, SumRate)
+    for delays in (None, 4.0, rng.integers(1, 6, post_size * k).astype(float)):
+        col = np.concatenate([np.sort(rng.choice(pre_size, k, replace=False)) for _ in range(post_size)])
+        csr = conn.from_arrays(post_size, pre_size, np.arange(post_size + 1) * k, col, rng.normal(size=post_size * k))
+        net.connect(inp, pop, "exc").from_csr(csr, storage_format="csr", **({} if delays is None else {"delays": delays}))
+    mons = [net.monitor(pop, ["r"], capacity=64), net.monitor(inp, ["r", "phase"], capacity=64)]
+    net.compile(graph_batch=20)
+    inp.phase = np.linspace(0.0, 2.0, pre_size)
+    return net, inp, pop, mons
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pre_size, post_size", [(1, 3), (64, 5), (257, 300)])
+@pytest.mark.parametrize("precision", ["double", "float"])
+def test_rates_ahead_are_the_steps(gpu, pre_size, post_size, precision):
+    many, one = _rate(pre_size, post_size, precision), _rate(pre_size, post_size, precision)
+    for steps in RUNS:
+        many[0].run(steps)
+        for _ in range(steps):
+            one[0].run(1)
+        for a, b in zip(many[3], one[3]):
+            np.testing.assert_array_equal(a.get("r"), b.get("r"))
+        np.testing.assert_array_equal(many[1].r, one[1].r)
+    np.testing.assert_array_equal(many[2].r, one[2].r)
+
+
+def _spiking(n, uniform_delay):
+    net = ah.Network(dt=1.0, seed=5)
+    inp, pop = net.create(n, PoissonPre), net.create(300, Every5)
+    proj = net.connect(inp, pop, "exc")
+    rng = np.random.default_rng(n)
+    k = min(4, n)
+    col = np.concatenate([np.sort(rng.choice(n, k, replace=False)) for _ in range(300)])
+    csr = conn.from_arrays(300, n, np.arange(301) * k, col, np.full(300 * k, 0.5))
+    proj.from_csr(csr, **({"delays": uniform_delay} if uniform_delay else {}))
+    mons = [net.monitor(inp, ["spike", "p"], capacity=64), net.monitor(pop, ["q"], capacity=64),
+            net.monitor(inp, ["spike"], capacity=64)]
+    net.compile(graph_batch=20)
+    inp.rates = np.linspace(50.0, 400.0, n)
+    return net, inp, mons
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 64, 257, 4100])
+@pytest.mark.parametrize("uniform_delay", [0.0, 3.0])
+def test_spikes_ahead_are_the_steps(gpu, n, uniform_delay):
+    many, one = _spiking(n, uniform_delay), _spiking(n, uniform_delay)
+    for steps in RUNS:
+        many[0].run(steps)
+        for _ in range(steps):
+            one[0].run(1)
+        for k, name in ((0, "p"), (1, "q")):
+            np.testing.assert_array_equal(many[2][k].get(name), one[2][k].get(name))
+        for k in (0, 2):
+            a, b = many[2][k].get("spike"), one[2][k].get("spike")
+            assert a == b if isinstance(a, dict) else np.array_equal(a, b)
+        np.testing.assert_array_equal(many[1].p, one[1].p)

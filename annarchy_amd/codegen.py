@@ -28,7 +28,7 @@ import re
 
 from .equations import DISTRIBUTIONS, NeuronDescription, analyse_neuron, equation_code
 
-ABI = 14  # AHIP_MODEL_ABI in include/annarchy_hip_model.h
+ABI = 15  # AHIP_MODEL_ABI in include/annarchy_hip_model.h
 
 _PRELUDE = r"""// Generated neuron-model library for the MI355X simulation backend.
 // Model: %(name)s
@@ -278,8 +278,8 @@ __global__ __launch_bounds__(AHIP_PERSIST_THREADS) void persistent_steps(ahip_po
     if (tid == 0) {
         nspk_s = *pa.spike_count;
         if (pa.rec_counts) {
-            fill_s[0] = pa.rec_fill[0];
-            fill_s[1] = pa.rec_fill[1];
+            const int64_t row = max((int64_t)0, *a.t_base + a.step - pa.rec_state->t_start);
+            fill_s[0] = fill_s[1] = pa.rec_fill[row & (AHIP_FILL_RING - 1)];
         }
     }
     persist_sync();
@@ -464,10 +464,8 @@ __global__ __launch_bounds__(AHIP_PERSIST_THREADS) void persistent_steps(ahip_po
     }
     if (tid == 0) {
         *pa.spike_count = nspk;
-        if (pa.rec_counts) {
-            pa.rec_fill[0] = fill_s[0];
-            pa.rec_fill[1] = fill_s[1];
-        }
+        if (pa.rec_counts)   // (the next row's entry is all that is read)
+            for (int r = 0; r < AHIP_FILL_RING; r++) pa.rec_fill[r] = fill_s[r & 1];
     }
 }
 

@@ -77,6 +77,9 @@ struct Pop {
     // slice of its mask and counts this step's compaction reads (-1: of one step)
     bool ahead = false;
     int32_t ahead_at = -1;
+    // spikes read from the mask by the scatter of the next step, compacted
+    // AHIP_AHEAD steps at a time
+    bool deferred = false;
     bool fused = false;
     ahip_fuse_args fuse;
     // mean firing rate over fr_window steps (0: off): a fr_window-bit history
@@ -180,7 +183,7 @@ struct Monitor {
     DevBuf state;                 // ahip_record_state: what the kernels read of the above
     DevBuf data;                  // values [capacity][size] (T), or spike indices
     DevBuf counts;                // spikes: int32[capacity]
-    DevBuf fill;                  // spikes: int64[2], indices written before recorded step s in fill[s & 1]
+    DevBuf fill;                  // spikes: int64[AHIP_FILL_RING], indices before row s in fill[s mod AHIP_FILL_RING]
     int64_t idx_capacity = 0;
 };
 
@@ -221,7 +224,15 @@ struct ScatterDesc {
     void* ring;
     const int16_t* delay_col;
     int32_t ring_depth, n_post;
+    // spikes of a step that is not compacted yet (mask != NULL: instead of list):
+    // its mask words and the counts of its n_blocks update blocks
+    const uint64_t* mask;
+    const int32_t* block_counts;
+    int32_t n_blocks, n_words;
+    int32_t pre;              // host: the pre population
 };
+// blocks of a mask that a wave's lanes can hold the counts of
+constexpr int32_t kMaskBlocks = 8 * 64;
 constexpr int kMaxScatter = 8;
 // One projection feeding an ordered target: its keys are [gid_off, gid_end),
 // key k names column-order synapse k - gid_off of that projection.
@@ -330,7 +341,12 @@ inline const Monitor* first_spike_monitor(const ahip_net* net, int32_t pop) {
     return nullptr;
 }
 int launch_update_rate(const ahip_net* net, const Pop& p, int32_t step, hipStream_t s, bool active = true);
-int launch_scatter_group(const ahip_net* net, const ScatterGroup& g, int32_t step, hipStream_t s);
+// `deferred`: the lists of deferred populations are those of a step of this batch
+// that is not compacted yet
+int launch_scatter_group(const ahip_net* net, const ScatterGroup& g, int32_t step, bool deferred, hipStream_t s);
+// the last `steps` steps of the batch up to `step`, of deferred populations
+int launch_compact_steps(const ahip_net* net, const std::vector<int32_t>& pops, const int64_t* t_base, int32_t step,
+                         int32_t steps, hipStream_t s);
 int launch_deliver(const ahip_net* net, hipStream_t s);
 int launch_push_values(const ahip_net* net, const void* src, void* hist, int32_t n, int32_t D, int32_t step,
                        hipStream_t s);

@@ -12,6 +12,8 @@ constexpr int kCompactWaves = kCompactThreads / kWave;
 constexpr int kCompactWords = 4;                                      // 64-neuron words of a wave
 constexpr int kCompactChunk = kCompactThreads * kCompactWords;        // 4096 neurons
 static_assert(kCompactChunk % AHIP_UPDATE_BLOCK == 0, "chunk must cover whole update blocks");
+static_assert(kMaskBlocks % kWave == 0 && AHIP_FILL_RING > AHIP_AHEAD + 1 && AHIP_FILL_RING <= kWave,
+              "a launch reads no fill count that it writes; one count a lane");
 static_assert(kCompactWaves == 16, "the wave totals are read as one row");
 
 // Spike compaction, ascending neuron order (the order of the CPU gather,
@@ -27,14 +29,14 @@ static_assert(kCompactWaves == 16, "the wave totals are read as one row");
 // neurons in a kernel trace; this form takes 3.6.
 // With a spike monitor (rec_counts != NULL) the kernel also appends the list
 // to it: the monitor's index buffer holds the lists of the recorded steps
-// back to back; fill[s & 1] is the number of indices before the list of
-// recorded step s (written by step s - 1's launch, so no workgroup of this
+// back to back; fill[s mod AHIP_FILL_RING] is the number of indices before the
+// list of row s (written by the launch of row s - 1, so no workgroup of this
 // launch reads a value another one writes), the last workgroup writes
-// counts[s] and fill[(s + 1) & 1].
+// counts[s] and fill[s + 1].
 struct SpikeRec {
     int32_t* counts;          // int32[capacity] spikes per recorded step, NULL: no monitor
     int32_t* idx;             // int32[idx_capacity]
-    int64_t* fill;            // int64[2]
+    int64_t* fill;            // int64[AHIP_FILL_RING]
     int64_t idx_capacity;
     const ahip_record_state* state;
 };
@@ -51,10 +53,14 @@ struct CompactArgs {
     SpikeRec rec;
 };
 
-// Chunk b of a population's compaction at step t_base + step.
+// Chunk b of a population's compaction at step t_base + step.  STEPS: step y of a
+// launch of `steps` that starts there; the mask words and block counts of a step
+// follow those of the step before.  The list goes to the monitor; spiked and count
+// are those of the last step.
+template <bool STEPS>
 __device__ inline void compact_chunk(const CompactArgs& c, int32_t b, const int64_t* __restrict__ t_base,
-                                     int32_t step) {
-    __shared__ int32_t wave_part[kCompactWaves], wave_total[kCompactWaves];
+                                     int32_t step, int32_t y, int32_t steps) {
+    __shared__ int32_t wave_part[kCompactWaves], wave_total[kCompactWaves], wave_rec[kCompactWaves];
     const int32_t size = c.size;
     const SpikeRec& rec = c.rec;
     const int lane = threadIdx.x & (kWave - 1);
@@ -65,29 +71,43 @@ __device__ inline void compact_chunk(const CompactArgs& c, int32_t b, const int6
     // mask words, this thread's share of the block counts before the chunk, the
     // monitor's fill counts
     const int32_t n0 = chunk0 + wave * kCompactWords * kWave;   // first neuron of the wave
+    const int32_t nw = (size + kWave - 1) / kWave, nub = (size + AHIP_UPDATE_BLOCK - 1) / AHIP_UPDATE_BLOCK;
+    const uint64_t* mask = c.mask + (STEPS ? (int64_t)y * nw : 0);
+    const int32_t* bcnt = c.bcnt + (STEPS ? (int64_t)y * nub : 0);
     uint64_t word[kCompactWords];
 #pragma unroll
     for (int k = 0; k < kCompactWords; k++) {
         const int32_t left = size - (n0 + k * kWave);           // neurons from this word on
-        word[k] = left > 0 ? c.mask[n0 / kWave + k] : 0ull;
+        word[k] = left > 0 ? mask[n0 / kWave + k] : 0ull;
         if (left > 0 && left < kWave) word[k] &= (1ull << left) - 1ull;
     }
     int32_t part = 0;
-    for (int32_t k = threadIdx.x; k < ub0; k += kCompactThreads) part += c.bcnt[k];
+    for (int32_t k = threadIdx.x; k < ub0; k += kCompactThreads) part += bcnt[k];
     int64_t slot = -1, f = 0;
-    const int64_t t = *t_base + step;
+    const int64_t t = *t_base + step + (STEPS ? y : 0);
+    int32_t earlier = 0;   // spikes of the launch's recorded steps before this one
     if (rec.counts) {
-        const int64_t fill0 = rec.fill[0], fill1 = rec.fill[1];
+        const int64_t fills = rec.fill[lane & (AHIP_FILL_RING - 1)];
         slot = record_row(*rec.state, t);
-        if (slot >= 0) f = (slot & 1) ? fill1 : fill0;
+        if (slot >= 0) {
+            // (a spike monitor's rows are consecutive steps)
+            const int32_t back = STEPS ? (int32_t)min((int64_t)y, slot) : 0;
+            const int at = (int)(slot - back) & (AHIP_FILL_RING - 1);
+            f = ((int64_t)__builtin_amdgcn_readlane((int)(fills >> 32), at) << 32) |
+                (uint32_t)__builtin_amdgcn_readlane((int)fills, at);
+            if (STEPS)
+                for (int32_t k = (y - back) * nub + (int32_t)threadIdx.x; k < y * nub; k += kCompactThreads) earlier += c.bcnt[k];
+        }
     }
     part = group_sum<kWave>(part);
+    if (STEPS) earlier = group_sum<kWave>(earlier);
     int32_t total = 0;
 #pragma unroll
     for (int k = 0; k < kCompactWords; k++) total += (int32_t)__popcll(word[k]);
     if (lane == 0) {
         wave_part[wave] = part;
         wave_total[wave] = total;
+        if (STEPS) wave_rec[wave] = earlier;
     }
     __syncthreads();
     // spikes before the chunk, before this wave in it, and in all of it
@@ -98,7 +118,9 @@ __device__ inline void compact_chunk(const CompactArgs& c, int32_t b, const int6
         base += wave_part[w];
         before += w < wave ? v : 0;
         all += v;
+        if (STEPS) f += wave_rec[w];
     }
+    const bool last = !STEPS || y == steps - 1;
     int32_t pos0 = base + before;
 #pragma unroll
     for (int k = 0; k < kCompactWords; k++) {
@@ -106,18 +128,23 @@ __device__ inline void compact_chunk(const CompactArgs& c, int32_t b, const int6
             const int32_t pos = pos0 + (int32_t)__builtin_amdgcn_mbcnt_hi(
                                            (uint32_t)(word[k] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)word[k], 0u));
             const int32_t i = n0 + k * kWave + lane;
-            c.spiked[pos] = i;
-            if (c.last_spike) c.last_spike[i] = t;
+            if (last) c.spiked[pos] = i;
+            if (c.last_spike) {
+                bool later = false;   // the neuron's last spike of the launch counts
+                if (STEPS)
+                    for (int32_t u = 1; u < steps - y; u++) later |= ((mask[(int64_t)u * nw + n0 / kWave + k] >> lane) & 1ull) != 0;
+                if (!later) c.last_spike[i] = t;
+            }
             if (slot >= 0 && f + pos < rec.idx_capacity) rec.idx[f + pos] = i;
         }
         pos0 += (int32_t)__popcll(word[k]);
     }
     // grand total: the last chunk knows base + its own total
     if (b == c.nb - 1 && threadIdx.x == 0) {
-        *c.count = base + all;
+        if (last) *c.count = base + all;
         if (slot >= 0) {
             rec.counts[slot] = base + all;
-            rec.fill[(slot + 1) & 1] = f + base + all;
+            rec.fill[(slot + 1) & (AHIP_FILL_RING - 1)] = f + base + all;
         }
     }
 }
@@ -131,12 +158,13 @@ struct CompactBatch {
     int32_t n;
 };
 
+template <bool STEPS>
 __global__ __launch_bounds__(kCompactThreads) void compact_spikes(const CompactBatch B,
                                                                   const int64_t* __restrict__ t_base, int32_t step) {
     const int32_t bid = __builtin_amdgcn_readfirstlane((int32_t)blockIdx.x);
     int32_t k = 0;
     while (k < B.n - 1 && bid >= B.b0[k + 1]) k++;
-    compact_chunk(B.c[k], bid - B.b0[k], t_base, step);
+    compact_chunk<STEPS>(B.c[k], bid - B.b0[k], t_base, step, (int32_t)blockIdx.y, (int32_t)gridDim.y);
 }
 
 // Event-driven propagation over the compacted spike list, CSRC backward view
@@ -224,7 +252,83 @@ struct ScatterArgs {
     int32_t waves_per;
 };
 
-template <typename T>
+// The spikes of a step as its update left them: a mask and the counts of its
+// blocks of 256 neurons.  The lanes of a wave hold the counts (up to
+// kMaskBlocks) and their running sums; spike s is in the block whose sum passes
+// s, at the bit of its 4 words with as many bits below.  Reading the mask takes
+// the compaction out of the chain of a step (launch, mask -> barrier -> list) for
+// some 200 cycles more here (us per step with a compaction at every step / at
+// every 16th: COBA with 20003 neurons 12.7 / 10.5, with 80000 15.1 / 12.5).
+struct MaskSpikes {
+    gptr<const uint64_t> mask;
+    int32_t cnt[kMaskBlocks / kWave];
+    int32_t per, sum, incl, nw, nb;
+    int32_t at, rank;   // block of the next spike, its rank there
+    uint64_t word;      // lane l: word l & 3 of the block
+    __device__ inline int32_t load(const ScatterDesc& d, int lane) {
+        mask = as_global(d.mask);
+        nb = d.n_blocks;
+        nw = d.n_words;
+        per = (nb + kWave - 1) / kWave;
+        const auto bc = as_global(d.block_counts);
+#pragma unroll
+        for (int q = 0; q < kMaskBlocks / kWave; q++) {
+            const int32_t b = lane * per + q;
+            cnt[q] = q < per && b < nb ? bc[b] : 0;
+        }
+        sum = 0;
+#pragma unroll
+        for (int q = 0; q < kMaskBlocks / kWave; q++) sum += cnt[q];
+        int v = sum;
+        v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr 1, 2, 4, 8
+        v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+        v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+        v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+        v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast 15, 31
+        v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+        incl = v;
+        return __builtin_amdgcn_readlane(v, kWave - 1);
+    }
+    // the loads of spike s (below the number of spikes)
+    __device__ inline void seek(int32_t s, int lane) {
+        const int l = __builtin_ctzll(__ballot(incl > s));
+        int32_t r = s - (__builtin_amdgcn_readlane(incl, l) - __builtin_amdgcn_readlane(sum, l));
+        int32_t q = 0;
+        bool found = false;
+#pragma unroll
+        for (int k = 0; k < kMaskBlocks / kWave; k++) {
+            const int32_t c = __builtin_amdgcn_readlane(cnt[k], l);
+            found = found || r < c;
+            if (!found) {
+                r -= c;
+                q++;
+            }
+        }
+        at = l * per + q;
+        rank = r;
+        const int32_t w = at * (AHIP_UPDATE_BLOCK / kWave) + (lane & (AHIP_UPDATE_BLOCK / kWave - 1));
+        word = w < nw ? mask[w] : 0ull;
+    }
+    __device__ inline int32_t neuron(int lane) const {
+        int32_t r = rank;
+        int32_t pre = -1;
+#pragma unroll
+        for (int k = 0; k < AHIP_UPDATE_BLOCK / kWave; k++) {
+            const uint64_t m = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(word >> 32), k) << 32) |
+                               (uint32_t)__builtin_amdgcn_readlane((int)word, k);
+            const int32_t c = (int32_t)__builtin_popcountll(m);
+            if (r >= 0 && r < c) {
+                const int32_t below = (int32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                                         __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                pre = at * AHIP_UPDATE_BLOCK + k * kWave + __builtin_ctzll(__ballot(((m >> lane) & 1ull) && below == r));
+            }
+            r -= c;
+        }
+        return pre;
+    }
+};
+
+template <typename T, bool MASK>
 __global__ __launch_bounds__(256) void scatter_multi(const ScatterArgs A, const int64_t* __restrict__ t_base,
                                                      int32_t step) {
     const int lane = threadIdx.x & (kWave - 1);
@@ -241,12 +345,24 @@ __global__ __launch_bounds__(256) void scatter_multi(const ScatterArgs A, const 
     // (a list never holds more than n_cols entries)
     const EventWalk W(lw, A.waves_per, d.chunks);
     int32_t s = W.s0, c_next = W.c0;
-    int32_t next = s < d.n_cols ? list[s] : -1;
-    const int32_t n = as_global(d.count)[sl];
+    MaskSpikes M;
+    const bool masked = MASK && d.mask != nullptr;
+    int32_t next = -1, n;
+    if (masked) {
+        n = M.load(d, lane);
+        if (s < n) M.seek(s, lane);
+    } else {
+        next = s < d.n_cols ? list[s] : -1;
+        n = as_global(d.count)[sl];
+    }
     while (s < n) {
-        const int32_t pre = next, c = c_next;
+        const int32_t pre = masked ? M.neuron(lane) : next, c = c_next;
         W.step(s, c_next);
-        next = s < n ? list[s] : -1;
+        if (masked) {
+            if (s < n) M.seek(s, lane);
+        } else {
+            next = s < n ? list[s] : -1;
+        }
         if (pre < 0 || pre >= d.n_cols) continue;
         const int64_t b = as_global(d.col_ptr)[pre], e = as_global(d.col_ptr)[pre + 1];
         const auto ri = as_global(d.row_idx);
@@ -383,12 +499,12 @@ __global__ __launch_bounds__(256) void record_spikes(const int32_t* __restrict__
     const int64_t slot = record_row(*state, *t_base + step);
     if (slot < 0) return;
     const int32_t n = *count;
-    const int64_t f = fill[slot & 1];   // same double-buffered fill as compact_spikes
+    const int64_t f = fill[slot & (AHIP_FILL_RING - 1)];   // as compact_spikes
     for (int32_t k = threadIdx.x; k < n; k += 256)
         if (f + k < idx_capacity) idx[f + k] = spiked[k];
     if (threadIdx.x == 0) {
         counts[slot] = n;
-        fill[(slot + 1) & 1] = f + n;
+        fill[(slot + 1) & (AHIP_FILL_RING - 1)] = f + n;
     }
 }
 
@@ -438,8 +554,8 @@ int launch_update_rate(const ahip_net* net, const Pop& p, int32_t step, hipStrea
     return (int)hipGetLastError();
 }
 
-int launch_compact(const ahip_net* net, const std::vector<int32_t>& pops, const int64_t* t_base, int32_t step,
-                   hipStream_t s) {
+static int launch_compactions(const ahip_net* net, const std::vector<int32_t>& pops, const int64_t* t_base,
+                              int32_t step, int32_t steps, hipStream_t s) {
     for (size_t first = 0; first < pops.size(); first += kMaxCompact) {
         CompactBatch B;
         std::memset(&B, 0, sizeof(B));
@@ -452,9 +568,10 @@ int launch_compact(const ahip_net* net, const std::vector<int32_t>& pops, const 
             c.mask = p.spike_mask.as<uint64_t>();
             c.bcnt = p.block_counts.as<int32_t>();
             if (p.ahead_at >= 0) {
-                c.mask += (int64_t)p.ahead_at * p.nwords();
-                c.bcnt += (int64_t)p.ahead_at * p.nblocks();
-                c.last_spike = p.last_spike.as<int64_t>();
+                // (steps > 0: the launch starts at the first of the kept steps)
+                c.mask += steps > 0 ? 0 : (int64_t)p.ahead_at * p.nwords();
+                c.bcnt += steps > 0 ? 0 : (int64_t)p.ahead_at * p.nblocks();
+                if (p.ahead) c.last_spike = p.last_spike.as<int64_t>();
             }
             c.spiked = p.spiked.as<int32_t>();
             c.count = p.spike_count.as<int32_t>();
@@ -469,27 +586,59 @@ int launch_compact(const ahip_net* net, const std::vector<int32_t>& pops, const 
             B.n++;
         }
         if (B.b0[B.n] == 0) continue;
-        hipLaunchKernelGGL(compact_spikes, dim3((unsigned)B.b0[B.n]), dim3(kCompactThreads), 0, s, B, t_base, step);
+        if (steps > 0)
+            hipLaunchKernelGGL(compact_spikes<true>, dim3((unsigned)B.b0[B.n], (unsigned)steps), dim3(kCompactThreads), 0,
+                               s, B, t_base, step);
+        else
+            hipLaunchKernelGGL(compact_spikes<false>, dim3((unsigned)B.b0[B.n]), dim3(kCompactThreads), 0, s, B, t_base,
+                               step);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return (int)e;
     }
     return 0;
 }
 
-int launch_scatter_group(const ahip_net* net, const ScatterGroup& g, int32_t step, hipStream_t s) {
+int launch_compact(const ahip_net* net, const std::vector<int32_t>& pops, const int64_t* t_base, int32_t step,
+                   hipStream_t s) {
+    return launch_compactions(net, pops, t_base, step, 0, s);
+}
+
+int launch_compact_steps(const ahip_net* net, const std::vector<int32_t>& pops, const int64_t* t_base, int32_t step,
+                         int32_t steps, hipStream_t s) {
+    return launch_compactions(net, pops, t_base, step - (steps - 1), steps, s);
+}
+
+template <typename T>
+static void launch_scatter(const ahip_net* net, const ScatterGroup& g, const ScatterArgs& A, int32_t step, bool mask,
+                           hipStream_t s) {
+    if (mask)
+        hipLaunchKernelGGL((scatter_multi<T, true>), dim3(g.blocks), dim3(256), 0, s, A, net->t_dev.as<int64_t>(), step);
+    else
+        hipLaunchKernelGGL((scatter_multi<T, false>), dim3(g.blocks), dim3(256), 0, s, A, net->t_dev.as<int64_t>(), step);
+}
+
+int launch_scatter_group(const ahip_net* net, const ScatterGroup& g, int32_t step, bool deferred, hipStream_t s) {
     if (g.n == 0) return 0;
     if (g.n > kMaxScatter) return (int)hipErrorInvalidValue;
     ScatterArgs A;
     std::memset(&A, 0, sizeof(A));
-    for (int32_t k = 0; k < g.n; k++) A.d[k] = g.descs[k];
+    bool mask = false;
+    for (int32_t k = 0; k < g.n; k++) {
+        ScatterDesc& d = A.d[k] = g.descs[k];
+        const Pop& pre = *net->pops[d.pre];
+        if (!deferred || !pre.deferred) continue;
+        // the step before, of this batch
+        const int32_t at = (step - 1) % AHIP_AHEAD;
+        d.mask = pre.spike_mask.as<uint64_t>() + (int64_t)at * pre.nwords();
+        d.block_counts = pre.block_counts.as<int32_t>() + (int64_t)at * pre.nblocks();
+        d.n_blocks = pre.nblocks();
+        d.n_words = pre.nwords();
+        mask = true;
+    }
     A.nd = g.n;
     A.waves_per = g.waves_per;
-    if (net->precision == AHIP_F64)
-        hipLaunchKernelGGL(scatter_multi<double>, dim3(g.blocks), dim3(256), 0, s, A, net->t_dev.as<int64_t>(),
-                           step);
-    else
-        hipLaunchKernelGGL(scatter_multi<float>, dim3(g.blocks), dim3(256), 0, s, A, net->t_dev.as<int64_t>(),
-                           step);
+    if (net->precision == AHIP_F64) launch_scatter<double>(net, g, A, step, mask, s);
+    else launch_scatter<float>(net, g, A, step, mask, s);
     return (int)hipGetLastError();
 }
 

@@ -699,6 +699,10 @@ int prepare(ahip_net* net) {
             d.shards = 1;
             d.shard_cap = 0;
             d.gid_off = 0;
+            d.mask = nullptr;
+            d.block_counts = nullptr;
+            d.n_blocks = d.n_words = 0;
+            d.pre = p.pre;
             d.ring = !p.counted ? nullptr : p.delay_per_syn ? p.ring.p : p.cnt.p;
             d.delay_col = p.delay_per_syn ? p.delay_dev.as<int16_t>() : nullptr;
             d.ring_depth = p.delay_per_syn ? p.ring_depth() : 1;
@@ -805,6 +809,24 @@ static bool fuse_desc(ahip_net* net, const Proj& p, int32_t sum, ahip_fuse_proj&
 // (45.7 / 81.6 at 12000 x 2000, dense 89.3 / 90.2 at 8000 x 8000).
 constexpr int64_t kFuseMaxGathered = 1 << 24, kFuseMaxStaged = 1 << 27;
 
+// Populations whose compaction can wait for the end of 16 steps: every reader of
+// their spikes inside a batch is a scatter of the next step (which reads the
+// mask), none a plastic projection, a delay queue, the firing-rate window, a
+// second spike monitor or the ring kernel of delays per synapse.  Up to
+// kMaskBlocks blocks, 131072 neurons.
+static bool may_defer(const ahip_net* net, const Pop& p) {
+    if (!p.model->spiking || !p.active || p.depth > 1 || p.fr_window > 0 || p.nblocks() > kMaskBlocks) return false;
+    for (auto& qq : net->projs) {
+        const Proj& q = *qq;
+        if (q.pre != p.id && q.post != p.id) continue;
+        if (q.syn) return false;
+        if (q.pre == p.id && (!q.spiking || (q.delay_per_syn && !q.counted && q.nnz > 0 && transmits(net, q)))) return false;
+    }
+    for (auto& mp : net->mons)
+        if (mp->spikes && mp->pop == p.id && !mp->paused && first_spike_monitor(net, p.id) != mp.get()) return false;
+    return true;
+}
+
 // The input populations that run ahead: nothing inside a batch may read their
 // values other than through the rings and spike lists, which hold every step's
 // (plastic projections that read pre.<name>, monitors with a kernel of their own
@@ -823,9 +845,11 @@ static int assign_ahead(ahip_net* net) {
         if (!p.model->spiking && p.depth > 1 && p.depth < oldest + AHIP_AHEAD) ok = false;
         for (auto& mp : net->mons)
             if (mp->pop == p.id && !mp->paused && !mp->spikes && (!mp->in_update || (mp->after_psp && p.model->spiking))) ok = false;
-        if (ok != p.ahead) drop_graph(net);
+        const bool defer = may_defer(net, p);
+        if (ok != p.ahead || defer != p.deferred) drop_graph(net);
         p.ahead = ok;
-        if (ok && p.model->spiking && p.spike_mask.bytes < (size_t)AHIP_AHEAD * p.nwords() * sizeof(uint64_t)) {
+        p.deferred = defer;
+        if (p.model->spiking && (ok || defer) && p.spike_mask.bytes < (size_t)AHIP_AHEAD * p.nwords() * sizeof(uint64_t)) {
             HIPCHK(hipStreamSynchronize(net->stream));
             int rc = dev_alloc(p.spike_mask, (size_t)AHIP_AHEAD * p.nwords() * sizeof(uint64_t));
             if (!rc) rc = dev_alloc(p.block_counts, (size_t)AHIP_AHEAD * p.nblocks() * sizeof(int32_t));
@@ -1106,12 +1130,14 @@ ahip_pop_args make_args(ahip_net* net, Pop& p, int32_t step) {
 int enqueue_step(ahip_net* net, int32_t step, int32_t nsteps, const std::vector<int32_t>& zero_before) {
     hipStream_t s = net->stream;
     const size_t es = net->elem();
+    // several steps at a time: input populations, compactions
+    const bool deferring = nsteps > 1 && net->probe_kind < 0;
     // 1. compute_psp: the spiking projections in fused scatter groups, then
     // the rate-coded ones
     for (size_t gi = 0; gi < net->scatter_groups.size(); gi++) {
         const bool probe = net->probe_kind == AHIP_PROBE_SCATTER && net->probe_proj == (int32_t)gi;
         if (probe) HIPCHK(hipEventRecord(net->probe_ev[0], s));
-        LCHK(launch_scatter_group(net, net->scatter_groups[gi], step, s));
+        LCHK(launch_scatter_group(net, net->scatter_groups[gi], step, deferring && step > 0, s));
         if (probe) HIPCHK(hipEventRecord(net->probe_ev[1], s));
     }
     if (net->deliver_waves > 0) {
@@ -1168,7 +1194,7 @@ int enqueue_step(ahip_net* net, int32_t step, int32_t nsteps, const std::vector<
     // compactions of the updated spiking populations in one launch (no
     // update reads another population's compaction), then each population's
     // firing-rate window and delay push
-    std::vector<int32_t> compact;
+    std::vector<int32_t> compact, deferred;
     for (auto& pp : net->pops) {
         Pop& p = *pp;
         if (!p.active) {
@@ -1182,15 +1208,18 @@ int enqueue_step(ahip_net* net, int32_t step, int32_t nsteps, const std::vector<
             continue;
         }
         ahip_pop_args a = make_args(net, p, step);
-        p.ahead_at = -1;
-        if (p.ahead && nsteps > 1 && net->probe_kind < 0) {
+        p.ahead_at = deferring && (p.ahead || p.deferred) ? step % AHIP_AHEAD : -1;
+        if (p.ahead && deferring) {
             if (step % AHIP_AHEAD == 0) {
                 const ahip_ahead_fn fn = net->precision == AHIP_F64 ? p.model->ahead_f64 : p.model->ahead_f32;
                 LCHK(fn(&a, std::min<int32_t>(AHIP_AHEAD, nsteps - step), (void*)s));
             }
-            p.ahead_at = step % AHIP_AHEAD;
-            if (p.model->spiking) compact.push_back(p.id);
+            if (p.model->spiking) (p.deferred ? deferred : compact).push_back(p.id);
             continue;
+        }
+        if (p.ahead_at >= 0) {
+            a.spike_mask += (int64_t)p.ahead_at * p.nwords();
+            a.block_counts += (int64_t)p.ahead_at * p.nblocks();
         }
         ahip_launch_fn fn = net->precision == AHIP_F64 ? p.model->launch_f64 : p.model->launch_f32;
         const bool probe_u = net->probe_kind == AHIP_PROBE_UPDATE && net->probe_proj == p.id;
@@ -1200,8 +1229,11 @@ int enqueue_step(ahip_net* net, int32_t step, int32_t nsteps, const std::vector<
         if (rc != 0) return fail(AHIP_EHIP, "update of population %d failed: %s", p.id,
                                  hipGetErrorString((hipError_t)rc));
         if (probe_u) HIPCHK(hipEventRecord(net->probe_ev[1], s));
-        if (p.model->spiking) compact.push_back(p.id);
+        if (p.model->spiking) (p.ahead_at >= 0 ? deferred : compact).push_back(p.id);
     }
+    const int32_t kept = step % AHIP_AHEAD + 1;
+    if (!deferred.empty() && (kept == AHIP_AHEAD || step == nsteps - 1))
+        LCHK(launch_compact_steps(net, deferred, net->t_dev.as<int64_t>(), step, kept, s));
     if (!compact.empty()) {
         const bool probe_c = net->probe_kind == AHIP_PROBE_COMPACT &&
                              std::find(compact.begin(), compact.end(), net->probe_proj) != compact.end();
@@ -2755,7 +2787,7 @@ int ahip_monitor_create(ahip_net* net, int32_t pop, const char* attr, int64_t ca
         m->idx_capacity = cap;
         if ((rc = dev_alloc(m->data, cap * sizeof(int32_t)))) return rc;
         if ((rc = dev_alloc(m->counts, capacity * sizeof(int32_t)))) return rc;
-        if ((rc = dev_alloc(m->fill, 2 * sizeof(int64_t)))) return rc;
+        if ((rc = dev_alloc(m->fill, AHIP_FILL_RING * sizeof(int64_t)))) return rc;
     } else {
         m->slot = p->slot_index(attr);
         if (m->slot < 0 || !p->model->slot_local[m->slot])
@@ -2870,9 +2902,9 @@ int ahip_monitor_get_spikes(ahip_net* net, int32_t mon, int32_t* counts, int64_t
     ahip_monitor_steps(net, mon, &have);
     if (steps != have) return fail(AHIP_EINVAL, "monitor holds %lld steps", (long long)have);
     HIPCHK(hipStreamSynchronize(net->stream));
-    int64_t fills[2] = {0, 0};
-    HIPCHK(hipMemcpy(fills, m->fill.p, 2 * sizeof(int64_t), hipMemcpyDeviceToHost));
-    const int64_t fill = have > 0 ? fills[have & 1] : 0;   // indices before recorded step `have`
+    int64_t fills[AHIP_FILL_RING] = {0};
+    HIPCHK(hipMemcpy(fills, m->fill.p, sizeof(fills), hipMemcpyDeviceToHost));
+    const int64_t fill = have > 0 ? fills[have % AHIP_FILL_RING] : 0;   // indices before recorded step `have`
     *total = fill;
     if (fill > m->idx_capacity) return fail(AHIP_ESTATE, "spike monitor overflowed its buffer");
     if (counts && steps > 0) HIPCHK(hipMemcpy(counts, m->counts.p, steps * sizeof(int32_t), hipMemcpyDeviceToHost));
@@ -2890,7 +2922,7 @@ int ahip_monitor_clear(ahip_net* net, int32_t mon) {
     if (m->spikes) {
         m->t_start = net->t;
         m->seg_base = 0;
-        LCHK(launch_fill_i64(m->fill.as<int64_t>(), 2, 0, net->stream));
+        LCHK(launch_fill_i64(m->fill.as<int64_t>(), AHIP_FILL_RING, 0, net->stream));
         HIPCHK(hipStreamSynchronize(net->stream));
     } else {
         m->seg_base = 0;

@@ -22,7 +22,7 @@
 extern "C" {
 #endif
 
-#define AHIP_MODEL_ABI 14
+#define AHIP_MODEL_ABI 15
 #define AHIP_MAX_SLOTS 48
 #define AHIP_MAX_RAND 8
 #define AHIP_UPDATE_BLOCK 256 /* threads per block of every update kernel */
@@ -69,6 +69,7 @@ typedef struct ahip_record_state {
     int64_t t_start, base, period, capacity;
 } ahip_record_state;
 #define AHIP_MAX_REC 4     /* value monitors one update records */
+#define AHIP_FILL_RING 32  /* > steps of one compaction launch + 1, a power of two */
 
 /* Arguments of one population update launch.  Device pointers unless noted. */
 typedef struct ahip_pop_args {
@@ -85,7 +86,7 @@ typedef struct ahip_pop_args {
     int32_t* refractory;                /* steps, per neuron */
     int32_t* refractory_remaining;
     int64_t* last_spike;
-    uint64_t* spike_mask;               /* ceil(size/64) words, bit i = neuron spiked */
+    uint64_t* spike_mask;               /* ceil(size/64) words, bit i = neuron spiked (of this step) */
     int32_t* block_counts;              /* ceil(size/256) spike counts per update block */
     const ahip_deliver_desc* deliver;   /* ordered conductances delivered by this update, or NULL */
     int32_t n_deliver;
@@ -210,7 +211,7 @@ typedef struct ahip_persist_args {
      * by the compaction of the per-kernel step */
     int32_t* rec_counts;
     int32_t* rec_idx;
-    int64_t* rec_fill;
+    int64_t* rec_fill;                  /* [s mod AHIP_FILL_RING]: indices before the list of row s */
     int64_t rec_idx_capacity;
     const ahip_record_state* rec_state;
 } ahip_persist_args;

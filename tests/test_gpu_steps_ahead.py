@@ -102,3 +102,46 @@ def test_spikes_ahead_are_the_steps(gpu, n, uniform_delay):
             a, b = many[2][k].get("spike"), one[2][k].get("spike")
             assert a == b if isinstance(a, dict) else np.array_equal(a, b)
         np.testing.assert_array_equal(many[1].p, one[1].p)
+
+
+def _deferred(n, m, capacity):
+    """Spikes that a scatter reads from the mask, compacted 16 steps at a time."""
+    net = ah.Network(dt=1.0, seed=5)
+    pre, pop = net.create(n, Every5), net.create(m, Every5)
+    rng = np.random.default_rng(n)
+    k = min(3, n)
+    for w in (0.5, 0.25):
+        col = np.sort(rng.integers(0, n // k, (m, k)) + np.arange(k) * (n // k), axis=1).reshape(-1)
+        net.connect(pre, pop, "exc").from_csr(conn.from_arrays(m, n, np.arange(m + 1) * k, col, np.full(m * k, w)))
+    mons = [net.monitor(pre, ["spike"], capacity=capacity), net.monitor(pop, ["q", "spike"], capacity=capacity)]
+    net.compile(graph_batch=20)
+    # spikes in every block and in few of them
+    pre.v = np.where(np.arange(n) % 7 < 3, np.arange(n) % 5.0, 5.0 * (np.arange(n) >= n // 2) - 40.0)
+    pop.v = np.arange(m) % 5.0
+    return net, pop, mons
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 64, 257, 4100, 20011, 131072, 131073])
+def test_spikes_read_from_the_mask(gpu, n):
+    many, one = _deferred(n, 300, sum(RUNS)), _deferred(n, 300, sum(RUNS))
+    for steps in RUNS:
+        many[0].run(steps)
+        for _ in range(steps):
+            one[0].run(1)
+        np.testing.assert_array_equal(many[2][1].get("q", keep=True), one[2][1].get("q", keep=True))
+        for a, b in zip(many[2], one[2]):
+            for x, y in zip(a.raw_spikes(), b.raw_spikes()):
+                np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.gpu
+def test_a_full_monitor_keeps_its_rows(gpu):
+    # rows 24 on are not recorded: inside a launch of 16 steps, then all of them
+    many, one = _deferred(300, 300, 24), _deferred(300, 300, 24)
+    for steps in (20, 9, 20):
+        many[0].run(steps)
+        for _ in range(steps):
+            one[0].run(1)
+        for a, b in zip(many[2], one[2]):
+            assert a.get("spike", keep=True) == b.get("spike", keep=True)

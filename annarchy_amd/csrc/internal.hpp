@@ -146,6 +146,7 @@ struct Proj {
     // plasticity: a generated synapse model and its state.  State order:
     // spiking -> column order (as w_col), rate -> forward order (CSR val).
     void* syn_dl = nullptr;
+    int32_t syn_events = 0;       // AHIP_SYN_EVENTS_* of its library
     std::string syn_path;
     const ahip_synapse_desc* syn = nullptr;
     std::vector<DevBuf> syn_attr;            // per attribute: nnz / n_rows / 1 values (a per-synapse
@@ -231,8 +232,6 @@ struct ScatterDesc {
     int32_t n_blocks, n_words;
     int32_t pre;              // host: the pre population
 };
-// blocks of a mask that a wave's lanes can hold the counts of
-constexpr int32_t kMaskBlocks = 8 * 64;
 constexpr int kMaxScatter = 8;
 // One projection feeding an ordered target: its keys are [gid_off, gid_end),
 // key k names column-order synapse k - gid_off of that projection.

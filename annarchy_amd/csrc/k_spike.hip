@@ -12,7 +12,7 @@ constexpr int kCompactWaves = kCompactThreads / kWave;
 constexpr int kCompactWords = 4;                                      // 64-neuron words of a wave
 constexpr int kCompactChunk = kCompactThreads * kCompactWords;        // 4096 neurons
 static_assert(kCompactChunk % AHIP_UPDATE_BLOCK == 0, "chunk must cover whole update blocks");
-static_assert(kMaskBlocks % kWave == 0 && AHIP_FILL_RING > AHIP_AHEAD + 1 && AHIP_FILL_RING <= kWave,
+static_assert(AHIP_MASK_BLOCKS % kWave == 0 && AHIP_FILL_RING > AHIP_AHEAD + 1 && AHIP_FILL_RING <= kWave,
               "a launch reads no fill count that it writes; one count a lane");
 static_assert(kCompactWaves == 16, "the wave totals are read as one row");
 
@@ -252,82 +252,6 @@ struct ScatterArgs {
     int32_t waves_per;
 };
 
-// The spikes of a step as its update left them: a mask and the counts of its
-// blocks of 256 neurons.  The lanes of a wave hold the counts (up to
-// kMaskBlocks) and their running sums; spike s is in the block whose sum passes
-// s, at the bit of its 4 words with as many bits below.  Reading the mask takes
-// the compaction out of the chain of a step (launch, mask -> barrier -> list) for
-// some 200 cycles more here (us per step with a compaction at every step / at
-// every 16th: COBA with 20003 neurons 12.7 / 10.5, with 80000 15.1 / 12.5).
-struct MaskSpikes {
-    gptr<const uint64_t> mask;
-    int32_t cnt[kMaskBlocks / kWave];
-    int32_t per, sum, incl, nw, nb;
-    int32_t at, rank;   // block of the next spike, its rank there
-    uint64_t word;      // lane l: word l & 3 of the block
-    __device__ inline int32_t load(const ScatterDesc& d, int lane) {
-        mask = as_global(d.mask);
-        nb = d.n_blocks;
-        nw = d.n_words;
-        per = (nb + kWave - 1) / kWave;
-        const auto bc = as_global(d.block_counts);
-#pragma unroll
-        for (int q = 0; q < kMaskBlocks / kWave; q++) {
-            const int32_t b = lane * per + q;
-            cnt[q] = q < per && b < nb ? bc[b] : 0;
-        }
-        sum = 0;
-#pragma unroll
-        for (int q = 0; q < kMaskBlocks / kWave; q++) sum += cnt[q];
-        int v = sum;
-        v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr 1, 2, 4, 8
-        v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
-        v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
-        v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
-        v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast 15, 31
-        v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
-        incl = v;
-        return __builtin_amdgcn_readlane(v, kWave - 1);
-    }
-    // the loads of spike s (below the number of spikes)
-    __device__ inline void seek(int32_t s, int lane) {
-        const int l = __builtin_ctzll(__ballot(incl > s));
-        int32_t r = s - (__builtin_amdgcn_readlane(incl, l) - __builtin_amdgcn_readlane(sum, l));
-        int32_t q = 0;
-        bool found = false;
-#pragma unroll
-        for (int k = 0; k < kMaskBlocks / kWave; k++) {
-            const int32_t c = __builtin_amdgcn_readlane(cnt[k], l);
-            found = found || r < c;
-            if (!found) {
-                r -= c;
-                q++;
-            }
-        }
-        at = l * per + q;
-        rank = r;
-        const int32_t w = at * (AHIP_UPDATE_BLOCK / kWave) + (lane & (AHIP_UPDATE_BLOCK / kWave - 1));
-        word = w < nw ? mask[w] : 0ull;
-    }
-    __device__ inline int32_t neuron(int lane) const {
-        int32_t r = rank;
-        int32_t pre = -1;
-#pragma unroll
-        for (int k = 0; k < AHIP_UPDATE_BLOCK / kWave; k++) {
-            const uint64_t m = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(word >> 32), k) << 32) |
-                               (uint32_t)__builtin_amdgcn_readlane((int)word, k);
-            const int32_t c = (int32_t)__builtin_popcountll(m);
-            if (r >= 0 && r < c) {
-                const int32_t below = (int32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
-                                                                         __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-                pre = at * AHIP_UPDATE_BLOCK + k * kWave + __builtin_ctzll(__ballot(((m >> lane) & 1ull) && below == r));
-            }
-            r -= c;
-        }
-        return pre;
-    }
-};
-
 template <typename T, bool MASK>
 __global__ __launch_bounds__(256) void scatter_multi(const ScatterArgs A, const int64_t* __restrict__ t_base,
                                                      int32_t step) {
@@ -349,7 +273,7 @@ __global__ __launch_bounds__(256) void scatter_multi(const ScatterArgs A, const 
     const bool masked = MASK && d.mask != nullptr;
     int32_t next = -1, n;
     if (masked) {
-        n = M.load(d, lane);
+        n = M.load(d.mask, d.block_counts, d.n_blocks, d.n_words, lane);
         if (s < n) M.seek(s, lane);
     } else {
         next = s < d.n_cols ? list[s] : -1;

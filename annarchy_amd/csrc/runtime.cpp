@@ -303,20 +303,20 @@ int init_syn_state(ahip_net* net, Proj& p) {
 }
 
 
-int launch_syn_now(ahip_net* net, Proj& p, int kind, int32_t step);
+int launch_syn_now(ahip_net* net, Proj& p, int kind, int32_t step, bool deferring);
 
 // Pre events (kind 0), update_synapse (1) or post events (2) of a plastic
 // projection at `step`, between the probe events when this kernel is probed.
-int launch_syn(ahip_net* net, Proj& p, int kind, int32_t step) {
+int launch_syn(ahip_net* net, Proj& p, int kind, int32_t step, bool deferring) {
     const bool probe = net->probe_proj == p.id && net->probe_kind == kind;
     if (probe) HIPCHK(hipEventRecord(net->probe_ev[0], net->stream));
-    int rc = launch_syn_now(net, p, kind, step);
+    int rc = launch_syn_now(net, p, kind, step, deferring);
     if (rc) return rc;
     if (probe) HIPCHK(hipEventRecord(net->probe_ev[1], net->stream));
     return 0;
 }
 
-int launch_syn_now(ahip_net* net, Proj& p, int kind, int32_t step) {
+int launch_syn_now(ahip_net* net, Proj& p, int kind, int32_t step, bool deferring) {
     Pop& pre = *net->pops[p.pre];
     Pop& post = *net->pops[p.post];
     ahip_syn_args a;
@@ -332,6 +332,22 @@ int launch_syn_now(ahip_net* net, Proj& p, int kind, int32_t step) {
             a.pre_spiked = pre.spiked.as<int32_t>();
             a.pre_count = pre.spike_count.as<int32_t>();
             a.pre_depth = 1;
+        }
+        // spikes inside a batch that are compacted later: the pre events are those
+        // of the step before, the post events of this one
+        if (kind == 0 && deferring && step > 0 && pre.deferred) {
+            const int32_t at = (step - 1) % AHIP_AHEAD;
+            a.pre_mask = pre.spike_mask.as<uint64_t>() + (int64_t)at * pre.nwords();
+            a.pre_block_counts = pre.block_counts.as<int32_t>() + (int64_t)at * pre.nblocks();
+            a.pre_blocks = pre.nblocks();
+            a.pre_words = pre.nwords();
+        }
+        if (kind == 2 && deferring && post.deferred) {
+            const int32_t at = step % AHIP_AHEAD;
+            a.post_mask = post.spike_mask.as<uint64_t>() + (int64_t)at * post.nwords();
+            a.post_block_counts = post.block_counts.as<int32_t>() + (int64_t)at * post.nblocks();
+            a.post_blocks = post.nblocks();
+            a.post_words = post.nwords();
         }
         a.col_ptr = p.col_ptr.as<int64_t>();
         a.row_idx = p.row_idx.as<int32_t>();
@@ -810,16 +826,18 @@ static bool fuse_desc(ahip_net* net, const Proj& p, int32_t sum, ahip_fuse_proj&
 constexpr int64_t kFuseMaxGathered = 1 << 24, kFuseMaxStaged = 1 << 27;
 
 // Populations whose compaction can wait for the end of 16 steps: every reader of
-// their spikes inside a batch is a scatter of the next step (which reads the
-// mask), none a plastic projection, a delay queue, the firing-rate window, a
-// second spike monitor or the ring kernel of delays per synapse.  Up to
-// kMaskBlocks blocks, 131072 neurons.
+// their spikes inside a batch is a scatter of the next step or the events of a
+// plastic projection (which read the mask), none a delay queue, the firing-rate
+// window, a second spike monitor, the ring kernel of delays per synapse, or t_pre
+// of a population that runs ahead (its last spikes are kept by the compactions).
+// Up to AHIP_MASK_BLOCKS blocks, 131072 neurons.
 static bool may_defer(const ahip_net* net, const Pop& p) {
-    if (!p.model->spiking || !p.active || p.depth > 1 || p.fr_window > 0 || p.nblocks() > kMaskBlocks) return false;
+    if (!p.model->spiking || !p.active || p.depth > 1 || p.fr_window > 0 || p.nblocks() > AHIP_MASK_BLOCKS) return false;
     for (auto& qq : net->projs) {
         const Proj& q = *qq;
         if (q.pre != p.id && q.post != p.id) continue;
-        if (q.syn) return false;
+        if (q.syn && (!(q.syn_events & AHIP_SYN_EVENTS_MASK) ||
+                      (q.pre == p.id && p.ahead && (q.syn_events & AHIP_SYN_EVENTS_T_PRE)))) return false;
         if (q.pre == p.id && (!q.spiking || (q.delay_per_syn && !q.counted && q.nnz > 0 && transmits(net, q)))) return false;
     }
     for (auto& mp : net->mons)
@@ -845,10 +863,10 @@ static int assign_ahead(ahip_net* net) {
         if (!p.model->spiking && p.depth > 1 && p.depth < oldest + AHIP_AHEAD) ok = false;
         for (auto& mp : net->mons)
             if (mp->pop == p.id && !mp->paused && !mp->spikes && (!mp->in_update || (mp->after_psp && p.model->spiking))) ok = false;
-        const bool defer = may_defer(net, p);
-        if (ok != p.ahead || defer != p.deferred) drop_graph(net);
+        const bool was_ahead = p.ahead, was_deferred = p.deferred;
         p.ahead = ok;
-        p.deferred = defer;
+        const bool defer = p.deferred = may_defer(net, p);
+        if (p.ahead != was_ahead || p.deferred != was_deferred) drop_graph(net);
         if (p.model->spiking && (ok || defer) && p.spike_mask.bytes < (size_t)AHIP_AHEAD * p.nwords() * sizeof(uint64_t)) {
             HIPCHK(hipStreamSynchronize(net->stream));
             int rc = dev_alloc(p.spike_mask, (size_t)AHIP_AHEAD * p.nwords() * sizeof(uint64_t));
@@ -1131,7 +1149,7 @@ int enqueue_step(ahip_net* net, int32_t step, int32_t nsteps, const std::vector<
     hipStream_t s = net->stream;
     const size_t es = net->elem();
     // several steps at a time: input populations, compactions
-    const bool deferring = nsteps > 1 && net->probe_kind < 0;
+    const bool deferring = nsteps > 1 && net->probe_kind < 0;   // (probes run single steps)
     // 1. compute_psp: the spiking projections in fused scatter groups, then
     // the rate-coded ones
     for (size_t gi = 0; gi < net->scatter_groups.size(); gi++) {
@@ -1155,7 +1173,7 @@ int enqueue_step(ahip_net* net, int32_t step, int32_t nsteps, const std::vector<
             if (!transmits(net, p)) continue;
             if (p.syn) {
                 if (p.nnz > 0) {
-                    int rc = launch_syn(net, p, 0, step);
+                    int rc = launch_syn(net, p, 0, step, deferring);
                     if (rc) return rc;
                 }
             } else if (p.delay_per_syn && p.nnz > 0 && !p.counted) {
@@ -1257,11 +1275,11 @@ int enqueue_step(ahip_net* net, int32_t step, int32_t nsteps, const std::vector<
         Proj& p = *pp;
         if (!p.syn || p.nnz == 0 || !transmits(net, p)) continue;
         if (p.syn->has_update && p.syn_update) {
-            int rc = launch_syn(net, p, 1, step);
+            int rc = launch_syn(net, p, 1, step, deferring);
             if (rc) return rc;
         }
         if (p.spiking && p.syn->has_post) {
-            int rc = launch_syn(net, p, 2, step);
+            int rc = launch_syn(net, p, 2, step, deferring);
             if (rc) return rc;
         }
     }
@@ -2473,6 +2491,8 @@ int ahip_proj_set_synapse(ahip_net* net, int32_t proj, const char* synapse_lib) 
     p->syn_dl = dl;  // stays mapped, as the neuron model libraries
     p->syn_path = synapse_lib;
     p->syn = d;
+    const auto events = (int32_t (*)(void))dlsym(dl, "ahip_synapse_events");
+    p->syn_events = events ? events() : 0;
     p->dep_pre = dep_pre;
     p->dep_post = dep_post;
     invalidate(net);

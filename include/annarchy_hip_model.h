@@ -69,6 +69,7 @@ typedef struct ahip_record_state {
     int64_t t_start, base, period, capacity;
 } ahip_record_state;
 #define AHIP_MAX_REC 4     /* value monitors one update records */
+#define AHIP_MASK_BLOCKS 512 /* blocks of 256 neurons whose spikes kernels read from the mask, at most */
 #define AHIP_FILL_RING 32  /* > steps of one compaction launch + 1, a power of two */
 
 /* Arguments of one population update launch.  Device pointers unless noted. */

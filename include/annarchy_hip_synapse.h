@@ -87,6 +87,13 @@ typedef struct ahip_syn_args {
     int32_t plasticity;       /* 0: w is left unchanged (_plasticity) */
     int32_t update_period;    /* update every period steps ... */
     int32_t update_offset;    /* ... when (t - offset) mod period == 0 */
+    /* steps that are not compacted yet: the mask words and block counts of the
+     * spikes instead of the lists (NULL: the lists) */
+    const uint64_t* pre_mask;
+    const int32_t* pre_block_counts;
+    const uint64_t* post_mask;
+    const int32_t* post_block_counts;
+    int32_t pre_blocks, pre_words, post_blocks, post_words;
 } ahip_syn_args;
 
 typedef int (*ahip_syn_launch_fn)(const ahip_syn_args* a, void* stream);
@@ -109,6 +116,12 @@ typedef struct ahip_synapse_desc {
 } ahip_synapse_desc;
 
 const ahip_synapse_desc* ahip_synapse_describe(void);
+
+/* What the event kernels of a library take and read.  A library without this
+ * function gets lists only. */
+#define AHIP_SYN_EVENTS_MASK 1    /* pre_mask, post_mask */
+#define AHIP_SYN_EVENTS_T_PRE 2   /* pre_last_spike */
+int32_t ahip_synapse_events(void);
 
 #ifdef __cplusplus
 }

@@ -145,3 +145,57 @@ def test_a_full_monitor_keeps_its_rows(gpu):
             one[0].run(1)
         for a, b in zip(many[2], one[2]):
             assert a.get("spike", keep=True) == b.get("spike", keep=True)
+
+
+STDP_A = ah.STDP(tau_plus=20.0, tau_minus=20.0, A_plus=0.01, A_minus=0.0105, w_min=0.0, w_max=1.0)
+# reads t_pre: its input population is compacted at every step
+TIME_RULE = ah.Synapse(
+    parameters="""
+        tau_pre = 10.0 : projection
+        tau_post = 10.0 : projection
+        cApre = 0.01 : projection
+        cApost = 0.0105 : projection
+        wmax = 0.01 : projection
+    """,
+    pre_spike="""
+        g_target += w
+        w = clip(w - cApost * exp((t_post - t)/tau_post) , 0.0 , wmax)
+    """,
+    post_spike="""
+        w = clip(w + cApre * exp((t_pre - t)/tau_pre) , 0.0 , wmax)
+    """,
+    name="TimeDependent",
+)
+PoissonPostG = ah.Neuron(parameters="rates = 30.0", equations="p = Uniform(0.0, 1.0) * 1000.0 / dt\nmp = g_exc",
+                         spike="p < rates", name="PoissonPostG")
+
+
+def _plastic(synapse, n):
+    net = ah.Network(dt=1.0, seed=7)
+    pre, post = net.create(n, PoissonPre), net.create(300, PoissonPostG)
+    rng = np.random.default_rng(n)
+    k = min(5, n)
+    col = np.sort(rng.integers(0, n // k, (300, k)) + np.arange(k) * (n // k), axis=1).reshape(-1)
+    proj = net.connect(pre, post, "exc", synapse=synapse).from_csr(
+        conn.from_arrays(300, n, np.arange(301) * k, col, rng.uniform(0.001, 0.009, 300 * k)))
+    mons = [net.monitor(pre, ["spike"], capacity=sum(RUNS)), net.monitor(post, ["spike"], capacity=sum(RUNS))]
+    net.compile(graph_batch=20)
+    pre.rates, post.rates = 200.0, 100.0
+    return net, proj, mons
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("synapse", [STDP_A, TIME_RULE], ids=["stdp", "t_pre"])
+@pytest.mark.parametrize("n", [3, 300, 20011])
+def test_plastic_events_from_the_mask(gpu, synapse, n):
+    many, one = _plastic(synapse, n), _plastic(synapse, n)
+    w0 = many[1].w.copy()
+    for steps in RUNS:
+        many[0].run(steps)
+        for _ in range(steps):
+            one[0].run(1)
+        np.testing.assert_array_equal(many[1].w, one[1].w)
+        for a, b in zip(many[2], one[2]):
+            for x, y in zip(a.raw_spikes(), b.raw_spikes()):
+                np.testing.assert_array_equal(x, y)
+    assert np.any(many[1].w != w0)

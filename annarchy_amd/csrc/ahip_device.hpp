@@ -328,16 +328,19 @@ __device__ inline gptr<const V> as_global(const V* p) {
 
 // ---- spikes of a step that is not compacted yet ---------------------------
 // The spikes of a step as its update left them: a mask and the counts of its
-// blocks of 256 neurons.  The lanes of a wave hold the counts (up to
-// AHIP_MASK_BLOCKS) and their running sums; spike s is in the block whose sum passes
-// s, at the bit of its 4 words with as many bits below.  Reading the mask takes
-// the compaction out of the chain of a step (launch, mask -> barrier -> list) for
-// some 200 cycles more here (us per step with a compaction at every step / at
-// every 16th: COBA with 20003 neurons 12.7 / 10.5, with 80000 15.1 / 12.5).
+// blocks of 256 neurons.  Lane l of a wave holds the counts of blocks l, 64 + l, ...
+// (up to AHIP_MASK_BLOCKS in all) and the lanes' running sums; spike s is in the lane
+// whose sum passes s (the order of the events does not matter), in the block of that
+// lane where it falls, at the bit of its 4 words with as many bits below.  Reading
+// the mask takes the compaction out of the chain of a step (launch, mask -> barrier
+// -> list) for some 200 cycles more here (us per step with a compaction at every step
+// / at every 16th: COBA with 20003 neurons 12.7 / 10.5, with 80000 15.1 / 12.4).
+// Not beyond: with 32 counts a lane, 400000 neurons took 40.5 us a step instead of
+// 26.7.
 struct MaskSpikes {
     gptr<const uint64_t> mask;
     int32_t cnt[AHIP_MASK_BLOCKS / kWave];
-    int32_t per, sum, incl, nw, nb;
+    int32_t sum, incl, nw, nb;
     int32_t at, rank;   // block of the next spike, its rank there
     uint64_t word;      // lane l: word l & 3 of the block
     __device__ inline int32_t load(const uint64_t* words, const int32_t* counts, int32_t n_blocks, int32_t n_words,
@@ -345,12 +348,11 @@ struct MaskSpikes {
         mask = as_global(words);
         nb = n_blocks;
         nw = n_words;
-        per = (nb + kWave - 1) / kWave;
         const auto bc = as_global(counts);
 #pragma unroll
         for (int q = 0; q < AHIP_MASK_BLOCKS / kWave; q++) {
-            const int32_t b = lane * per + q;
-            cnt[q] = q < per && b < nb ? bc[b] : 0;
+            const int32_t b = q * kWave + lane;
+            cnt[q] = b < nb ? bc[b] : 0;
         }
         sum = 0;
 #pragma unroll
@@ -380,7 +382,7 @@ struct MaskSpikes {
                 q++;
             }
         }
-        at = l * per + q;
+        at = q * kWave + l;
         rank = r;
         const int32_t w = at * (AHIP_UPDATE_BLOCK / kWave) + (lane & (AHIP_UPDATE_BLOCK / kWave - 1));
         word = w < nw ? mask[w] : 0ull;

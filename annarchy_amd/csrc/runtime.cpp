@@ -830,7 +830,8 @@ constexpr int64_t kFuseMaxGathered = 1 << 24, kFuseMaxStaged = 1 << 27;
 // plastic projection (which read the mask), none a delay queue, the firing-rate
 // window, a second spike monitor, the ring kernel of delays per synapse, or t_pre
 // of a population that runs ahead (its last spikes are kept by the compactions).
-// Up to AHIP_MASK_BLOCKS blocks, 131072 neurons.
+// Up to AHIP_MASK_BLOCKS blocks, 131072 neurons (13.7 us a step there, 16.9 with one
+// neuron more and a list; ahip::MaskSpikes has the figure above it).
 static bool may_defer(const ahip_net* net, const Pop& p) {
     if (!p.model->spiking || !p.active || p.depth > 1 || p.fr_window > 0 || p.nblocks() > AHIP_MASK_BLOCKS) return false;
     for (auto& qq : net->projs) {

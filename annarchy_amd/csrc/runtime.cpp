@@ -1206,6 +1206,7 @@ int enqueue_step(ahip_net* net, int32_t step, int32_t nsteps, const std::vector<
         Monitor& m = *mp;
         if (!m.after_psp || m.paused || m.in_update) continue;
         Pop& p = *net->pops[m.pop];
+        if (p.fused) continue;   // its sums are there after its update: recorded below
         LCHK(launch_record_values(m, p.slots[m.slot].p, p.size, (int32_t)es,
                                   net->t_dev.as<int64_t>(), step, s));
     }
@@ -1287,8 +1288,9 @@ int enqueue_step(ahip_net* net, int32_t step, int32_t nsteps, const std::vector<
     // 5. record variables and spikes
     for (auto& mp : net->mons) {
         Monitor& m = *mp;
-        if (m.after_psp || m.paused || m.in_update) continue;
+        if (m.paused || m.in_update) continue;
         Pop& p = *net->pops[m.pop];
+        if (m.after_psp && !p.fused) continue;
         if (m.spikes) {
             // an inactive population keeps its last spike list, which its
             // monitors record again (its compaction does not run)

@@ -8,6 +8,8 @@ most four of a population), a launch of its own, or the spike compaction.
 
 * a rate population whose update sums its own rows, its sum and r recorded,
   r every third step as well, against the trajectory computed on the host;
+* the sum in a monitor of its own, the fifth of such a population, which the
+  update does not record: at every step and at every second one;
 * an `Every5` population with six monitors (five values, spikes), g_exc recorded
   after the events of a one-to-one projection arrive and before the neuron's own
   step.
@@ -49,6 +51,31 @@ def test_rate_records_follow_the_clock(gpu, n):
         np.testing.assert_allclose(each.get("_sum_exc"), r, rtol=0, atol=1e-14)
         rows = [u - t for u in range(t, t + steps) if u % 3 == 1]
         np.testing.assert_allclose(third.get("r"), r[rows], rtol=0, atol=1e-14)
+        t += steps
+
+
+@pytest.mark.parametrize("period", [1.0, 2.0])
+def test_a_fifth_monitor_records_the_sum_of_its_step(gpu, period):
+    n = 130
+    W = np.random.default_rng(3).normal(0.0, 1.0, (n, 3))
+    csr = conn.from_arrays(n, 3, np.arange(n + 1) * 3, np.tile(np.arange(3), n), W.reshape(-1))
+    net = ah.Network(dt=1.0, seed=1)
+    inp, pop = net.create(3, SinRate), net.create(n, SumRate)
+    net.connect(inp, pop, "exc").from_csr(csr, storage_format="csr")
+    r = [net.monitor(pop, ["r"], capacity=40) for _ in range(4)]
+    total = net.monitor(pop, ["_sum_exc"], capacity=40, period=period)
+    net.compile(graph_batch=20)
+    phase = np.array([0.0, 1.0, 2.0])
+    inp.phase = phase
+    t = 0
+    for steps in (30, 30, 30, 1):
+        net.run(steps)
+        x = [0.5 + 0.5 * np.sin(0.1 * (u - 1) + phase) if u > 0 else np.zeros(3) for u in range(t, t + steps)]
+        s = np.array([W @ v for v in x])   # r = sum(exc)
+        for m in r:
+            np.testing.assert_allclose(m.get("r"), s, rtol=0, atol=1e-14)
+        np.testing.assert_allclose(total.get("_sum_exc"), s[[u % int(period) == 0 for u in range(t, t + steps)]],
+                                   rtol=0, atol=1e-14)
         t += steps
 
 

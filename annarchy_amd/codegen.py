@@ -245,13 +245,19 @@ __device__ inline void persist_range(const ahip_persist_proj& P, const int32_t* 
     }
 }
 
+// Rows of the spike monitor filled before step t; a full one stays at its
+// capacity, the entry that the host reads then.
+__device__ inline int64_t persist_rec_row(const ahip_persist_args& pa, int64_t t) {
+    return min(max((int64_t)0, t - pa.rec_state->t_start), pa.rec_state->capacity);
+}
+
 template <typename T>
 __global__ __launch_bounds__(AHIP_PERSIST_THREADS) void persistent_steps(ahip_pop_args a_in, ahip_persist_args pa) {
     extern __shared__ unsigned char lds_raw[];
     __shared__ int32_t wsum[kPersistWaves];
     __shared__ uint32_t wlo[kPersistWaves], whi[kPersistWaves];
     __shared__ int64_t fill_s[2];
-    __shared__ int32_t nspk_s;
+    __shared__ int32_t nspk_s, rec_end_s;   // rec_end_s: the entry of the row after the launch
     __shared__ ahip_persist_proj proj_s[AHIP_PERSIST_MAX_PROJ];   // read per lane: LDS, not kernel arguments
     const int32_t N = a_in.size;
     const int tid = threadIdx.x;
@@ -278,8 +284,9 @@ __global__ __launch_bounds__(AHIP_PERSIST_THREADS) void persistent_steps(ahip_po
     if (tid == 0) {
         nspk_s = *pa.spike_count;
         if (pa.rec_counts) {
-            const int64_t row = max((int64_t)0, *a.t_base + a.step - pa.rec_state->t_start);
+            const int64_t row = persist_rec_row(pa, *a.t_base + a.step);
             fill_s[0] = fill_s[1] = pa.rec_fill[row & (AHIP_FILL_RING - 1)];
+            rec_end_s = (int32_t)(persist_rec_row(pa, *a.t_base + a.step + pa.steps) & (AHIP_FILL_RING - 1));
         }
     }
     persist_sync();
@@ -464,8 +471,8 @@ __global__ __launch_bounds__(AHIP_PERSIST_THREADS) void persistent_steps(ahip_po
     }
     if (tid == 0) {
         *pa.spike_count = nspk;
-        if (pa.rec_counts)   // (the next row's entry is all that is read)
-            for (int r = 0; r < AHIP_FILL_RING; r++) pa.rec_fill[r] = fill_s[r & 1];
+        // (the next row's entry is all that is read)
+        if (pa.rec_counts) pa.rec_fill[rec_end_s] = fill_s[rec_end_s & 1];
     }
 }
 

@@ -15,7 +15,9 @@ neuron update, ascending spike list, spike recording).
   strongly driven network) and column ranges read from global memory when
   they do not fit in LDS (4500 neurons);
 * a spike monitor paused and resumed, and a network the path does not take
-  (a Poisson input population) -- uses_persistent() says which.
+  (a Poisson input population) -- uses_persistent() says which;
+* a spike monitor that fills inside a launch, and launches after it that start
+  at an odd and at an even step: its rows stay as they are.
 """
 
 import numpy as np
@@ -26,6 +28,8 @@ from annarchy_amd import models
 from oracle import oracle as orc
 
 pytestmark = pytest.mark.gpu
+
+Every5 = ah.Neuron(equations="v = v + 1.0\nmp = t\nq = g_exc", spike="v == 5.0", reset="v = 0.0", name="Every5")
 
 
 def _coba(n=4000, ne=3200, seed=7, precision="double", extra=False, persistent=True, graph_batch=200, I=20.0):
@@ -153,3 +157,26 @@ def test_persistent_probe_continues_the_run(gpu):
     net2.compile()
     with pytest.raises(Exception, match="persistent"):
         net2.time_kernel(7, 0, 1)
+
+
+@pytest.mark.parametrize("capacity", [1, 24, 25, 40])
+def test_a_full_monitor_keeps_its_last_row(gpu, capacity):
+    n = 300
+    nets = []
+    for persistent in (True, False):
+        net = ah.Network(dt=1.0, seed=1)
+        P = net.create(n, Every5)
+        net.connect(P, P, "exc").one_to_one(0.5)
+        mon = net.monitor(P, ["spike"], capacity=capacity)
+        net.compile(graph_batch=20)
+        net.set_persistent(persistent)
+        assert net.uses_persistent() is persistent
+        P.v = np.arange(n) % 5.0
+        nets.append((net, mon))
+    for steps in (20, 20, 20, 1, 20, 7, 20):
+        (a, ma), (b, mb) = nets
+        a.run(steps)
+        b.run(steps)
+        (ca, ia), (cb, ib) = ma.raw_spikes(), mb.raw_spikes()
+        assert np.array_equal(ca, cb) and np.array_equal(ia, ib)
+        assert ca.size == min(capacity, a.time) and ia.size == ca.sum() == ca.size * n // 5

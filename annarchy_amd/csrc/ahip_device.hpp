@@ -205,6 +205,9 @@ __device__ inline int64_t mod_pos(int64_t u, int64_t n) {
     return u < 0 ? n - 1 - (int64_t)r : (int64_t)r;
 }
 
+// slot of step u in a ring of D steps
+__device__ inline int64_t ring_slot(int64_t u, int32_t D) { return (D & (D - 1)) == 0 ? u & (D - 1) : mod_pos(u, D); }
+
 __device__ inline int64_t sim_time(const ahip_pop_args& a) { return *a.t_base + a.step; }
 
 // Row of a monitor at step t, -1: not recorded.
@@ -533,6 +536,7 @@ __device__ inline void deliver_buckets(const ahip_pop_args& a, int32_t i) {
 template <typename T>
 struct Counted {
     int32_t n[AHIP_MAX_COUNTED];
+    int32_t slot[AHIP_MAX_COUNTED];   // of the ring, uniform
     T sum[AHIP_MAX_COUNTED];
 };
 template <typename T>
@@ -540,11 +544,12 @@ __device__ inline Counted<T> load_counted(const ahip_pop_args& a, int64_t t, int
     Counted<T> c;
 #pragma unroll
     for (int k = 0; k < AHIP_MAX_COUNTED; k++) {
-        c.n[k] = 0;
+        c.n[k] = c.slot[k] = 0;
         c.sum[k] = T(0);
         if (k >= a.n_counted || i >= a.size) continue;
         const ahip_counted_desc& d = a.counted[k];
-        const int64_t at = (t & (d.depth - 1)) * a.size + i;
+        c.slot[k] = (int32_t)ring_slot(t, d.depth);
+        const int64_t at = (int64_t)c.slot[k] * a.size + i;
         if (d.sums) c.sum[k] = static_cast<const T*>(d.ring)[at];
         else c.n[k] = static_cast<const int32_t*>(d.ring)[at];
     }
@@ -559,7 +564,7 @@ __device__ inline T add_counted(const ahip_pop_args& a, const Counted<T>& c, int
         if (k >= a.n_counted || a.counted[k].slot != slot) continue;
         const ahip_counted_desc& d = a.counted[k];
         if (c.n[k] == 0 && c.sum[k] == T(0)) continue;
-        const int64_t at = (t & (d.depth - 1)) * a.size + i;
+        const int64_t at = (int64_t)c.slot[k] * a.size + i;
         if (d.sums) {
             g += c.sum[k];
             static_cast<T*>(d.ring)[at] = T(0);

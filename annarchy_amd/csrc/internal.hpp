@@ -133,13 +133,7 @@ struct Proj {
     int32_t max_delay = 1;
     std::vector<int32_t> h_delay; // per synapse, forward order (delay_per_syn)
     DevBuf delay_dev;             // int16: rate -> forward order, spiking -> column order
-    DevBuf ring;                  // spiking per-synapse delays: ring_depth() x n_rows events
-    // slots of the ring: max_delay rounded up to a power of two
-    int32_t ring_depth() const {
-        int32_t d = 1;
-        while (d < max_delay) d *= 2;
-        return d;
-    }
+    DevBuf ring;                  // spiking per-synapse delays: max_delay x n_rows events
     bool counted = false;         // spiking: the scatter counts the events, the post update adds them
     DevBuf cnt;                   // counted without a delay per synapse: int32[n_rows], 0 between steps
     DevBuf xd;                    // rate uniform delay: the delayed pre-synaptic rates
@@ -220,8 +214,7 @@ struct ScatterDesc {
     uint32_t gid_off;
     // counted delivery (ring != NULL): the event of column-order synapse j adds 1
     // (w_col: its weight) at ring slot (t - 1 + delay_col[j]) mod ring_depth of
-    // its post neuron (ring_depth a power of two); the post update adds what has
-    // arrived
+    // its post neuron; the post update adds what has arrived
     void* ring;
     const int16_t* delay_col;
     int32_t ring_depth, n_post;

@@ -260,7 +260,7 @@ int launch_spike_ring(const ahip_net* net, const Proj& p, const Pop& pre, void* 
     if (nb > 512) nb = 512;
     if (nb < 1) nb = 1;
     const unsigned nbd = blocks_for(p.n_rows);
-    const int32_t D = p.ring_depth();
+    const int32_t D = p.max_delay;
     if (net->precision == AHIP_F64) {
         if (p.single_w) {
             hipLaunchKernelGGL((ring_scatter<double, true>), dim3(nb), dim3(kBlock), 0, s, pre.spiked.as<int32_t>(),

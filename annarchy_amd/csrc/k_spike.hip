@@ -279,6 +279,8 @@ __global__ __launch_bounds__(256) void scatter_multi(const ScatterArgs A, const 
         next = s < d.n_cols ? list[s] : -1;
         n = as_global(d.count)[sl];
     }
+    // ring slot of the step whose spikes these are
+    const int32_t now = d.delay_col ? (int32_t)ring_slot(*t_base + step - 1, d.ring_depth) : 0;
     while (s < n) {
         const int32_t pre = masked ? M.neuron(lane) : next, c = c_next;
         W.step(s, c_next);
@@ -296,7 +298,6 @@ __global__ __launch_bounds__(256) void scatter_multi(const ScatterArgs A, const 
         if (d.ring) {
             // counted delivery: equal addends (or, with a weight and a delay per
             // synapse, sums) wait in the slot of the step they arrive at
-            const int32_t now = d.delay_col ? (int32_t)(*t_base + step) - 1 : 0;
             const auto dl = as_global(d.delay_col);
             for (int64_t base = b + (int64_t)c * 256; base < e; base += (int64_t)d.chunks * 256) {
                 int32_t at[4];
@@ -307,7 +308,11 @@ __global__ __launch_bounds__(256) void scatter_multi(const ScatterArgs A, const 
                     at[u] = -1;
                     v[u] = T(0);
                     if (j >= e) continue;
-                    const int32_t slot = d.delay_col ? (now + dl[j]) & (d.ring_depth - 1) : 0;
+                    int32_t slot = 0;
+                    if (d.delay_col) {
+                        slot = now + dl[j];   // (a delay is at most ring_depth)
+                        slot -= slot >= d.ring_depth ? d.ring_depth : 0;
+                    }
                     at[u] = slot * d.n_post + ri[j];
                     if (wc) v[u] = wg[j];
                 }

@@ -43,9 +43,6 @@ struct Acc<float> {
 __device__ inline void wave_join(Acc<double>& a) { a.s = group_sum<kWave>(a.s); }
 __device__ inline void wave_join(Acc<float>& a) { group_join_kahan(a.k.s, a.k.c, log2_of(kWave)); }
 
-// slot of step u in a ring of D steps
-__device__ inline int64_t ring_slot(int64_t u, int32_t D) { return (D & (D - 1)) == 0 ? u & (D - 1) : mod_pos(u, D); }
-
 typedef double v2d_t __attribute__((ext_vector_type(2)));
 typedef float v4f_t __attribute__((ext_vector_type(4)));
 

@@ -204,7 +204,7 @@ int ensure_delay_buffers(ahip_net* net) {
             // pending events of steps [t, t + old depth) keep their delivery step
             const size_t slot = (size_t)p.n_rows * (p.single_w ? sizeof(int32_t) : es);
             const int32_t d_old = p.ring.p ? (int32_t)(p.ring.bytes / std::max<size_t>(slot, 1)) : 0;
-            const int32_t d_new = std::max(p.ring_depth(), d_old);
+            const int32_t d_new = std::max(p.max_delay, d_old);
             if (!p.ring.p || d_old < d_new) {
                 HIPCHK(hipStreamSynchronize(net->stream));
                 int rc = regrow_ring(p.ring, slot, d_old, d_new, net->t, net->t + d_old);
@@ -601,7 +601,7 @@ static int assign_counted(ahip_net* net) {
         std::vector<Proj*> pick;
         for (Proj* p : in) {
             bool ok = !p->syn && (p->single_w || p->delay_per_syn) &&
-                      (int64_t)p->ring_depth() * p->n_rows < INT32_MAX;
+                      (int64_t)p->max_delay * p->n_rows < INT32_MAX;
             for (const Proj* q : in) {
                 if (q->target_slot != p->target_slot) continue;
                 // plastic events add to the conductance themselves; ordered
@@ -721,7 +721,7 @@ int prepare(ahip_net* net) {
             d.pre = p.pre;
             d.ring = !p.counted ? nullptr : p.delay_per_syn ? p.ring.p : p.cnt.p;
             d.delay_col = p.delay_per_syn ? p.delay_dev.as<int16_t>() : nullptr;
-            d.ring_depth = p.delay_per_syn ? p.ring_depth() : 1;
+            d.ring_depth = p.delay_per_syn ? p.max_delay : 1;
             d.n_post = p.n_rows;
             for (OrderedTarget& o : net->ordered) {
                 if (o.g != g || p.counted) continue;
@@ -1127,7 +1127,7 @@ ahip_pop_args make_args(ahip_net* net, Pop& p, int32_t step) {
             d.ring = q.delay_per_syn ? q.ring.p : q.cnt.p;
             d.w = q.w_const;
             d.slot = q.target_slot;
-            d.depth = q.delay_per_syn ? q.ring_depth() : 1;
+            d.depth = q.delay_per_syn ? q.max_delay : 1;
             d.sums = q.delay_per_syn && !q.single_w ? 1 : 0;
         }
     for (auto& mp : net->mons) {

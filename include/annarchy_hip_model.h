@@ -22,7 +22,7 @@
 extern "C" {
 #endif
 
-#define AHIP_MODEL_ABI 15
+#define AHIP_MODEL_ABI 16
 #define AHIP_MAX_SLOTS 48
 #define AHIP_MAX_RAND 8
 #define AHIP_UPDATE_BLOCK 256 /* threads per block of every update kernel */
@@ -49,8 +49,7 @@ typedef struct ahip_deliver_desc {
 #define AHIP_MAX_PSUM 2    /* psp sums one update completes from panel partials */
 
 /* Spike events counted per post neuron: the scatter adds 1 (or, `sums`, the
- * synapse's weight) at ring slot (arrival step) mod depth, a power of two, the
- * update adds
+ * synapse's weight) at ring slot (arrival step) mod depth, the update adds
  * them to the conductance in slot `slot` before its statements, projection by
  * projection, one addition of the weight per event, and clears them.  All
  * addends of a projection are equal, so the result does not depend on the

@@ -9,8 +9,13 @@ The sums of the last projection arrive by atomics, in no fixed order: its
 conductance agrees to the rounding of its additions (in-degree 9 at most, values
 below 10: 1e-13).  With a fifth projection into the population, more than one
 update delivers, everything goes the other way (scatters and delivery launches)
-and has to give the same bits.  Delays up to 5 make a ring of 8 slots, 1 and 2
-its smallest."""
+and has to give the same bits.  Delays up to 5 make a ring of 5 slots,
+up to 2 the smallest one.
+
+Events that wait while their projection does not transmit, or while the clock is
+set back, stay in their slot of the ring of max_delay steps: they arrive at the
+next step that transmits and has the slot.  A host ring gives the same conductances, for counts
+and for sums, by the post update and by the kernels of their own."""
 
 import numpy as np
 import pytest
@@ -92,3 +97,46 @@ def test_counted_events(gpu, n, max_delay, extra):
         np.testing.assert_array_equal(exc[t], g)
         np.testing.assert_allclose(inh[t], h, rtol=0, atol=1e-13)
         g, h = g + step * -g, h + step * -h
+
+
+Emit = ah.Neuron(spike="t==1", name="Emit")
+Recv = ah.Neuron(equations="g_exc = 0", spike="g_exc>30", name="Recv")
+
+
+@pytest.mark.parametrize("max_delay", [3, 5, 8])
+@pytest.mark.parametrize("pause", [0, 1, 2, 5])
+@pytest.mark.parametrize("single_w", [True, False])
+@pytest.mark.parametrize("counted", [True, False])
+def test_events_wait_in_their_slot(gpu, max_delay, pause, single_w, counted):
+    n = max_delay
+    delay = np.arange(1, n + 1)
+    w = np.full(n, 0.5) if single_w else 0.25 * np.arange(1, n + 1)
+    net = ah.Network(dt=1.0, seed=1)
+    pre, pop = net.create(n, Emit), net.create(n, Recv)
+    csr = conn.from_arrays(n, n, np.arange(n + 1), np.arange(n), None if single_w else w, 0.5)
+    proj = net.connect(pre, pop, "exc").from_csr(csr, delays=delay.astype(float))
+    for _ in range(0 if counted else 4):   # more than one update delivers
+        net.connect(pre, pop, "exc").from_csr(conn.from_arrays(n, n, np.arange(n + 1), np.arange(n), None, 0.0),
+                                              delays=delay.astype(float))
+    mon = net.monitor(pop, ["g_exc"], capacity=100)
+    net.compile(graph_batch=4)
+    ring, emitted, t = np.zeros((max_delay, n)), False, 0
+    for steps, transmits, back in ((3, True, False), (pause, False, False), (5, True, True), (4, True, False),
+                                   (2 * max_delay, True, False)):
+        proj.transmission = transmits
+        net.run(steps)
+        g = np.zeros((steps, n))
+        for k in range(steps):
+            if transmits:
+                if emitted:   # the spikes of the step before
+                    ring[(t - 1 + delay) % max_delay, np.arange(n)] += w
+                g[k] = ring[t % max_delay]
+                ring[t % max_delay] = 0.0
+            emitted = t == 1
+            t += 1
+        if steps:
+            np.testing.assert_array_equal(mon.get("g_exc"), g)
+        if back:
+            net.reset(populations=False)
+            t = 0
+    assert not ring.any()

@@ -66,6 +66,7 @@ struct Pop {
     // rate-coded: the psp variable, depth x size; spiking: spike lists,
     // depth x size int32 with counts int32[depth]
     int32_t depth = 1;
+    int32_t queue = 1;            // steps of it that are the queue's: the largest delay so far
     DevBuf hist, hist_count;
     // rate-coded: r at the end of the last steps (rbuf_depth slots: 2, of an
     // ahead population 2 AHIP_AHEAD), kept by the population's update while a
@@ -345,6 +346,9 @@ int launch_push_values(const ahip_net* net, const void* src, void* hist, int32_t
 int launch_gather_delayed(const ahip_net* net, const void* hist, void* dst, int32_t n, int32_t D, int32_t d,
                           int32_t step, hipStream_t s);
 int launch_fill_hist(const ahip_net* net, const void* src, void* hist, int32_t n, int32_t D, hipStream_t s);
+// the queue of `queue` steps in a ring of D slots, when the clock goes from t to u
+int launch_reslot(const ahip_net* net, const void* src, void* dst, int32_t n, int32_t D, int32_t queue, int64_t t,
+                  int64_t u, hipStream_t s);
 int launch_push_spikes(const ahip_net* net, const Pop& p, int32_t step, hipStream_t s);
 int launch_rate_psp_delayed(const ahip_net* net, const Proj& p, const Pop& pre, void* target, int32_t step,
                             hipStream_t s);

@@ -55,6 +55,20 @@ __global__ __launch_bounds__(kBlock) void fill_hist(const T* __restrict__ src, T
     hist[i] = src[i % n];
 }
 
+// A queue of `queue` steps whose ring has more slots (D), when the clock is set
+// from t to u: read from u on it holds what a ring of `queue` slots would, so the
+// spare slots do not show.  (That ring's slot of step u - d is the one of the
+// last step before t that is congruent to it.)
+template <typename T>
+__global__ __launch_bounds__(kBlock) void reslot(const T* __restrict__ src, T* __restrict__ dst, int32_t n, int32_t D,
+                                                 int32_t queue, int64_t t, int64_t u) {
+    const int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (k >= (int64_t)n * queue) return;
+    const int64_t to = u - 1 - k / n;
+    const int64_t from = t - 1 - ring_slot(t - 1 - to, queue);
+    dst[ring_slot(to, D) * n + k % n] = src[ring_slot(from, D) * n + k % n];
+}
+
 // spike-list ring: slot (t mod D) = the step's list and count
 __global__ __launch_bounds__(kBlock) void push_spikes(const int32_t* __restrict__ spiked,
                                                       const int32_t* __restrict__ count,
@@ -197,6 +211,19 @@ int launch_fill_hist(const ahip_net* net, const void* src, void* hist, int32_t n
     else
         hipLaunchKernelGGL(fill_hist<float>, dim3(blocks_for((int64_t)n * D)), dim3(kBlock), 0, s,
                            (const float*)src, (float*)hist, n, D);
+    return (int)hipGetLastError();
+}
+
+int launch_reslot(const ahip_net* net, const void* src, void* dst, int32_t n, int32_t D, int32_t queue, int64_t t,
+                  int64_t u, hipStream_t s) {
+    const unsigned nb = blocks_for((int64_t)n * queue);
+    if (nb == 0) return 0;
+    if (net->precision == AHIP_F64)
+        hipLaunchKernelGGL(reslot<double>, dim3(nb), dim3(kBlock), 0, s, (const double*)src, (double*)dst, n, D, queue,
+                           t, u);
+    else
+        hipLaunchKernelGGL(reslot<float>, dim3(nb), dim3(kBlock), 0, s, (const float*)src, (float*)dst, n, D, queue, t,
+                           u);
     return (int)hipGetLastError();
 }
 

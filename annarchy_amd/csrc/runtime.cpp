@@ -177,20 +177,23 @@ int ensure_delay_buffers(ahip_net* net) {
         // while another workgroup of its launch reads step t - max_delay's
         // (AHIP_AHEAD slots more where the population's updates may run that
         // many steps ahead of the readers)
-        const int32_t want = need[p.id] > 1 && !p.model->spiking
-                                 ? need[p.id] + (may_run_ahead(net, p) ? AHIP_AHEAD : 1) : need[p.id];
+        const int32_t queue = std::max(need[p.id], p.queue);
+        const int32_t want = queue > 1 && !p.model->spiking ? queue + (may_run_ahead(net, p) ? AHIP_AHEAD : 1) : queue;
         const int32_t D = std::max(want, p.depth);
-        if (D == p.depth && (D == 1 || p.hist.p)) continue;
+        if (D == p.depth && queue == p.queue && (D == 1 || p.hist.p)) continue;
         HIPCHK(hipStreamSynchronize(net->stream));
-        const int32_t d_old = p.hist.p ? p.depth : 0;
+        // (the slots beyond the queue hold older steps, which a longer delay
+        // does not see)
+        const int32_t d_old = p.hist.p ? p.depth : 0, kept = p.hist.p ? p.queue : 0;
         int rc;
         if (p.model->spiking) {
-            if ((rc = regrow_ring(p.hist, (size_t)p.size * sizeof(int32_t), d_old, D, net->t - d_old, net->t))) return rc;
-            if ((rc = regrow_ring(p.hist_count, sizeof(int32_t), d_old, D, net->t - d_old, net->t))) return rc;
+            if ((rc = regrow_ring(p.hist, (size_t)p.size * sizeof(int32_t), d_old, D, net->t - kept, net->t))) return rc;
+            if ((rc = regrow_ring(p.hist_count, sizeof(int32_t), d_old, D, net->t - kept, net->t))) return rc;
         } else {
-            if ((rc = regrow_ring(p.hist, (size_t)p.size * es, d_old, D, net->t - d_old, net->t))) return rc;
+            if ((rc = regrow_ring(p.hist, (size_t)p.size * es, d_old, D, net->t - kept, net->t))) return rc;
         }
         p.depth = D;
+        p.queue = queue;
         invalidate(net);
     }
     for (auto& pp : net->projs) {
@@ -1657,6 +1660,17 @@ int ahip_get_time(ahip_net* net, int64_t* t) {
 int ahip_set_time(ahip_net* net, int64_t t) {
     if (!net || !net->initialized) return fail(AHIP_ESTATE, "network not initialized");
     HIPCHK(hipStreamSynchronize(net->stream));
+    HIPCHK(hipSetDevice(net->device));
+    for (auto& pp : net->pops) {
+        Pop& p = *pp;
+        if (!p.hist.p || p.depth == p.queue || t == net->t) continue;
+        DevBuf tmp;
+        int rc = dev_alloc(tmp, p.hist.bytes);
+        if (rc) return rc;
+        LCHK(launch_reslot(net, p.hist.p, tmp.p, p.size, p.depth, p.queue, net->t, t, net->stream));
+        HIPCHK(hipMemcpyAsync(p.hist.p, tmp.p, p.hist.bytes, hipMemcpyDeviceToDevice, net->stream));
+        HIPCHK(hipStreamSynchronize(net->stream));
+    }
     HIPCHK(hipMemcpy(net->t_dev.p, &t, sizeof(int64_t), hipMemcpyHostToDevice));
     net->t = t;
     net->rbuf_stale = true;

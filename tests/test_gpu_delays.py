@@ -10,6 +10,12 @@ Known answers of the reference tests, run through the same Python calls:
 Random networks against the oracle's delay queues (orc_rate_run_delayed,
 orc_spiking_run with uniform and per-synapse delays): rates to 1e-9, spike
 lists bit for bit, also through captured graphs.
+
+A queue is as long as the largest delay so far, whatever the ring behind it
+holds: a longer delay given later reads zeros beyond it, and a clock set back
+(reset without the populations) reads it as a ring of that many slots.  A host
+ring gives the same rates, for an input whose steps run ahead and for one that
+keeps state.
 """
 
 import numpy as np
@@ -162,3 +168,46 @@ def test_coba_delays_bit_exact_vs_oracle(gpu, case):
     np.testing.assert_array_equal(counts, ref["counts"])
     np.testing.assert_array_equal(idx, ref["idx"])
     assert np.array_equal(P.v.reshape(-1), ref["v"])
+
+
+RateT = ah.Neuron(equations="r = t", name="RateT")
+
+
+@pytest.mark.parametrize("source", ["ahead", "state"])
+@pytest.mark.parametrize("per_synapse, fmt", [(False, "csr"), (False, "ellr"), (True, "csr")])
+@pytest.mark.parametrize("first", [7, 10, 40])
+def test_the_queue_is_as_long_as_its_largest_delay(gpu, source, per_synapse, fmt, first):
+    n = 3
+    net = ah.Network(dt=1.0, seed=1)
+    inp = net.create(n, RateT if source == "ahead" else DelayIn)
+    out = net.create(n, DelayOut)
+    csr = conn.from_arrays(n, n, np.arange(n + 1), np.arange(n), np.full(n, 0.5))
+    delay = np.array([2, 5, 3]) if per_synapse else np.full(n, 5)
+    give = lambda: delay.astype(float) if per_synapse else float(delay[0])
+    proj = net.connect(inp, out, "ff").from_csr(csr, storage_format=fmt, delays=give())
+    mon = net.monitor(out, ["r"], capacity=100)
+    net.compile(graph_batch=20)
+    r, ring, t = 0.0 if source == "ahead" else -1.0, np.zeros(5), 0
+
+    def run(steps):
+        nonlocal r, t
+        net.run(steps)
+        ref = np.zeros((steps, n))
+        for k in range(steps):
+            ref[k] = 0.5 * ring[(t - delay) % ring.size]
+            r = float(t) if source == "ahead" else r + t
+            ring[t % ring.size] = r
+            t += 1
+        np.testing.assert_array_equal(mon.get("r"), ref)
+
+    run(first)
+    longer = np.zeros(8)
+    for u in range(t - 5, t):
+        longer[u % 8] = ring[u % 5]
+    ring = longer
+    delay = np.array([8, 5, 2]) if per_synapse else np.full(n, 8)
+    proj.delay = give()
+    run(21)
+    net.reset(populations=False)
+    t = 0
+    run(25)

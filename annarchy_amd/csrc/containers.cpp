@@ -457,6 +457,8 @@ int build_layout(const Proj& p, int32_t precision, const ahip_format_opts& o, Ra
             L.sigma = waves;
             L.panel_cols = pc;
             L.chunk = rb_rows;
+            L.asked_chunk = o.chunk;
+            L.asked_panel_cols = o.panel_cols;
             L.n_units = np;
             L.width = nrb;
             L.stored = total;

@@ -38,6 +38,9 @@ struct RateLayout {
     int32_t chunk = 64;       // SELL rows per slice / BSR tile
     int32_t sigma = 1;
     int32_t panel_cols = 0;
+    // SELL_PANEL: the tile height and panel width asked for (0: automatic; the
+    // ones above are those built): what the layout is rebuilt from
+    int32_t asked_chunk = 0, asked_panel_cols = 0;
     int64_t stored = 0;       // stored entries including padding
     int32_t width = 0;        // ELL max row length / DENSE values per stored row
     int32_t n_units = 0;      // SELL slices / BSR block rows / panels

@@ -2235,6 +2235,16 @@ int ahip_proj_get_csr(ahip_net* net, int32_t proj, int64_t* row_ptr, int32_t* co
     return 0;
 }
 
+// The options that give the layout L again.
+static ahip_format_opts rebuild_opts(const RateLayout& L) {
+    ahip_format_opts o{L.format, L.lanes, L.chunk, L.sigma, L.panel_cols};
+    if (L.format == AHIP_FMT_SELL_PANEL) {
+        o.chunk = L.asked_chunk;
+        o.panel_cols = L.asked_panel_cols;
+    }
+    return o;
+}
+
 int ahip_proj_set_format(ahip_net* net, int32_t proj, const ahip_format_opts* opts) {
     Proj* p = get_proj(net, proj);
     if (!p || !opts || p->nnz < 0) return fail(AHIP_EINVAL, "bad projection");
@@ -2252,7 +2262,12 @@ int ahip_proj_set_format(ahip_net* net, int32_t proj, const ahip_format_opts* op
     }
     std::string err;
     RateLayout L;
-    int rc = build_layout(*p, net->precision, *opts, L, err);
+    ahip_format_opts o = *opts;
+    // the format the projection reports is the one it has
+    if (o.format == AHIP_FMT_SELL_PANEL && p->rate.format == o.format && o.chunk == p->rate.chunk &&
+        o.panel_cols == p->rate.panel_cols && o.lanes_per_row == p->rate.lanes && o.sigma == p->rate.sigma)
+        o = rebuild_opts(p->rate);
+    int rc = build_layout(*p, net->precision, o, L, err);
     if (rc) return fail(rc, "%s", err.c_str());
     p->rate = std::move(L);
     return 0;
@@ -2457,7 +2472,7 @@ int ahip_proj_set_w(ahip_net* net, int32_t proj, const double* w, int64_t nnz) {
     invalidate(net);
     if (p->syn) return syn_field_io(net, *p, -1, const_cast<double*>(w), nullptr, true);
     if (p->spiking) return build_backward(net, *p);
-    ahip_format_opts o{p->rate.format, p->rate.lanes, p->rate.chunk, p->rate.sigma, p->rate.panel_cols};
+    const ahip_format_opts o = rebuild_opts(p->rate);
     std::string err;
     RateLayout L;
     int rc = build_layout(*p, net->precision, o, L, err);

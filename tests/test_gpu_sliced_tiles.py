@@ -3,7 +3,10 @@ CUs (narrower panels, rows shared by several lanes), fewer than the CUs (lower
 tiles), at least as many (as asked).  One psp of ragged rows with empty and
 very long ones against the dense product in float64; FP64 to the summation
 bound K u sum|w r| (K <= 2000 terms: 1e-12 of the largest sum), FP32 rows are
-compensated: 2e-6, the bar of every psp format."""
+compensated: 2e-6, the bar of every psp format.
+
+Weights written back, or the reported format set again, leave the layout and so
+every bit of the psp as they were."""
 
 import numpy as np
 import pytest
@@ -39,3 +42,43 @@ def test_tile_heights(gpu, n, opts, precision, tol):
     np.testing.assert_allclose(np.asarray(pop.sum("exc")).reshape(-1), ref, rtol=0,
                                atol=tol * max(1.0, np.max(np.abs(ref))))
     assert proj.get_format()["panel_cols"] <= opts["panel_cols"]
+
+
+def _one_psp(n, precision, opts):
+    rng = np.random.default_rng(n)
+    deg = np.minimum(n, rng.integers(0, 120, n))
+    deg[::5] = 0
+    deg[:: max(1, n // 7)] = min(n, 2000)
+    csr = conn.random_in_degree(n, n, rng, deg, conn.Normal(0.0, 0.1, rng=rng))
+    r0 = rng.random(n)
+    net = ah.Network(dt=1.0, seed=3, precision=precision)
+    pop = net.create(n, ah.RateNoisy)
+    proj = net.connect(pop, pop, "exc").from_csr(csr, storage_format="csr")
+    net.compile()
+    proj.set_format("sell_panel", **opts)
+    pop.r = r0
+    pop.inject_random(0, np.zeros((1, n)))
+    r = r0 if precision == "double" else r0.astype(np.float32).astype(np.float64)
+    rows = np.repeat(np.arange(n), np.diff(csr.row_ptr))
+    return net, pop, proj, r0, np.bincount(rows, weights=csr.w * r[csr.col_idx], minlength=n)
+
+
+@pytest.mark.parametrize("opts", [{}, dict(panel_cols=9001, chunk=2048, sigma=8, lanes=2)],
+                         ids=["automatic", "given"])
+def test_a_rebuilt_layout_is_the_same(gpu, opts):
+    n = 9001
+    net, pop, proj, r0, _ = _one_psp(n, "double", opts)
+
+    def psp():
+        pop.r = r0
+        net.step()
+        return np.asarray(pop.sum("exc")).reshape(-1).copy()
+
+    form, first = proj.get_format(), psp()
+    proj.w = proj.w
+    assert proj.get_format() == form
+    np.testing.assert_array_equal(psp(), first)
+    f = dict(form)
+    proj.set_format(f.pop("format"), **f)
+    assert proj.get_format() == form
+    np.testing.assert_array_equal(psp(), first)

@@ -99,6 +99,7 @@ _SIGS = {
     "ahip_pop_inject_random": ([_P, _I32, _I32, _PD, _I64], _I32),
     "ahip_proj_create": ([_P, _I32, _I32, C.c_char_p, _I32, _PI32], _I32),
     "ahip_proj_init_csr": ([_P, _I32, _I32, _I32, _PI64, _PI32, _PD, _D, C.POINTER(FormatOpts)], _I32),
+    "ahip_proj_fit_tiles": ([_P, _I32], _I32),
     "ahip_proj_set_format": ([_P, _I32, C.POINTER(FormatOpts)], _I32),
     "ahip_proj_get_format": ([_P, _I32, C.POINTER(FormatOpts)], _I32),
     "ahip_proj_nb_synapses": ([_P, _I32, _PI64], _I32),

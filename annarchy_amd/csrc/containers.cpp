@@ -96,7 +96,7 @@ static int32_t equal_panels(int32_t n_cols, int32_t pmax) {
     return (n_cols + np - 1) / np;
 }
 
-int build_layout(const Proj& p, int32_t precision, const ahip_format_opts& o, RateLayout& L,
+int build_layout(const Proj& p, int32_t precision, const ahip_format_opts& o, bool fit_tiles, RateLayout& L,
                  std::string& err) {
     const int32_t R = p.n_rows;
     const std::vector<int64_t>& rp = p.h_row_ptr;
@@ -333,6 +333,8 @@ int build_layout(const Proj& p, int32_t precision, const ahip_format_opts& o, Ra
                 err = "sliced tiles: steps in flight must be 2, 4 or 8 (1 with 4 waves)";
                 return AHIP_EINVAL;
             }
+            // Sizes that were given are built.  Automatic ones, and those given
+            // as upper limits (the selector's), fit the device.
             // With fewer tiles than CUs at the height asked for, lower tiles fill
             // the device's workgroup slots (CUs x the panels one CU's LDS holds,
             // at most 32 waves a CU) in one round; at the default height of very
@@ -345,10 +347,11 @@ int build_layout(const Proj& p, int32_t precision, const ahip_format_opts& o, Ra
             // 256 rows 17 us, 790 of 128 20.6 us.
             const int32_t cus = device_cus();
             const int64_t asked = (int64_t)std::max<int32_t>(1, (p.n_cols + pc - 1) / pc) * ((R + rb_rows - 1) / rb_rows);
-            const bool few = asked < cus / 2;
-            if (few) pc = equal_panels(p.n_cols, std::min(pc, 10239));
+            const bool fit_rows = fit_tiles || o.chunk <= 0;
+            const bool few = fit_rows && asked < cus / 2;
+            if (few && (fit_tiles || o.panel_cols <= 0)) pc = equal_panels(p.n_cols, std::min(pc, 10239));
             const int32_t np = std::max<int32_t>(1, (p.n_cols + pc - 1) / pc);
-            if (o.chunk <= 0 || asked < cus) {
+            if (fit_rows && (o.chunk <= 0 || asked < cus)) {
                 const int64_t fit = std::min<int64_t>((160 * 1024) / ((int64_t)(pc + 1) * es), 32 / waves);
                 const int64_t slots = (int64_t)cus * std::max<int64_t>(1, fit);
                 const int64_t nrb = std::max<int64_t>(1, slots / np);
@@ -459,6 +462,7 @@ int build_layout(const Proj& p, int32_t precision, const ahip_format_opts& o, Ra
             L.chunk = rb_rows;
             L.asked_chunk = o.chunk;
             L.asked_panel_cols = o.panel_cols;
+            L.fit = fit_tiles;
             L.n_units = np;
             L.width = nrb;
             L.stored = total;

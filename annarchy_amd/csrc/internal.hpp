@@ -39,8 +39,10 @@ struct RateLayout {
     int32_t sigma = 1;
     int32_t panel_cols = 0;
     // SELL_PANEL: the tile height and panel width asked for (0: automatic; the
-    // ones above are those built): what the layout is rebuilt from
+    // ones above are those built) and whether they were upper limits: what the
+    // layout is rebuilt from
     int32_t asked_chunk = 0, asked_panel_cols = 0;
+    bool fit = false;
     int64_t stored = 0;       // stored entries including padding
     int32_t width = 0;        // ELL max row length / DENSE values per stored row
     int32_t n_units = 0;      // SELL slices / BSR block rows / panels
@@ -141,6 +143,7 @@ struct Proj {
     bool counted = false;         // spiking: the scatter counts the events, the post update adds them
     DevBuf cnt;                   // counted without a delay per synapse: int32[n_rows], 0 between steps
     DevBuf xd;                    // rate uniform delay: the delayed pre-synaptic rates
+    bool fit_tiles = false;       // tile sizes of the next format are upper limits
     // plasticity: a generated synapse model and its state.  State order:
     // spiking -> column order (as w_col), rate -> forward order (CSR val).
     void* syn_dl = nullptr;
@@ -421,7 +424,8 @@ int batch_launch_advance(const BatchDev& B, int64_t n, hipStream_t s);
 int report_error(int code, const char* msg);
 
 // Format builders (host, from the forward CSR view).
-int build_layout(const Proj& p, int32_t precision, const ahip_format_opts& o, RateLayout& out,
+// fit: the tile sizes of a SELL_PANEL layout are upper limits
+int build_layout(const Proj& p, int32_t precision, const ahip_format_opts& o, bool fit, RateLayout& out,
                  std::string& err);
 double psp_bytes(const Proj& p, int32_t precision);
 // Compute units of the current device.

@@ -19,6 +19,7 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "internal.hpp"
@@ -2159,7 +2160,7 @@ int ahip_proj_init_csr(ahip_net* net, int32_t proj, int32_t n_rows, int32_t n_co
         o = ahip_format_opts{AHIP_FMT_CSR, 64, 0, 1, 0};
     }
     std::string err;
-    int rc = build_layout(*p, net->precision, o, p->rate, err);
+    int rc = build_layout(*p, net->precision, o, std::exchange(p->fit_tiles, false), p->rate, err);
     if (rc) return fail(rc, "%s", err.c_str());
     return p->syn ? init_syn_state(net, *p) : 0;
 }
@@ -2235,13 +2236,21 @@ int ahip_proj_get_csr(ahip_net* net, int32_t proj, int64_t* row_ptr, int32_t* co
     return 0;
 }
 
+int ahip_proj_fit_tiles(ahip_net* net, int32_t proj) {
+    Proj* p = get_proj(net, proj);
+    if (!p || p->spiking) return fail(AHIP_EINVAL, "bad projection");
+    p->fit_tiles = true;
+    return 0;
+}
+
 // The options that give the layout L again.
-static ahip_format_opts rebuild_opts(const RateLayout& L) {
+static ahip_format_opts rebuild_opts(const RateLayout& L, bool* fit) {
     ahip_format_opts o{L.format, L.lanes, L.chunk, L.sigma, L.panel_cols};
     if (L.format == AHIP_FMT_SELL_PANEL) {
         o.chunk = L.asked_chunk;
         o.panel_cols = L.asked_panel_cols;
     }
+    *fit = L.fit;
     return o;
 }
 
@@ -2263,11 +2272,12 @@ int ahip_proj_set_format(ahip_net* net, int32_t proj, const ahip_format_opts* op
     std::string err;
     RateLayout L;
     ahip_format_opts o = *opts;
+    bool fit = std::exchange(p->fit_tiles, false);
     // the format the projection reports is the one it has
-    if (o.format == AHIP_FMT_SELL_PANEL && p->rate.format == o.format && o.chunk == p->rate.chunk &&
+    if (!fit && o.format == AHIP_FMT_SELL_PANEL && p->rate.format == o.format && o.chunk == p->rate.chunk &&
         o.panel_cols == p->rate.panel_cols && o.lanes_per_row == p->rate.lanes && o.sigma == p->rate.sigma)
-        o = rebuild_opts(p->rate);
-    int rc = build_layout(*p, net->precision, o, L, err);
+        o = rebuild_opts(p->rate, &fit);
+    int rc = build_layout(*p, net->precision, o, fit, L, err);
     if (rc) return fail(rc, "%s", err.c_str());
     p->rate = std::move(L);
     return 0;
@@ -2472,10 +2482,11 @@ int ahip_proj_set_w(ahip_net* net, int32_t proj, const double* w, int64_t nnz) {
     invalidate(net);
     if (p->syn) return syn_field_io(net, *p, -1, const_cast<double*>(w), nullptr, true);
     if (p->spiking) return build_backward(net, *p);
-    const ahip_format_opts o = rebuild_opts(p->rate);
+    bool fit = false;
+    const ahip_format_opts o = rebuild_opts(p->rate, &fit);
     std::string err;
     RateLayout L;
-    int rc = build_layout(*p, net->precision, o, L, err);
+    int rc = build_layout(*p, net->precision, o, fit, L, err);
     if (rc) return fail(rc, "%s", err.c_str());
     p->rate = std::move(L);
     return 0;
@@ -2541,7 +2552,7 @@ int ahip_proj_set_synapse(ahip_net* net, int32_t proj, const char* synapse_lib) 
         ahip_format_opts o{csr ? p->rate.format : AHIP_FMT_CSR, csr ? p->rate.lanes : 64, 0, 1, 0};
         std::string err;
         RateLayout L;
-        if ((rc = build_layout(*p, net->precision, o, L, err))) return fail(rc, "%s", err.c_str());
+        if ((rc = build_layout(*p, net->precision, o, false, L, err))) return fail(rc, "%s", err.c_str());
         p->rate = std::move(L);
     }
     return init_syn_state(net, *p);

@@ -424,6 +424,7 @@ class Projection:
         self._generator = "numpy"
         self._delays = 0.0
         self._format = _lib.opts("csr", 64)
+        self._fit = False
         self._auto_format = True
         self._selected = None
         self._syn_init = {}
@@ -755,6 +756,7 @@ class Projection:
             spec.w_kind, spec.w_a = 0, float(w)
         spec.seed = int(self.net.rng.integers(1 << 63))
         L = _lib.lib()
+        self._send_fit()
         _lib.check(L.ahip_proj_generate(self.net._h, self.id, C.byref(spec), C.byref(self._format)))
         nnz = C.c_int64()
         _lib.check(L.ahip_proj_nb_synapses(self.net._h, self.id, C.byref(nnz)))
@@ -788,6 +790,8 @@ class Projection:
                 sel = self._selected
                 self._format = _lib.opts(sel["fmt"], sel.get("lanes", 0), sel.get("chunk", 0), sel.get("sigma", 1),
                                          sel.get("panel_cols", 0))
+                self._fit = True
+                self._send_fit()
                 _lib.check(L.ahip_proj_set_format(self.net._h, self.id, C.byref(self._format)))
         else:
             self.csr = self._build_csr()
@@ -798,8 +802,10 @@ class Projection:
                 sel = self._selected
                 self._format = _lib.opts(sel["fmt"], sel.get("lanes", 0), sel.get("chunk", 0), sel.get("sigma", 1),
                                          sel.get("panel_cols", 0))
+                self._fit = True
             c = self.csr
             w = c.w
+            self._send_fit()
             _lib.check(L.ahip_proj_init_csr(self.net._h, self.id, c.n_rows, c.n_cols,
                                             _lib.ptr(c.row_ptr, C.c_int64), _lib.ptr(c.col_idx, C.c_int32),
                                             _lib.ptr(w, C.c_double) if w is not None else None,
@@ -812,6 +818,13 @@ class Projection:
             self._upload_learning()
         if not self.transmission:
             self.transmission = False
+
+    def _send_fit(self) -> None:
+        """The tile sizes of the format that follows are upper limits (the
+        selector's picks are fitted to the device; sizes a program gives are
+        built as they are)."""
+        if self._fit and _lib.FORMAT_NAMES[self._format.format] == "sell_panel":
+            _lib.check(_lib.lib().ahip_proj_fit_tiles(self.net._h, self.id))
 
     # -- accessors ------------------------------------------------------------
     @property
@@ -878,10 +891,14 @@ class Projection:
         v = np.ascontiguousarray(np.broadcast_to(np.asarray(value, dtype=np.float64), (self.nb_synapses,)))
         _lib.check(_lib.lib().ahip_proj_set_w(self.net._h, self.id, _lib.ptr(v, C.c_double), v.size))
 
-    def set_format(self, fmt="csr", lanes=0, chunk=0, sigma=1, panel_cols=0):
+    def set_format(self, fmt="csr", lanes=0, chunk=0, sigma=1, panel_cols=0, fit_tiles=False):
+        """Another storage format.  fit_tiles: the tile sizes of "sell_panel" are
+        upper limits, fitted to the device as for storage_format "auto"."""
         self._format = _lib.opts(fmt, lanes, chunk, sigma, panel_cols)
+        self._fit = bool(fit_tiles)
         self._auto_format = False
         if self.net.compiled:
+            self._send_fit()
             _lib.check(_lib.lib().ahip_proj_set_format(self.net._h, self.id, C.byref(self._format)))
 
     @property

@@ -210,6 +210,13 @@ int ahip_proj_generate(ahip_net* net, int32_t proj, const ahip_connect_spec* spe
 /* The forward CSR view of a projection: row_ptr (n_rows + 1) and col (nnz);
  * either may be NULL. */
 int ahip_proj_get_csr(ahip_net* net, int32_t proj, int64_t* row_ptr, int32_t* col, int64_t nnz);
+/* The sizes of SELL_PANEL tiles in the next ahip_format_opts given for the
+ * projection (ahip_proj_init_csr, ahip_proj_generate or ahip_proj_set_format)
+ * are upper limits: where the tiles would be fewer than the CUs they are made
+ * lower, and narrower, until they fill the device.  Without it sizes above 0 are
+ * the ones built.  ahip_proj_get_format reports the sizes built, and setting
+ * what it reports keeps the layout. */
+int ahip_proj_fit_tiles(ahip_net* net, int32_t proj);
 /* Re-layout an initialised rate projection in another format. */
 int ahip_proj_set_format(ahip_net* net, int32_t proj, const ahip_format_opts* opts);
 int ahip_proj_get_format(ahip_net* net, int32_t proj, ahip_format_opts* opts);

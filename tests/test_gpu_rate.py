@@ -175,6 +175,9 @@ def test_sell_panel_large_lds_panels(gpu, precision):
     fmt = dict(storage_format="sell_panel", lanes=2, sigma=8, panel_cols=pc, chunk=2048)
     net, pop, proj = _net_one_step(csr, r0, fmt, precision)
     assert proj.get_format()["panel_cols"] > 8192   # more than 64 KiB of LDS in FP64
+    # built as given: 3 panels in FP64 and 2 in FP32 (88 KiB), tall tiles
+    got = proj.get_format()
+    assert got["panel_cols"] == (15000 if precision == "double" else 22500) and got["chunk"] == 2048
     got = pop.get("_sum_exc").reshape(-1)
     if precision == "double":
         np.testing.assert_allclose(got, ref, rtol=1e-12, atol=1e-13 * np.max(np.abs(ref)))

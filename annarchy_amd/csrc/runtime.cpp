@@ -943,11 +943,13 @@ static int plan_fused(ahip_net* net) {
         // Staging the rates pays when a CU's gathers (one lane per cycle from
         // global memory) outweigh copying them (64 bytes per cycle and about
         // 2000 cycles of latency), and when the rows occupy its 15 summing
-        // waves on at least half the CUs.
+        // waves on at least half the CUs.  A CU's 160 KiB hold them beside the
+        // kernel's own sums, AHIP_FUSE_ROWS of every psp sum of the model.
+        const int64_t own = (int64_t)sums.size() * AHIP_FUSE_ROWS * (int64_t)net->elem() + 64;
         int32_t lanes = lanes_for(10);
         int32_t per_wave = sell ? 1 : kWaveSize / lanes;   // units of a wave
         const int32_t stage_waves = AHIP_FUSE_STAGE_THREADS / kWaveSize - 1;
-        stage = stage && lds <= 128 * 1024 && nnz / cus > lds / 64 + 2000 &&
+        stage = stage && lds <= 128 * 1024 && lds + own <= 160 * 1024 && nnz / cus > lds / 64 + 2000 &&
                 (int64_t)F.units * 2 >= cus * stage_waves * per_wave;
         if (nnz > (stage || F.kind == AHIP_FUSE_DENSE ? kFuseMaxStaged : kFuseMaxGathered)) continue;
         if (!stage) {
@@ -959,7 +961,7 @@ static int plan_fused(ahip_net* net) {
         const int32_t max_share = AHIP_FUSE_ROWS / unit_rows;
         if (stage) {
             // one round on the CUs, as many workgroups on each as its LDS holds
-            const int64_t slots = cus * (2 * (lds + 16 * 1024) <= 160 * 1024 ? 2 : 1);
+            const int64_t slots = cus * (2 * (lds + std::max<int64_t>(16 * 1024, own)) <= 160 * 1024 ? 2 : 1);
             F.share = (int32_t)std::min<int64_t>(max_share, std::max<int64_t>(per_wave, (F.units + slots - 1) / slots));
             F.lds_values = (int32_t)values;
         } else if (F.kind == AHIP_FUSE_DENSE) {

@@ -7,6 +7,8 @@ and update).
   rates has to follow); and against the same network with an idle inactive
   population, which takes the separate psp and update launches;
 * the form that stages the rates in LDS (a network wide enough for it);
+* a model of 24 sums, whose own LDS leaves no room for the rates of 16000
+  neurons that a model of few sums stages;
 * a population with three targets: an undelayed CSR, a CSR with a delay per
   synapse and a dense projection with a uniform delay, against a numpy
   simulation, with a transmission pause and a disabled input in between.
@@ -90,6 +92,27 @@ def test_staged_rates(gpu, fmt):
     a, _, _ = orc.rate_run(csr.row_ptr, csr.col_idx, csr.w, r0, 10.0, 1.0, noise[:12], 12)
     for x, ref in zip(got, (a, b, s)):
         np.testing.assert_allclose(x, ref, rtol=0, atol=1e-11 * max(1.0, np.max(np.abs(ref))))
+
+
+Sum24 = ah.Neuron(equations="r = " + " + ".join(f"sum(t{k})" for k in range(24)), name="Sum24")
+
+
+def test_many_sums_beside_wide_rates(gpu):
+    m, n = 8000, 8000
+    net = ah.Network(dt=1.0, seed=1)
+    a, b, pop = net.create(m, SinRate), net.create(m, SinRate), net.create(n, Sum24)
+    rng, ref = np.random.default_rng(4), np.zeros(n)
+    phases = [rng.random(m) * 6.0 for _ in range(2)]
+    for pre, target, phase in ((a, "t0", phases[0]), (b, "t23", phases[1])):
+        csr = conn.random_in_degree(m, n, rng, np.full(n, 150), conn.Normal(0.0, 0.1, rng=rng))
+        net.connect(pre, pop, target).from_csr(csr, storage_format="csr")
+        # r of step 1 enters the sums of step 2
+        ref += np.bincount(np.repeat(np.arange(n), 150), minlength=n,
+                           weights=csr.w * (0.5 + 0.5 * np.sin(0.1 + phase))[csr.col_idx])
+    net.compile()
+    a.phase, b.phase = phases
+    net.run(3)
+    np.testing.assert_allclose(np.asarray(pop.r).reshape(-1), ref, rtol=0, atol=1e-12 * np.max(np.abs(ref)))
 
 
 def test_three_targets_with_delays(gpu):

@@ -16,6 +16,9 @@ holds: a longer delay given later reads zeros beyond it, and a clock set back
 (reset without the populations) reads it as a ring of that many slots.  A host
 ring gives the same rates, for an input whose steps run ahead and for one that
 keeps state.
+
+The clock may pass 2^32 steps or be negative: ring slots, the rows of a monitor
+with a period and the rows of injected draws follow it there.
 """
 
 import numpy as np
@@ -211,3 +214,35 @@ def test_the_queue_is_as_long_as_its_largest_delay(gpu, source, per_synapse, fmt
     net.reset(populations=False)
     t = 0
     run(25)
+
+
+@pytest.mark.parametrize("t0", [2 ** 32 - 11, 2 ** 40 + 3, -12])
+@pytest.mark.parametrize("per_synapse", [False, True])
+def test_clocks_beyond_32_bits(gpu, t0, per_synapse):
+    n, steps = 3, 30
+    net = ah.Network(dt=1.0, seed=1)
+    inp, out, noisy = net.create(n, RateT), net.create(n, DelayOut), net.create(n, ah.RateNoisy)
+    csr = conn.from_arrays(n, n, np.arange(n + 1), np.arange(n), np.full(n, 0.5))
+    delay = np.array([2, 5, 3]) if per_synapse else np.full(n, 5)
+    net.connect(inp, out, "ff").from_csr(csr, storage_format="csr", delays=delay.astype(float) if per_synapse else 5.0)
+    net.connect(inp, noisy, "exc").from_csr(conn.from_arrays(n, n, np.arange(n + 1), np.arange(n), np.zeros(n)),
+                                            storage_format="csr")
+    every, third = net.monitor(out, ["r"], capacity=100), net.monitor(out, ["r"], capacity=100, period=3.0)
+    r = net.monitor(noisy, ["r"], capacity=100)
+    net.compile(graph_batch=20)
+    draws = np.random.default_rng(2).random((7, n))
+    noisy.inject_random(0, draws)          # row 0 at step 0
+    ah._lib.check(ah._lib.lib().ahip_set_time(net._h, t0))
+    for m in (every, third, r):
+        m.clear()
+    net.run(steps)
+    t = np.arange(t0, t0 + steps)
+    ref = 0.5 * np.where(t[:, None] - delay >= t0, t[:, None] - delay, 0).astype(float)
+    np.testing.assert_array_equal(every.get("r"), ref)
+    if t0 > 0:
+        np.testing.assert_array_equal(third.get("r"), ref[t % 3 == 0])
+    x, xs = np.zeros(n), []
+    for k in range(steps):
+        x = np.maximum(x + (-x + draws[t[k] % 7]) / 10.0, 0.0)
+        xs.append(x)
+    np.testing.assert_allclose(r.get("r"), xs, rtol=0, atol=1e-15)   # 30 contracting steps of values below 1

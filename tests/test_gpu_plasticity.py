@@ -16,7 +16,14 @@
   update period of enable_learning and with learning disabled;
 * continuous spiking update (the pattern of test_SpikingContinuousUpdate):
   a hand-derived weight trajectory of traces set by pre / post events and
-  decremented every step.
+  decremented every step;
+* rows at the edges of what a wave takes at a time (256 synapses) and long enough
+  to be shared by several waves: the three rate rules against the oracle (all
+  terms positive: a sum of K <= 9000 of them is right to K u = 1e-12, a weight
+  moves by at most a tenth of itself: rtol 1e-10; FP32 sums are compensated, 60
+  steps of a few roundings of 6e-8: 1e-5), the continuous rule against a host
+  loop, exactly;
+* fields of more synapses than one staging chunk (2^22) read back as written.
 """
 
 import numpy as np
@@ -330,3 +337,103 @@ def test_spiking_continuous_update_kat(gpu):
     g = mon.get("g_exc")[:, 0]
     np.testing.assert_array_equal(np.flatnonzero(g), [6, 9])
     np.testing.assert_array_equal(g[[6, 9]], [3.0, 2.0])
+
+
+# -- long rows ----------------------------------------------------------------
+
+def _rows(lengths, n_pre, seed):
+    rng = np.random.default_rng(seed)
+    col = np.concatenate([np.sort(rng.choice(n_pre, k, replace=False)) for k in lengths])
+    return np.concatenate([[0], np.cumsum(lengths)]).astype(np.int64), col.astype(np.int32)
+
+
+@pytest.mark.parametrize("rule,precision", [("hebb", "double"), ("oja", "double"), ("ibcm", "double"), ("oja", "float")])
+def test_rate_rules_on_long_rows(gpu, rule, precision):
+    # a slow rule: eta sum(r^2) of the longest row is 7e-4 a step
+    kind, syn, prm = RULES[rule]
+    prm = [2e-7, *prm[1:]]
+    lengths, n_pre, steps = [1, 255, 256, 257, 1023, 1024, 1025, 1500, 9000], 9000, 60
+    ptr, col = _rows(lengths, n_pre, 3)
+    w0 = np.random.default_rng(8).uniform(0.5, 1.5, col.size) / np.repeat(lengths, lengths)
+    net = ah.Network(dt=1.0, seed=3, precision=precision)
+    pre, post = net.create(n_pre, SinRate), net.create(len(lengths), SumRate)
+    proj = net.connect(pre, post, "exc", synapse=syn).from_csr(conn.from_arrays(len(lengths), n_pre, ptr, col, w0))
+    phase = np.linspace(0.0, 2.0 * np.pi, n_pre)
+    pre.phase, proj.eta = phase, prm[0]
+    net.compile(graph_batch=20)
+    start = proj.w.copy()
+    net.run(steps)
+    seq = 0.5 + 0.5 * np.sin(0.1 * np.arange(steps, dtype=np.float64)[:, None] + phase[None, :])
+    ref = orc.rate_plastic_run(kind, ptr, col, start, prm, 1.0, 0.0, seq)
+    assert np.max(np.abs(ref["w"] / start - 1.0)) > 1e-3
+    np.testing.assert_allclose(proj.w, ref["w"], rtol=1e-10 if precision == "double" else 1e-5, atol=0)
+
+
+@pytest.mark.parametrize("precision", ["double", "float"])
+def test_continuous_update_on_long_rows(gpu, precision):
+    pre_n = ah.Neuron(equations="v = v + 1.0\nmp = t", spike="v == 3.0", reset="v = 0.0", name="Every3")
+    post_n = ah.Neuron(equations="v = v + 1.0\nmp = t\nq = g_exc", spike="v == 5.0", reset="v = 0.0",
+                       name="Every5")
+    syn = ah.Synapse(
+        pre_spike="pre_trace = pre.mp",
+        post_spike="post_trace = post.mp",
+        equations="""
+            post_trace = post_trace - 1 : min=0.0
+            pre_trace = pre_trace - 1 : min=0.0
+            w = post_trace + pre_trace
+        """, name="Traces")
+    lengths, n_pre = [1, 255, 257, 700, 1200], 1200
+    ptr, col = _rows(lengths, n_pre, 5)
+    row = np.repeat(np.arange(len(lengths)), lengths)
+    net = ah.Network(dt=1.0, precision=precision)
+    a, b = net.create(n_pre, pre_n), net.create(len(lengths), post_n)
+    proj = net.connect(a, b, "exc", synapse=syn).from_csr(conn.from_arrays(len(lengths), n_pre, ptr, col, np.zeros(col.size)))
+    mon = net.monitor(b, ["q"], capacity=40)
+    net.compile(graph_batch=9)
+    u, v = np.arange(n_pre) % 3.0, np.arange(len(lengths)) % 5.0
+    a.v, b.v = u, v
+    x, y, w, fired, t = np.zeros(col.size), np.zeros(col.size), np.zeros(col.size), np.zeros(n_pre, bool), 0
+    for steps in (1, 20, 9):
+        net.run(steps)
+        g = np.zeros((steps, len(lengths)))
+        for k in range(steps):
+            on = fired[col]
+            g[k] = np.bincount(row[on], weights=w[on], minlength=len(lengths))   # whole numbers
+            x[on] = t - 1.0
+            u, v = u + 1.0, v + 1.0
+            fired, spiked = u == 3.0, v == 5.0
+            u[fired], v[spiked] = 0.0, 0.0
+            x, y = np.maximum(x - 1.0, 0.0), np.maximum(y - 1.0, 0.0)
+            w = x + y
+            y[spiked[row]] = t
+            t += 1
+        np.testing.assert_array_equal(proj.w, w)
+        np.testing.assert_array_equal(proj.pre_trace, x)
+        np.testing.assert_array_equal(proj.post_trace, y)
+        np.testing.assert_array_equal(mon.get("q"), g)
+
+
+@pytest.mark.parametrize("precision", ["double", "float"])
+@pytest.mark.parametrize("spiking", [True, False])
+def test_fields_of_many_synapses(gpu, spiking, precision):
+    m, n = 2000, 2100
+    rng = np.random.default_rng(6)
+    as_held = lambda v: v if precision == "double" else v.astype(np.float32).astype(np.float64)
+    w = rng.random(m * n)
+    net = ah.Network(dt=1.0, seed=1, precision=precision)
+    pre, post = (net.create(m, PoissonPre), net.create(n, PoissonPostG)) if spiking else (
+        net.create(m, SinRate), net.create(n, SumRate))
+    proj = net.connect(pre, post, "exc", synapse=STDP_A if spiking else RULES["hebb"][1]).from_csr(
+        conn.from_arrays(n, m, np.arange(n + 1) * m, np.tile(np.arange(m), n), w))
+    net.compile()
+    assert proj.nb_synapses > 1 << 22
+    np.testing.assert_array_equal(proj.w, as_held(w))
+    proj.w = w[::-1]
+    np.testing.assert_array_equal(proj.w, as_held(w[::-1]))
+    if spiking:
+        x = rng.random(m * n)
+        proj.x = x
+        np.testing.assert_array_equal(proj.x, as_held(x))
+        np.testing.assert_array_equal(proj.y, 0.0)
+        np.testing.assert_array_equal(proj.w, as_held(w[::-1]))
+        np.testing.assert_array_equal(proj.last_event, -10000)

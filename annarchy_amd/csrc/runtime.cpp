@@ -33,6 +33,9 @@ namespace {
 thread_local std::string g_err;
 
 int fail(int code, const char* fmt, ...) {
+    // a HIP error is reported here, once: left in place the next launch would
+    // report it again
+    if (code == AHIP_EHIP || code == AHIP_ENOMEM) (void)hipGetLastError();
     char buf[1024];
     va_list ap;
     va_start(ap, fmt);

@@ -102,3 +102,27 @@ def test_non_finite_weights_propagate(gpu):
     net.run(2)
     s = post.sum("exc")
     assert np.isnan(s[0]) and s[1] == 2.0 and np.isposinf(s[2]) and s[3] == 7.0
+
+
+def test_a_failed_probe_leaves_no_error_behind(gpu):
+    # the update of an inactive population is not launched: no time to report;
+    # the weights, read through a kernel of their own, and the run after it are
+    # not its business
+    net = ah.Network(dt=1.0, seed=2)
+    pre = net.create(5, ah.Neuron(parameters="rates = 40.0", equations="p = Uniform(0.0, 1.0) * 1000.0 / dt",
+                                  spike="p < rates", name="PoissonPre"))
+    post = net.create(4, ah.Neuron(parameters="rates = 30.0", equations="p = Uniform(0.0, 1.0) * 1000.0 / dt\nmp = g_exc",
+                                   spike="p < rates", name="PoissonPostG"))
+    stdp = ah.STDP(tau_plus=20.0, tau_minus=20.0, A_plus=0.01, A_minus=0.0105, w_min=0.0, w_max=1.0)
+    proj = net.connect(pre, post, "exc", synapse=stdp).all_to_all(0.3)
+    net.compile(allow_build=False)
+    post.disable()
+    with pytest.raises(_lib.AhipError, match="probe"):
+        net.time_kernel(3, post.id, 2)
+    np.testing.assert_array_equal(proj.w, 0.3)
+    with pytest.raises(_lib.AhipError, match="probe"):
+        net.time_kernel(3, post.id, 2)
+    net.run(20)
+    post.enable()
+    net.run(20)
+    assert net.time_kernel(3, post.id, 2) > 0.0

@@ -1983,7 +1983,7 @@ int ahip_proj_size_in_bytes(ahip_net* net, int32_t proj, int64_t* bytes) {
     const RateLayout& L = p->rate;
     size_t b = 0;
     for (const DevBuf* d : std::initializer_list<const DevBuf*>{&L.ptr, &L.idx, &L.val, &L.rl, &L.perm, &L.aux, &L.tiles, &p->col_ptr, &p->row_idx,
-                            &p->w_col, &p->delay_dev, &p->ring, &p->xd, &p->syn_rec, &p->last_event,
+                            &p->w_col, &p->delay_dev, &p->ring, &p->cnt, &p->xd, &p->syn_rec, &p->last_event,
                             &p->fwd2col, &p->row_ptr_dev, &p->col_dev})
         b += d->bytes;
     for (const DevBuf& d : p->syn_attr) b += d.bytes;

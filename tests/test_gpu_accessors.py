@@ -30,6 +30,18 @@ def test_size_in_bytes_bounds(gpu):
     assert proj.size_in_bytes() >= nnz * (8 + 4) + 1001 * 8
 
 
+def test_size_in_bytes_holds_the_event_counts(gpu):
+    # a projection of one weight counts its events per post neuron, from the
+    # first run on
+    net = ah.Network(dt=0.5, seed=4)
+    pre, post = net.create(300, PoissonPre), net.create(200, PoissonPostG)
+    proj = net.connect(pre, post, "exc").fixed_probability(0.1, 0.2)
+    net.compile()
+    before = proj.size_in_bytes()
+    net.run(2)
+    assert proj.size_in_bytes() == before + 200 * 4
+
+
 def test_nb_efferent_and_delivered_events(gpu):
     net = ah.Network(dt=0.5, seed=4)
     pre = net.create(300, PoissonPre)

@@ -877,9 +877,14 @@ static int assign_ahead(ahip_net* net) {
         if (p.ahead != was_ahead || p.deferred != was_deferred) drop_graph(net);
         if (p.model->spiking && (ok || defer) && p.spike_mask.bytes < (size_t)AHIP_AHEAD * p.nwords() * sizeof(uint64_t)) {
             HIPCHK(hipStreamSynchronize(net->stream));
-            int rc = dev_alloc(p.spike_mask, (size_t)AHIP_AHEAD * p.nwords() * sizeof(uint64_t));
-            if (!rc) rc = dev_alloc(p.block_counts, (size_t)AHIP_AHEAD * p.nblocks() * sizeof(int32_t));
+            // both or neither: a run after one that found no memory for them
+            // must not meet a wide mask without counts
+            DevBuf mask, counts;
+            int rc = dev_alloc(mask, (size_t)AHIP_AHEAD * p.nwords() * sizeof(uint64_t));
+            if (!rc) rc = dev_alloc(counts, (size_t)AHIP_AHEAD * p.nblocks() * sizeof(int32_t));
             if (rc) return rc;
+            p.spike_mask = std::move(mask);
+            p.block_counts = std::move(counts);
         }
     }
     return 0;

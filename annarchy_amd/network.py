@@ -614,11 +614,14 @@ class Projection:
         from . import selector
         chosen = selector.select(self.csr, mode="mlp")
         # Of the two sliced-tile configurations the one of few wide panels when
-        # the narrow ones would be many: the network was trained on timings in
-        # which a network below 1e5 neurons left most CUs without a wide tile
-        # (us per step, narrow / wide: 20000 x 200 17 / 19, 25000 x 500 38 / 38,
-        # 40001 x 500 lognormal 65 / 54, 60000 x 200 53 / 37; in FP32 37 / 39 at
-        # 31000 x 600 lognormal, 40 / 42 at 40001 x 500, 19 / 14 at 50000 x 50).
+        # the narrow ones would be many: the network was trained on the sizes as
+        # given, which leave most CUs without a wide tile below 1e5 neurons; the
+        # pick is fitted to the device (_send_fit).  us per step, narrow / wide
+        # fitted, at in-degree 200 and lognormal 500: FP64 20000 17 / 19 and
+        # 37 / 44, 24000 20 / 19 and 45 / 41, 28000 22 / 20 and 49 / 44, 32000
+        # 22 / 21 and 49 / 44, 40000 31 / 25 and 64 / 52; FP32 28000 14 / 15 and
+        # 29 / 33, 36000 16 / 16 and 33 / 35, 40000 20 / 18 and 38 / 37, 46000
+        # 22 / 19 and 42 / 39.  (FP64 would gain a tenth from 24000 on.)
         wide = 30000 if self.net.precision in ("double", "float64", "f64") else 45000
         if chosen == selector.CLASSES[0] and self.csr.n_cols > wide:
             return dict(selector.CLASSES[-1])

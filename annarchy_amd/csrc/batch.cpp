@@ -54,13 +54,13 @@ int bfail(int code, const char* fmt, ...) {
 int balloc(DevBuf& b, size_t bytes, const void* src = nullptr) {
     b.release();
     if (bytes == 0) bytes = 8;
-    hipError_t e = hipMalloc(&b.p, bytes);
+    hipError_t e = mem_alloc(&b.p, bytes);
     if (e != hipSuccess) { b.p = nullptr; return bfail(AHIP_ENOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e)); }
     b.bytes = bytes;
-    if (src) BCHK(hipMemcpy(b.p, src, bytes, hipMemcpyHostToDevice));
-    else BCHK(hipMemset(b.p, 0, bytes));
+    if (src) BCHK(mem_copy(b.p, src, bytes, hipMemcpyHostToDevice));
+    else BCHK(mem_set(b.p, 0, bytes));
     // the batch stream is non-blocking: finish the clear before its kernels run
-    BCHK(hipDeviceSynchronize());
+    BCHK(device_sync());
     return 0;
 }
 
@@ -333,9 +333,9 @@ int ahip_batch_set_input(ahip_batch* b, const double* w_in, const double* phase,
                     lo[pos] = bf16_rne(v - bf16_f(hi[pos]));
                 }
     BCHK(hipStreamSynchronize(b->stream));
-    BCHK(hipMemcpy(B.w_hi.p, hi.data(), hi.size() * 2, hipMemcpyHostToDevice));
-    BCHK(hipMemcpy(B.w_lo.p, lo.data(), lo.size() * 2, hipMemcpyHostToDevice));
-    BCHK(hipMemcpy(B.phase.p, phase, (size_t)n * B.n_inst * 8, hipMemcpyHostToDevice));
+    BCHK(mem_copy(B.w_hi.p, hi.data(), hi.size() * 2, hipMemcpyHostToDevice));
+    BCHK(mem_copy(B.w_lo.p, lo.data(), lo.size() * 2, hipMemcpyHostToDevice));
+    BCHK(mem_copy(B.phase.p, phase, (size_t)n * B.n_inst * 8, hipMemcpyHostToDevice));
     B.omega = omega;
     drop_graph(b);
     b->ready_input = true;
@@ -347,7 +347,7 @@ int ahip_batch_set_gain(ahip_batch* b, const double* gain) {
     std::vector<float> g(b->B.n_inst);
     for (int32_t i = 0; i < b->B.n_inst; i++) g[i] = (float)gain[i];
     BCHK(hipStreamSynchronize(b->stream));
-    BCHK(hipMemcpy(b->B.gain.p, g.data(), g.size() * 4, hipMemcpyHostToDevice));
+    BCHK(mem_copy(b->B.gain.p, g.data(), g.size() * 4, hipMemcpyHostToDevice));
     return 0;
 }
 
@@ -356,7 +356,7 @@ int ahip_batch_set_rates(ahip_batch* b, const double* r) {
     std::vector<float> f(b->B.total);
     for (int32_t i = 0; i < b->B.total; i++) f[i] = (float)r[i];
     BCHK(hipStreamSynchronize(b->stream));
-    BCHK(hipMemcpy(b->B.r[b->parity].p, f.data(), f.size() * 4, hipMemcpyHostToDevice));
+    BCHK(mem_copy(b->B.r[b->parity].p, f.data(), f.size() * 4, hipMemcpyHostToDevice));
     return 0;
 }
 
@@ -364,7 +364,7 @@ int ahip_batch_get_rates(ahip_batch* b, double* r) {
     if (!b || !r) return bfail(AHIP_EINVAL, "null argument");
     std::vector<float> f(b->B.total);
     BCHK(hipStreamSynchronize(b->stream));
-    BCHK(hipMemcpy(f.data(), b->B.r[b->parity].p, f.size() * 4, hipMemcpyDeviceToHost));
+    BCHK(mem_copy(f.data(), b->B.r[b->parity].p, f.size() * 4, hipMemcpyDeviceToHost));
     for (int32_t i = 0; i < b->B.total; i++) r[i] = f[i];
     return 0;
 }
@@ -378,7 +378,7 @@ int ahip_batch_get_input_sums(ahip_batch* b, double* y) {
     const size_t block = (size_t)B.n_tiles * 32 * ld;
     std::vector<float> f(block);
     BCHK(hipStreamSynchronize(b->stream));
-    BCHK(hipMemcpy(f.data(), B.y.as<float>() + (size_t)(b->last_chunk - 1) * block, block * 4,
+    BCHK(mem_copy(f.data(), B.y.as<float>() + (size_t)(b->last_chunk - 1) * block, block * 4,
                    hipMemcpyDeviceToHost));
     for (int32_t m = 0; m < B.n_in; m++)
         for (int32_t i = 0; i < B.n_inst; i++) y[(size_t)m * B.n_inst + i] = f[(size_t)i * ld + m];
@@ -397,6 +397,7 @@ int ahip_batch_run(ahip_batch* b, int64_t steps, int32_t graph_batch) {
     if (left >= G) {
         if (!b->graph || b->graph_steps != G || b->graph_parity != b->parity) {
             drop_graph(b);
+            std::unique_lock<std::shared_mutex> alone(capture_lock());
             BCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
             int rc = enqueue_steps(b, G, b->parity);
             hipGraph_t g = nullptr;

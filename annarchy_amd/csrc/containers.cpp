@@ -36,7 +36,7 @@ namespace {
 int upload(DevBuf& b, const void* src, size_t bytes, std::string& err) {
     b.release();
     if (bytes == 0) bytes = 8;  // keep a valid pointer for empty arrays
-    hipError_t e = hipMalloc(&b.p, bytes);
+    hipError_t e = mem_alloc(&b.p, bytes);
     if (e != hipSuccess) {
         b.p = nullptr;
         err = std::string("hipMalloc failed: ") + hipGetErrorString(e);
@@ -44,15 +44,15 @@ int upload(DevBuf& b, const void* src, size_t bytes, std::string& err) {
     }
     b.bytes = bytes;
     if (src) {
-        e = hipMemcpy(b.p, src, bytes, hipMemcpyHostToDevice);
+        e = mem_copy(b.p, src, bytes, hipMemcpyHostToDevice);
         if (e != hipSuccess) {
             err = std::string("hipMemcpy failed: ") + hipGetErrorString(e);
             return AHIP_EHIP;
         }
     } else {
         // wait for the clear: later kernels run on a non-blocking stream
-        e = hipMemset(b.p, 0, bytes);
-        if (e == hipSuccess) e = hipDeviceSynchronize();
+        e = mem_set(b.p, 0, bytes);
+        if (e == hipSuccess) e = device_sync();
         if (e != hipSuccess) {
             err = std::string("hipMemset failed: ") + hipGetErrorString(e);
             return AHIP_EHIP;

@@ -5,6 +5,8 @@
 #include <stdint.h>
 
 #include <memory>
+#include <mutex>
+#include <shared_mutex>
 #include <string>
 #include <vector>
 
@@ -13,6 +15,33 @@
 #include "annarchy_hip_synapse.h"
 
 namespace ahip {
+
+// HIP fails a call that allocates, frees or touches the legacy stream while a
+// stream captures, whatever threads the two belong to, and the capture with it.
+// A capture holds this lock alone, such calls share it; nothing inside a capture
+// makes one.  (Networks of several threads: a run below a batch is captured
+// when its length comes a second time.)
+std::shared_mutex& capture_lock();
+inline hipError_t mem_alloc(void** p, size_t bytes) {
+    std::shared_lock<std::shared_mutex> lock(capture_lock());
+    return hipMalloc(p, bytes);
+}
+inline hipError_t mem_free(void* p) {
+    std::shared_lock<std::shared_mutex> lock(capture_lock());
+    return hipFree(p);
+}
+inline hipError_t mem_copy(void* dst, const void* src, size_t bytes, hipMemcpyKind kind) {
+    std::shared_lock<std::shared_mutex> lock(capture_lock());
+    return hipMemcpy(dst, src, bytes, kind);
+}
+inline hipError_t mem_set(void* p, int value, size_t bytes) {
+    std::shared_lock<std::shared_mutex> lock(capture_lock());
+    return hipMemset(p, value, bytes);
+}
+inline hipError_t device_sync() {
+    std::shared_lock<std::shared_mutex> lock(capture_lock());
+    return hipDeviceSynchronize();
+}
 
 // Device allocation owned by the network (RAII, moved, never copied).
 struct DevBuf {

@@ -198,6 +198,8 @@ static int mlp_alloc(DevBuf& b, size_t bytes) {
 int mlp_run(int32_t n, const float* X, const float* T, float* params, int32_t epochs, float lr,
             float wd, float* loss_curve, float* grad_out) {
     MlpWork w;
+    // (kernels and copies on the legacy stream: not while another thread captures)
+    std::shared_lock<std::shared_mutex> lock(capture_lock());
     int rc;
     const size_t fs = sizeof(float);
     if ((rc = mlp_alloc(w.X, (size_t)n * DIN * fs))) return rc;
@@ -248,6 +250,7 @@ int mlp_run(int32_t n, const float* X, const float* T, float* params, int32_t ep
 
 int mlp_predict_run(int32_t n, const float* X, const float* params, int32_t* cls, float* logits) {
     DevBuf dX, dP, dC, dL;
+    std::shared_lock<std::shared_mutex> lock(capture_lock());
     int rc;
     if ((rc = mlp_alloc(dX, (size_t)n * DIN * 4))) return rc;
     if ((rc = mlp_alloc(dP, NPAR * 4))) return rc;

@@ -64,7 +64,7 @@ int fail(int code, const char* fmt, ...) {
 int dev_alloc(DevBuf& b, size_t bytes) {
     b.release();
     if (bytes == 0) bytes = 8;
-    hipError_t e = hipMalloc(&b.p, bytes);
+    hipError_t e = mem_alloc(&b.p, bytes);
     if (e != hipSuccess) {
         b.p = nullptr;
         return fail(AHIP_ENOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
@@ -73,8 +73,8 @@ int dev_alloc(DevBuf& b, size_t bytes) {
     // The network's work runs on a non-blocking stream, which is not ordered
     // against the null stream a plain memset uses: wait for the clear here so
     // a later kernel on the network stream cannot be overtaken by it.
-    HIPCHK(hipMemset(b.p, 0, bytes));
-    HIPCHK(hipDeviceSynchronize());
+    HIPCHK(mem_set(b.p, 0, bytes));
+    HIPCHK(device_sync());
     return 0;
 }
 
@@ -140,7 +140,7 @@ static int regrow_ring(DevBuf& buf, size_t slot_bytes, int32_t d_old, int32_t d_
     if (buf.p && d_old > 0) {
         for (int64_t k = k_from; k < k_to; k++) {
             const int64_t so = ((k % d_old) + d_old) % d_old, sn = ((k % d_new) + d_new) % d_new;
-            HIPCHK(hipMemcpy((char*)nb.p + sn * slot_bytes, (char*)buf.p + so * slot_bytes, slot_bytes,
+            HIPCHK(mem_copy((char*)nb.p + sn * slot_bytes, (char*)buf.p + so * slot_bytes, slot_bytes,
                              hipMemcpyDeviceToDevice));
         }
     }
@@ -277,7 +277,7 @@ int init_syn_state(ahip_net* net, Proj& p) {
                 const int64_t le = -10000;
                 std::memcpy(r + p.rec_off_last, &le, 8);
             }
-            HIPCHK(hipMemcpy((char*)p.syn_rec.p + (size_t)q0 * p.rec_bytes, buf.data(), (size_t)m * p.rec_bytes,
+            HIPCHK(mem_copy((char*)p.syn_rec.p + (size_t)q0 * p.rec_bytes, buf.data(), (size_t)m * p.rec_bytes,
                              hipMemcpyHostToDevice));
         }
         p.w_col.release();   // the weights live in the records
@@ -290,7 +290,7 @@ int init_syn_state(ahip_net* net, Proj& p) {
         std::vector<int64_t> f2c(p.nnz);
         for (int64_t q = 0; q < p.nnz; q++) f2c[p.h_inv_idx[q]] = q;
         if ((rc = dev_alloc(p.fwd2col, (size_t)p.nnz * sizeof(int64_t)))) return rc;
-        if (p.nnz) HIPCHK(hipMemcpy(p.fwd2col.p, f2c.data(), f2c.size() * sizeof(int64_t), hipMemcpyHostToDevice));
+        if (p.nnz) HIPCHK(mem_copy(p.fwd2col.p, f2c.data(), f2c.size() * sizeof(int64_t), hipMemcpyHostToDevice));
     }
     // waves per spike: 64-synapse chunks of the longest column / row, at most 32
     int64_t max_row = 0;
@@ -301,10 +301,10 @@ int init_syn_state(ahip_net* net, Proj& p) {
     p.syn_pre_chunks = (int32_t)std::min<int64_t>(32, std::max<int64_t>(1, (max_col + 63) / 64));
     p.syn_post_chunks = (int32_t)std::min<int64_t>(32, std::max<int64_t>(1, (max_row + 63) / 64));
     if ((rc = dev_alloc(p.row_ptr_dev, p.h_row_ptr.size() * sizeof(int64_t)))) return rc;
-    HIPCHK(hipMemcpy(p.row_ptr_dev.p, p.h_row_ptr.data(), p.h_row_ptr.size() * sizeof(int64_t),
+    HIPCHK(mem_copy(p.row_ptr_dev.p, p.h_row_ptr.data(), p.h_row_ptr.size() * sizeof(int64_t),
                      hipMemcpyHostToDevice));
     if ((rc = dev_alloc(p.col_dev, (size_t)p.nnz * sizeof(int32_t)))) return rc;
-    if (p.nnz) HIPCHK(hipMemcpy(p.col_dev.p, p.h_col.data(), p.nnz * sizeof(int32_t), hipMemcpyHostToDevice));
+    if (p.nnz) HIPCHK(mem_copy(p.col_dev.p, p.h_col.data(), p.nnz * sizeof(int32_t), hipMemcpyHostToDevice));
     HIPCHK(hipStreamSynchronize(net->stream));
     return 0;
 }
@@ -497,7 +497,7 @@ int build_ordered_targets(ahip_net* net, const std::vector<const void*>& targets
         if (o.touched.bytes < touched_n * sizeof(int32_t) && (rc = dev_alloc(o.touched, touched_n * sizeof(int32_t))))
             return rc;
         if ((rc = dev_alloc(o.scnt, (size_t)o.shards * kShardStride * sizeof(int32_t)))) return rc;
-        HIPCHK(hipMemcpy(o.head.p, head.data(), head.size() * sizeof(uint64_t), hipMemcpyHostToDevice));
+        HIPCHK(mem_copy(o.head.p, head.data(), head.size() * sizeof(uint64_t), hipMemcpyHostToDevice));
         // the post population's update adds the buckets when no other kernel
         // writes the conductance and no monitor records it after compute_psp
         o.in_update = true;
@@ -516,7 +516,7 @@ int build_ordered_targets(ahip_net* net, const std::vector<const void*>& targets
         for (const OrderedTarget& q : net->ordered)
             if (q.in_update && q.pop == o.pop) fused_here++;
         if (fused_here >= AHIP_MAX_DELIVER) o.in_update = false;
-        HIPCHK(hipDeviceSynchronize());
+        HIPCHK(device_sync());
         net->ordered.push_back(std::move(o));
     }
     // the descriptors of every population's update
@@ -537,7 +537,7 @@ int build_ordered_targets(ahip_net* net, const std::vector<const void*>& targets
         if (!dd.empty()) {
             int rc;
             if ((rc = dev_alloc(p.deliver, dd.size() * sizeof(ahip_deliver_desc)))) return rc;
-            HIPCHK(hipMemcpy(p.deliver.p, dd.data(), dd.size() * sizeof(ahip_deliver_desc), hipMemcpyHostToDevice));
+            HIPCHK(mem_copy(p.deliver.p, dd.data(), dd.size() * sizeof(ahip_deliver_desc), hipMemcpyHostToDevice));
         }
     }
     // the merged delivery launch: one DeliverTarget per conductance, their
@@ -565,7 +565,7 @@ int build_ordered_targets(ahip_net* net, const std::vector<const void*>& targets
     if (!tg.empty()) {
         int rc;
         if ((rc = dev_alloc(net->deliver_targets, tg.size() * sizeof(DeliverTarget)))) return rc;
-        HIPCHK(hipMemcpy(net->deliver_targets.p, tg.data(), tg.size() * sizeof(DeliverTarget), hipMemcpyHostToDevice));
+        HIPCHK(mem_copy(net->deliver_targets.p, tg.data(), tg.size() * sizeof(DeliverTarget), hipMemcpyHostToDevice));
     }
     return 0;
 }
@@ -773,10 +773,10 @@ int prepare(ahip_net* net) {
             double v = vals[k];
             p.slot_host_global[k] = v;
             if (net->precision == AHIP_F64) {
-                HIPCHK(hipMemcpy(p.slots[k].p, &v, sizeof(double), hipMemcpyHostToDevice));
+                HIPCHK(mem_copy(p.slots[k].p, &v, sizeof(double), hipMemcpyHostToDevice));
             } else {
                 float f = (float)v;
-                HIPCHK(hipMemcpy(p.slots[k].p, &f, sizeof(float), hipMemcpyHostToDevice));
+                HIPCHK(mem_copy(p.slots[k].p, &f, sizeof(float), hipMemcpyHostToDevice));
             }
         }
     }
@@ -1431,6 +1431,7 @@ int enqueue_batch(ahip_net* net, int32_t nsteps, const std::vector<int32_t>& zb)
 // left in place (it must run first); only the previous executable graph is
 // dropped, so the tables stay valid for as long as the new graph lives.
 int capture_steps(ahip_net* net, int32_t steps, const std::vector<int32_t>& zb, hipGraphExec_t* exec) {
+    std::unique_lock<std::shared_mutex> alone(capture_lock());
     HIPCHK(hipStreamBeginCapture(net->stream, hipStreamCaptureModeThreadLocal));
     int rc = enqueue_batch(net, steps, zb);
     hipGraph_t g = nullptr;
@@ -1506,7 +1507,7 @@ int32_t auto_batch(ahip_net* net) {
 template <typename T>
 void to_host_t(const void* dev, double* out, int64_t n) {
     std::vector<T> tmp(n);
-    hipMemcpy(tmp.data(), dev, n * sizeof(T), hipMemcpyDeviceToHost);
+    mem_copy(tmp.data(), dev, n * sizeof(T), hipMemcpyDeviceToHost);
     for (int64_t i = 0; i < n; i++) out[i] = (double)tmp[i];
 }
 
@@ -1519,8 +1520,13 @@ int ahip::report_error(int code, const char* msg) {
     return code;
 }
 
+std::shared_mutex& ahip::capture_lock() {
+    static auto* lock = new std::shared_mutex;   // never destroyed: buffers may be freed at exit
+    return *lock;
+}
+
 void ahip::DevBuf::release() {
-    if (p) hipFree(p);
+    if (p) mem_free(p);
     p = nullptr;
     bytes = 0;
 }
@@ -1682,7 +1688,7 @@ int ahip_set_time(ahip_net* net, int64_t t) {
         HIPCHK(hipMemcpyAsync(p.hist.p, tmp.p, p.hist.bytes, hipMemcpyDeviceToDevice, net->stream));
         HIPCHK(hipStreamSynchronize(net->stream));
     }
-    HIPCHK(hipMemcpy(net->t_dev.p, &t, sizeof(int64_t), hipMemcpyHostToDevice));
+    HIPCHK(mem_copy(net->t_dev.p, &t, sizeof(int64_t), hipMemcpyHostToDevice));
     net->t = t;
     net->rbuf_stale = true;
     return 0;
@@ -1727,7 +1733,7 @@ int ahip_step(ahip_net* net) { return ahip_run(net, 1); }
 static int stop_reached(ahip_net* net, Pop& p, bool* out) {
     int32_t c = 0;
     if (p.stop_mode >= 3) {
-        HIPCHK(hipMemcpy(&c, p.spike_count.p, sizeof(int32_t), hipMemcpyDeviceToHost));
+        HIPCHK(mem_copy(&c, p.spike_count.p, sizeof(int32_t), hipMemcpyDeviceToHost));
         *out = p.stop_mode == 3 ? c > 0 : c == p.size;
         return 0;
     }
@@ -1863,11 +1869,11 @@ int ahip_pop_set(ahip_net* net, int32_t pop, const char* attr, const double* val
                                (long long)want, (long long)n);
     HIPCHK(hipStreamSynchronize(net->stream));
     if (net->precision == AHIP_F64) {
-        HIPCHK(hipMemcpy(p->slots[k].p, values, n * sizeof(double), hipMemcpyHostToDevice));
+        HIPCHK(mem_copy(p->slots[k].p, values, n * sizeof(double), hipMemcpyHostToDevice));
     } else {
         std::vector<float> f(n);
         for (int64_t i = 0; i < n; i++) f[i] = (float)values[i];
-        HIPCHK(hipMemcpy(p->slots[k].p, f.data(), n * sizeof(float), hipMemcpyHostToDevice));
+        HIPCHK(mem_copy(p->slots[k].p, f.data(), n * sizeof(float), hipMemcpyHostToDevice));
     }
     if (!p->model->slot_local[k]) p->slot_host_global[k] = values[0];
     net->rbuf_stale = true;
@@ -1884,7 +1890,7 @@ int ahip_pop_get(ahip_net* net, int32_t pop, const char* attr, double* values, i
                                attr, (long long)want, (long long)n);
     HIPCHK(hipStreamSynchronize(net->stream));
     if (net->precision == AHIP_F64) {
-        HIPCHK(hipMemcpy(values, p->slots[k].p, n * sizeof(double), hipMemcpyDeviceToHost));
+        HIPCHK(mem_copy(values, p->slots[k].p, n * sizeof(double), hipMemcpyDeviceToHost));
     } else {
         to_host_t<float>(p->slots[k].p, values, n);
     }
@@ -1905,7 +1911,7 @@ int ahip_pop_set_int(ahip_net* net, int32_t pop, const char* attr, const int32_t
     if (!b) return fail(AHIP_EINVAL, "population %d has no integer attribute '%s'", pop, attr);
     if (n != p->size) return fail(AHIP_EINVAL, "'%s' expects %d values", attr, p->size);
     HIPCHK(hipStreamSynchronize(net->stream));
-    HIPCHK(hipMemcpy(b->p, values, n * sizeof(int32_t), hipMemcpyHostToDevice));
+    HIPCHK(mem_copy(b->p, values, n * sizeof(int32_t), hipMemcpyHostToDevice));
     return 0;
 }
 
@@ -1916,7 +1922,7 @@ int ahip_pop_get_int(ahip_net* net, int32_t pop, const char* attr, int32_t* valu
     if (!b) return fail(AHIP_EINVAL, "population %d has no integer attribute '%s'", pop, attr);
     if (n != p->size) return fail(AHIP_EINVAL, "'%s' holds %d values", attr, p->size);
     HIPCHK(hipStreamSynchronize(net->stream));
-    HIPCHK(hipMemcpy(values, b->p, n * sizeof(int32_t), hipMemcpyDeviceToHost));
+    HIPCHK(mem_copy(values, b->p, n * sizeof(int32_t), hipMemcpyDeviceToHost));
     return 0;
 }
 
@@ -1925,7 +1931,7 @@ int ahip_pop_get_last_spike(ahip_net* net, int32_t pop, int64_t* values, int64_t
     if (!p || !values || !p->model->spiking) return fail(AHIP_EINVAL, "bad spiking population");
     if (n != p->size) return fail(AHIP_EINVAL, "last_spike holds %d values", p->size);
     HIPCHK(hipStreamSynchronize(net->stream));
-    HIPCHK(hipMemcpy(values, p->last_spike.p, n * sizeof(int64_t), hipMemcpyDeviceToHost));
+    HIPCHK(mem_copy(values, p->last_spike.p, n * sizeof(int64_t), hipMemcpyDeviceToHost));
     return 0;
 }
 
@@ -1934,11 +1940,11 @@ int ahip_pop_spikes(ahip_net* net, int32_t pop, int32_t* out, int32_t cap, int32
     if (!p || !n || !p->model->spiking) return fail(AHIP_EINVAL, "bad spiking population");
     HIPCHK(hipStreamSynchronize(net->stream));
     int32_t c = 0;
-    HIPCHK(hipMemcpy(&c, p->spike_count.p, sizeof(int32_t), hipMemcpyDeviceToHost));
+    HIPCHK(mem_copy(&c, p->spike_count.p, sizeof(int32_t), hipMemcpyDeviceToHost));
     *n = c;
     if (c > 0 && out) {
         if (c > cap) return fail(AHIP_EINVAL, "spike buffer too small (%d > %d)", c, cap);
-        HIPCHK(hipMemcpy(out, p->spiked.p, c * sizeof(int32_t), hipMemcpyDeviceToHost));
+        HIPCHK(mem_copy(out, p->spiked.p, c * sizeof(int32_t), hipMemcpyDeviceToHost));
     }
     return 0;
 }
@@ -2033,11 +2039,11 @@ int ahip_pop_inject_random(ahip_net* net, int32_t pop, int32_t k, const double* 
     int rc = dev_alloc(p->rand_inject[k], n * net->elem());
     if (rc) return rc;
     if (net->precision == AHIP_F64) {
-        HIPCHK(hipMemcpy(p->rand_inject[k].p, buf, n * sizeof(double), hipMemcpyHostToDevice));
+        HIPCHK(mem_copy(p->rand_inject[k].p, buf, n * sizeof(double), hipMemcpyHostToDevice));
     } else {
         std::vector<float> f(n);
         for (int64_t i = 0; i < n; i++) f[i] = (float)buf[i];
-        HIPCHK(hipMemcpy(p->rand_inject[k].p, f.data(), n * sizeof(float), hipMemcpyHostToDevice));
+        HIPCHK(mem_copy(p->rand_inject[k].p, f.data(), n * sizeof(float), hipMemcpyHostToDevice));
     }
     p->rand_inject_steps[k] = nsteps;
     p->rand_t0 = net->t;
@@ -2097,20 +2103,20 @@ static int build_backward(ahip_net* net, Proj& p) {
         }
     int rc;
     if ((rc = dev_alloc(p.col_ptr, col_ptr.size() * sizeof(int64_t)))) return rc;
-    HIPCHK(hipMemcpy(p.col_ptr.p, col_ptr.data(), col_ptr.size() * sizeof(int64_t), hipMemcpyHostToDevice));
+    HIPCHK(mem_copy(p.col_ptr.p, col_ptr.data(), col_ptr.size() * sizeof(int64_t), hipMemcpyHostToDevice));
     if ((rc = dev_alloc(p.row_idx, row_idx.size() * sizeof(int32_t)))) return rc;
-    if (p.nnz) HIPCHK(hipMemcpy(p.row_idx.p, row_idx.data(), row_idx.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+    if (p.nnz) HIPCHK(mem_copy(p.row_idx.p, row_idx.data(), row_idx.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     p.w_col.release();
     if (!p.single_w) {
         if ((rc = dev_alloc(p.w_col, p.nnz * net->elem()))) return rc;
         if (net->precision == AHIP_F64) {
             std::vector<double> w(p.nnz);
             for (int64_t q = 0; q < p.nnz; q++) w[q] = p.h_w[p.h_inv_idx[q]];
-            if (p.nnz) HIPCHK(hipMemcpy(p.w_col.p, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice));
+            if (p.nnz) HIPCHK(mem_copy(p.w_col.p, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice));
         } else {
             std::vector<float> w(p.nnz);
             for (int64_t q = 0; q < p.nnz; q++) w[q] = (float)p.h_w[p.h_inv_idx[q]];
-            if (p.nnz) HIPCHK(hipMemcpy(p.w_col.p, w.data(), w.size() * sizeof(float), hipMemcpyHostToDevice));
+            if (p.nnz) HIPCHK(mem_copy(p.w_col.p, w.data(), w.size() * sizeof(float), hipMemcpyHostToDevice));
         }
     }
     return 0;
@@ -2206,14 +2212,14 @@ int ahip_proj_generate(ahip_net* net, int32_t proj, const ahip_connect_spec* c, 
                                           0.0, net->stream));
         std::vector<int64_t> counts(n_rows);
         HIPCHK(hipStreamSynchronize(net->stream));
-        HIPCHK(hipMemcpy(counts.data(), d_counts.p, counts.size() * sizeof(int64_t), hipMemcpyDeviceToHost));
+        HIPCHK(mem_copy(counts.data(), d_counts.p, counts.size() * sizeof(int64_t), hipMemcpyDeviceToHost));
         for (int32_t r = 0; r < n_rows; r++) row_ptr[r + 1] = row_ptr[r] + counts[r];
     } else {
         return fail(AHIP_EINVAL, "unknown connector kind");
     }
     const int64_t nnz = row_ptr[n_rows];
     if ((rc = dev_alloc(d_rp, row_ptr.size() * sizeof(int64_t)))) return rc;
-    HIPCHK(hipMemcpy(d_rp.p, row_ptr.data(), row_ptr.size() * sizeof(int64_t), hipMemcpyHostToDevice));
+    HIPCHK(mem_copy(d_rp.p, row_ptr.data(), row_ptr.size() * sizeof(int64_t), hipMemcpyHostToDevice));
     if ((rc = dev_alloc(d_col, (size_t)std::max<int64_t>(nnz, 1) * sizeof(int32_t)))) return rc;
     if (c->w_kind != 0 && (rc = dev_alloc(d_w, (size_t)std::max<int64_t>(nnz, 1) * sizeof(double)))) return rc;
     if (c->kind == AHIP_CONN_FIXED_NUMBER_PRE)
@@ -2227,8 +2233,8 @@ int ahip_proj_generate(ahip_net* net, int32_t proj, const ahip_connect_spec* c, 
     HIPCHK(hipStreamSynchronize(net->stream));
     std::vector<int32_t> col(nnz);
     std::vector<double> w(c->w_kind != 0 ? nnz : 0);
-    if (nnz) HIPCHK(hipMemcpy(col.data(), d_col.p, nnz * sizeof(int32_t), hipMemcpyDeviceToHost));
-    if (nnz && c->w_kind != 0) HIPCHK(hipMemcpy(w.data(), d_w.p, nnz * sizeof(double), hipMemcpyDeviceToHost));
+    if (nnz) HIPCHK(mem_copy(col.data(), d_col.p, nnz * sizeof(int32_t), hipMemcpyDeviceToHost));
+    if (nnz && c->w_kind != 0) HIPCHK(mem_copy(w.data(), d_w.p, nnz * sizeof(double), hipMemcpyDeviceToHost));
     d_col.release();
     d_w.release();
     return ahip_proj_init_csr(net, proj, n_rows, pre.size, row_ptr.data(), col.data(),
@@ -2342,7 +2348,7 @@ int ahip_proj_set_delays(ahip_net* net, int32_t proj, const int32_t* steps, int6
         d16[q] = (int16_t)(p->spiking ? steps[p->h_inv_idx[q]] : steps[q]);
     int rc = dev_alloc(p->delay_dev, d16.size() * sizeof(int16_t));
     if (rc) return rc;
-    HIPCHK(hipMemcpy(p->delay_dev.p, d16.data(), d16.size() * sizeof(int16_t), hipMemcpyHostToDevice));
+    HIPCHK(mem_copy(p->delay_dev.p, d16.data(), d16.size() * sizeof(int16_t), hipMemcpyHostToDevice));
     return 0;
 }
 
@@ -2426,7 +2432,7 @@ static int syn_field_io(ahip_net* net, Proj& p, int field, double* dbl, int64_t*
     char* dev = !p.spiking ? (char*)(field == -1 ? p.rate.val.p : is_int ? p.last_event.p : p.syn_attr[field].p)
                            : (char*)p.syn_rec.p + (field == -1 ? p.rec_off_w : is_int ? p.rec_off_last : p.rec_off[field]);
     if (!p.spiking && (is_int || es == 8)) {
-        HIPCHK(hipMemcpy(write ? dev : host, write ? host : dev, (size_t)p.nnz * 8,
+        HIPCHK(mem_copy(write ? dev : host, write ? host : dev, (size_t)p.nnz * 8,
                          write ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost));
         return 0;
     }
@@ -2438,7 +2444,7 @@ static int syn_field_io(ahip_net* net, Proj& p, int field, double* dbl, int64_t*
     }
     for (int64_t j0 = 0; j0 < p.nnz; j0 += chunk) {
         const int64_t n = std::min(chunk, p.nnz - j0);
-        if (write) HIPCHK(hipMemcpy(net->io.p, host + j0 * 8, (size_t)n * 8, hipMemcpyHostToDevice));
+        if (write) HIPCHK(mem_copy(net->io.p, host + j0 * 8, (size_t)n * 8, hipMemcpyHostToDevice));
         if (p.spiking)
             LCHK(launch_syn_field(dev, p.rec_bytes, (int32_t)es, is_int, p.fwd2col.as<int64_t>() + j0, net->io.p, n,
                                   write, net->stream));
@@ -2447,7 +2453,7 @@ static int syn_field_io(ahip_net* net, Proj& p, int field, double* dbl, int64_t*
         else
             LCHK(launch_convert(dev + j0 * es, 0, net->io.p, 1, n, net->stream));
         HIPCHK(hipStreamSynchronize(net->stream));
-        if (!write) HIPCHK(hipMemcpy(host + j0 * 8, net->io.p, (size_t)n * 8, hipMemcpyDeviceToHost));
+        if (!write) HIPCHK(mem_copy(host + j0 * 8, net->io.p, (size_t)n * 8, hipMemcpyDeviceToHost));
     }
     return 0;
 }
@@ -2460,15 +2466,15 @@ static int syn_field_read(ahip_net* net, Proj& p, int field, double* out) {
 static int syn_plain_io(ahip_net* net, void* dev, double* v, int64_t n, bool write) {
     HIPCHK(hipStreamSynchronize(net->stream));
     if (net->precision == AHIP_F64) {
-        if (n) HIPCHK(hipMemcpy(write ? dev : (void*)v, write ? (void*)v : dev, n * 8,
+        if (n) HIPCHK(mem_copy(write ? dev : (void*)v, write ? (void*)v : dev, n * 8,
                                 write ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost));
     } else {
         std::vector<float> f(n);
         if (write) {
             for (int64_t q = 0; q < n; q++) f[q] = (float)v[q];
-            if (n) HIPCHK(hipMemcpy(dev, f.data(), n * 4, hipMemcpyHostToDevice));
+            if (n) HIPCHK(mem_copy(dev, f.data(), n * 4, hipMemcpyHostToDevice));
         } else {
-            if (n) HIPCHK(hipMemcpy(f.data(), dev, n * 4, hipMemcpyDeviceToHost));
+            if (n) HIPCHK(mem_copy(f.data(), dev, n * 4, hipMemcpyDeviceToHost));
             for (int64_t q = 0; q < n; q++) v[q] = f[q];
         }
     }
@@ -2837,7 +2843,7 @@ int ahip_scatter_groups(ahip_net* net, int32_t* n_groups) {
 static int write_record_state(const Monitor& m) {
     // spikes: rows count from t_start (the rows of earlier segments included)
     const ahip_record_state st = {m.t_start, m.spikes ? 0 : m.seg_base, m.spikes ? 1 : m.period, m.capacity};
-    HIPCHK(hipMemcpy(m.state.p, &st, sizeof(st), hipMemcpyHostToDevice));
+    HIPCHK(mem_copy(m.state.p, &st, sizeof(st), hipMemcpyHostToDevice));
     return 0;
 }
 
@@ -2960,7 +2966,7 @@ int ahip_monitor_get(ahip_net* net, int32_t mon, double* out, int64_t n) {
     HIPCHK(hipStreamSynchronize(net->stream));
     if (n == 0) return 0;
     if (net->precision == AHIP_F64) {
-        HIPCHK(hipMemcpy(out, m->data.p, n * sizeof(double), hipMemcpyDeviceToHost));
+        HIPCHK(mem_copy(out, m->data.p, n * sizeof(double), hipMemcpyDeviceToHost));
     } else {
         to_host_t<float>(m->data.p, out, n);
     }
@@ -2976,14 +2982,14 @@ int ahip_monitor_get_spikes(ahip_net* net, int32_t mon, int32_t* counts, int64_t
     if (steps != have) return fail(AHIP_EINVAL, "monitor holds %lld steps", (long long)have);
     HIPCHK(hipStreamSynchronize(net->stream));
     int64_t fills[AHIP_FILL_RING] = {0};
-    HIPCHK(hipMemcpy(fills, m->fill.p, sizeof(fills), hipMemcpyDeviceToHost));
+    HIPCHK(mem_copy(fills, m->fill.p, sizeof(fills), hipMemcpyDeviceToHost));
     const int64_t fill = have > 0 ? fills[have % AHIP_FILL_RING] : 0;   // indices before recorded step `have`
     *total = fill;
     if (fill > m->idx_capacity) return fail(AHIP_ESTATE, "spike monitor overflowed its buffer");
-    if (counts && steps > 0) HIPCHK(hipMemcpy(counts, m->counts.p, steps * sizeof(int32_t), hipMemcpyDeviceToHost));
+    if (counts && steps > 0) HIPCHK(mem_copy(counts, m->counts.p, steps * sizeof(int32_t), hipMemcpyDeviceToHost));
     if (idx) {
         if (fill > idx_cap) return fail(AHIP_EINVAL, "index buffer too small (%lld)", (long long)fill);
-        if (fill > 0) HIPCHK(hipMemcpy(idx, m->data.p, fill * sizeof(int32_t), hipMemcpyDeviceToHost));
+        if (fill > 0) HIPCHK(mem_copy(idx, m->data.p, fill * sizeof(int32_t), hipMemcpyDeviceToHost));
     }
     return 0;
 }

@@ -115,6 +115,9 @@ struct Pop {
     // spikes read from the mask by the scatter of the next step, compacted
     // AHIP_AHEAD steps at a time
     bool deferred = false;
+    // of the plan: the counted projections into it in the order their events
+    // are added, and the value monitors its update records
+    std::vector<int32_t> counted_in, records;
     bool fused = false;
     ahip_fuse_args fuse;
     // mean firing rate over fr_window steps (0: off): a fr_window-bit history
@@ -334,6 +337,7 @@ struct ahip_net {
     int32_t rest_steps = 0, rest_seen = 0;
     bool dirty = true;             // structure changed since the last capture
     bool scatter_dirty = true;     // the fused scatter tables need rebuilding
+    bool plan_dirty = true;        // which update, scatter and compaction does what needs planning
     uint64_t scatter_gen = 0;       // bumped whenever the scatter tables are rebuilt
     uint64_t graph_scatter_gen = ~0ull;  // the tables generation the step graph was captured with
     // kernel-time probe: HIP events around one plastic kernel inside eager steps

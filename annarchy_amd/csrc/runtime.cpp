@@ -113,6 +113,7 @@ void drop_graph(ahip_net* net) {
 void invalidate(ahip_net* net) {
     drop_graph(net);
     net->scatter_dirty = true;
+    net->plan_dirty = true;
     net->rbuf_stale = true;
 }
 
@@ -575,16 +576,16 @@ static int plan_fused(ahip_net* net);
 // The value monitors that an update records: up to AHIP_MAX_REC of an active
 // population; not the firing rate, which its own kernel writes later.
 static void assign_records(ahip_net* net) {
-    std::vector<int32_t> n(net->pops.size(), 0);
+    for (auto& pp : net->pops) pp->records.clear();
     for (auto& mp : net->mons) {
         Monitor& m = *mp;
         m.in_update = false;
         if (m.spikes || m.paused) continue;
-        const Pop& p = *net->pops[m.pop];
-        if (!p.active || n[m.pop] >= AHIP_MAX_REC) continue;
+        Pop& p = *net->pops[m.pop];
+        if (!p.active || p.records.size() >= AHIP_MAX_REC) continue;
         if (p.model->spiking && p.fr_window > 0 && m.slot == p.slot_index("r")) continue;
         m.in_update = true;
-        n[m.pop]++;
+        p.records.push_back(m.id);
     }
 }
 
@@ -601,6 +602,7 @@ static int assign_counted(ahip_net* net) {
         p.counted = false;
     }
     for (auto& pop : net->pops) {
+        pop->counted_in.clear();
         if (!pop->model->spiking || !pop->active) continue;
         std::vector<Proj*> in;
         for (auto& pp : net->projs)
@@ -620,6 +622,10 @@ static int assign_counted(ahip_net* net) {
             if (ok) pick.push_back(p);
         }
         if (pick.size() > AHIP_MAX_COUNTED) continue;
+        // the projections without a delay per synapse first, as their scatter was
+        for (int pass = 0; pass < 2; pass++)
+            for (const Proj* p : pick)
+                if (p->delay_per_syn == (pass == 1)) pop->counted_in.push_back(p->id);
         for (Proj* p : pick) {
             p->counted = true;
             if (!p->delay_per_syn && p->cnt.bytes < (size_t)p->n_rows * sizeof(int32_t)) {
@@ -640,8 +646,12 @@ int prepare(ahip_net* net) {
     }
     int rc0 = ensure_delay_buffers(net);
     if (rc0) return rc0;
-    assign_records(net);
-    if ((rc0 = assign_counted(net))) return rc0;
+    // planned anew when something it depends on changed (invalidate), not for
+    // every run: a network of many projections that steps one by one
+    if (net->plan_dirty) {
+        assign_records(net);
+        if ((rc0 = assign_counted(net))) return rc0;
+    }
     for (auto& pp : net->pops) {
         Pop& p = *pp;
         if (p.active || p.depth <= 1 || !p.hist.p) continue;
@@ -780,7 +790,11 @@ int prepare(ahip_net* net) {
             }
         }
     }
-    return plan_fused(net);
+    if (net->plan_dirty) {
+        if ((rc0 = plan_fused(net))) return rc0;
+        net->plan_dirty = false;
+    }
+    return 0;
 }
 
 // A projection that a fused update can sum, as its descriptor.  False: the
@@ -1132,21 +1146,17 @@ ahip_pop_args make_args(ahip_net* net, Pop& p, int32_t step) {
         a.push_buf[1] = p.rbuf.p;
         a.push_depth[1] = p.rbuf_depth;
     }
-    // the projections without a delay per synapse first, as their scatter was
-    for (int pass = 0; pass < 2; pass++)
-        for (auto& pp : net->projs) {
-            const Proj& q = *pp;
-            if (!q.counted || q.post != p.id || q.delay_per_syn != (pass == 1)) continue;
-            ahip_counted_desc& d = a.counted[a.n_counted++];
-            d.ring = q.delay_per_syn ? q.ring.p : q.cnt.p;
-            d.w = q.w_const;
-            d.slot = q.target_slot;
-            d.depth = q.delay_per_syn ? q.max_delay : 1;
-            d.sums = q.delay_per_syn && !q.single_w ? 1 : 0;
-        }
-    for (auto& mp : net->mons) {
-        const Monitor& m = *mp;
-        if (!m.in_update || m.pop != p.id) continue;
+    for (int32_t id : p.counted_in) {
+        const Proj& q = *net->projs[id];
+        ahip_counted_desc& d = a.counted[a.n_counted++];
+        d.ring = q.delay_per_syn ? q.ring.p : q.cnt.p;
+        d.w = q.w_const;
+        d.slot = q.target_slot;
+        d.depth = q.delay_per_syn ? q.max_delay : 1;
+        d.sums = q.delay_per_syn && !q.single_w ? 1 : 0;
+    }
+    for (int32_t id : p.records) {
+        const Monitor& m = *net->mons[id];
         const int32_t k = a.n_rec++;
         a.rec_slot[k] = m.slot;
         // psp sums of a rate-coded population stay what they are: recorded

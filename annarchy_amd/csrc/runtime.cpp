@@ -1684,10 +1684,31 @@ int ahip_get_time(ahip_net* net, int64_t* t) {
     return 0;
 }
 
+// A spike monitor's row is its step's distance from t_start: with the clock at t
+// the rows from there on are recorded again, behind the indices of the rows before
+// it (rows that a clock set forward passes over have no spikes).
+static int set_spike_row(ahip_net* net, const Monitor& m, int64_t t) {
+    const int64_t held = std::max<int64_t>(0, std::min(net->t - m.t_start, m.capacity));
+    const int64_t row = std::max<int64_t>(0, std::min(t - m.t_start, m.capacity));
+    std::vector<int32_t> counts(std::min(held, row));
+    if (!counts.empty())
+        HIPCHK(mem_copy(counts.data(), m.counts.p, counts.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
+    int64_t fill = 0;
+    for (int32_t c : counts) fill += c;
+    if (row > held) HIPCHK(mem_set(m.counts.as<int32_t>() + held, 0, (size_t)(row - held) * sizeof(int32_t)));
+    HIPCHK(mem_copy(m.fill.as<int64_t>() + row % AHIP_FILL_RING, &fill, sizeof(fill), hipMemcpyHostToDevice));
+    return 0;
+}
+
 int ahip_set_time(ahip_net* net, int64_t t) {
     if (!net || !net->initialized) return fail(AHIP_ESTATE, "network not initialized");
     HIPCHK(hipStreamSynchronize(net->stream));
     HIPCHK(hipSetDevice(net->device));
+    for (auto& mp : net->mons) {
+        if (!mp->spikes || mp->paused || t == net->t) continue;
+        int rc = set_spike_row(net, *mp, t);
+        if (rc) return rc;
+    }
     for (auto& pp : net->pops) {
         Pop& p = *pp;
         if (!p.hist.p || p.depth == p.queue || t == net->t) continue;

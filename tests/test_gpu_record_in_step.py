@@ -10,6 +10,8 @@ most four of a population), a launch of its own, or the spike compaction.
   r every third step as well, against the trajectory computed on the host;
 * the sum in a monitor of its own, the fifth of such a population, which the
   update does not record: at every step and at every second one;
+* a spike monitor that is kept while the clock is set back or forward: the rows
+  from the new step on are recorded again, a full one included;
 * an `Every5` population with six monitors (five values, spikes), g_exc recorded
   after the events of a one-to-one projection arrive and before the neuron's own
   step.
@@ -108,3 +110,37 @@ def test_spiking_records_follow_the_clock(gpu):
         np.testing.assert_array_equal(mon.get("q"), np.array(gs))
         np.testing.assert_array_equal(mon.get("mp"), np.repeat(np.arange(t - steps, t)[:, None], n, 1))
         assert mon.get("spike") == spikes
+
+
+@pytest.mark.parametrize("persistent", [True, False])
+@pytest.mark.parametrize("capacity", [60, 400])
+def test_spike_rows_are_recorded_again(gpu, persistent, capacity):
+    n = 40
+    net = ah.Network(dt=1.0, seed=1)
+    pop = net.create(n, Every5)
+    net.connect(pop, pop, "exc").one_to_one(0.5)
+    mon, second = (net.monitor(pop, ["spike"], capacity=capacity) for _ in range(2))
+    if persistent:
+        second.pause()
+    net.compile(graph_batch=20)
+    assert net.uses_persistent() == persistent
+    v = np.arange(n) % 7.0
+    pop.v = v
+    rows, t = [], 0
+    for steps, to in ((45, 0), (9, 20), (37, 3), (50, 55), (20, None)):
+        net.run(steps)
+        for _ in range(steps):
+            v = v + 1.0
+            fired = v == 5.0
+            v[fired] = 0.0
+            rows[t:t + 1] = [np.flatnonzero(fired)]
+            t += 1
+        held = rows[:min(t, capacity)]
+        for m in (mon,) if persistent else (mon, second):
+            counts, idx = m.raw_spikes()
+            np.testing.assert_array_equal(counts, [r.size for r in held])
+            np.testing.assert_array_equal(idx, np.concatenate(held))
+        if to is not None:
+            ah._lib.check(ah._lib.lib().ahip_set_time(net._h, to))
+            rows = rows[:to] + [np.zeros(0, int)] * (to - len(rows))
+            t = to

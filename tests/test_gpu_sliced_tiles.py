@@ -22,9 +22,9 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("precision,tol", [("double", 1e-12), ("float", 2e-6)])
 @pytest.mark.parametrize("n,opts", [
     (1, dict(panel_cols=64, chunk=64)), (63, dict(panel_cols=20, chunk=64, sigma=8, lanes=2)),
-    (1500, dict(panel_cols=300, chunk=2048, sigma=8, lanes=2)),     # 5 tiles asked: few
-    (2000, dict(panel_cols=500, chunk=64, sigma=8, lanes=4)),       # 128 asked: lower, not narrower
-    (2900, dict(panel_cols=300, chunk=64, lanes=4)),                # 460 asked: kept
+    (1500, dict(panel_cols=300, chunk=2048, sigma=8, lanes=2)),     # 5 tiles
+    (2000, dict(panel_cols=500, chunk=64, sigma=8, lanes=4)),       # 128
+    (2900, dict(panel_cols=300, chunk=64, lanes=4)),                # 460
 ])
 def test_tile_heights(gpu, n, opts, precision, tol):
     rng = np.random.default_rng(n)
